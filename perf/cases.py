@@ -348,6 +348,10 @@ def _linear_flops(n, l_in, c_in, l_out, c_out):
     return 2.0 * n * sum((2 * a + 1) * ca * cb for a, ca in zip(l_in, c_in) for b, cb in zip(l_out, c_out) if a == b)
 
 
+def _linear_weights(l_in, c_in, l_out, c_out):
+    return sum(ca * cb for a, ca in zip(l_in, c_in) for b, cb in zip(l_out, c_out) if a == b)
+
+
 def _interaction_work(n, E, C, L, l_in, S):
     """(flops, weights) of one interaction, forward and input gradients."""
     ls, lo = list(l_in), list(range(L + 1))
@@ -356,7 +360,7 @@ def _interaction_work(n, E, C, L, l_in, S):
     lin = [(ls, [C] * len(ls), ls, [C] * len(ls)), (lo, per_l, [0] + lo, [C * (L + 1)] + [C] * (L + 1)),
            (lo, [C] * (L + 1), lo, [C] * (L + 1))]
     res = (ls, [C] * len(ls), lo, [C] * (L + 1))
-    weights = sum(_linear_flops(1, *v) / 2 for v in lin) + S * _linear_flops(1, *res) / 2
+    weights = sum(_linear_weights(*v) for v in lin) + S * _linear_weights(*res)
     W = C * len(paths)
     mlp = 2.0 * (E / 2) * (8 * 64 + 2 * 64 * 64 + 64 * W)
     tp = 4.0 * E * C * _couplings(ls, lo, lo)
@@ -382,7 +386,7 @@ def _product_work(n, C, L, S, form, l_out):
         up = (lo, [C] * len(lo), [0] + lo, [gates] + [2 * C] * len(lo))
         lins.append(up)
         S = 1
-    weights = S * sum(_linear_flops(1, *v) / 2 for v in lins)
+    weights = S * sum(_linear_weights(*v) for v in lins)
     lins.append((l_out, [C] * len(l_out), l_out, [C] * len(l_out)))
     return flops + 2 * sum(_linear_flops(n, *v) for v in lins), weights
 
