@@ -219,6 +219,15 @@ __device__ __forceinline__ void sb_store_k16(unsigned short* lds, int plane, int
   }
 }
 
+// 8 k of one row (two f4, k-contiguous) -> planes p[row][kofs ..]
+__device__ __forceinline__ void sb_store_k8(unsigned short* lds, int plane, int off, const f4 (&v)[2]) {
+  const float u[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
+  bx3_bf8 h[3];
+  bx3_split8(u, h);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *(bx3_bf8*)&lds[p * plane + off] = h[p];
+}
+
 // 32 k rows x 128 columns of W [k, n] from column c0: thread t holds k rows
 // k0 + 2 (t/16) and the next, columns 4 (t%16) + 64 q (q < 2) -- v[2 q + r]
 // for row 2 (t/16) + r
@@ -490,9 +499,24 @@ __global__ __launch_bounds__(256) void k_seg_linear_bx3s(const float* __restrict
 //    operand), so a lane holds 4 consecutive columns of one output row, and
 //    the stores trade blocks between lanes fr and fr ^ 8 as the task kernel's
 //    do (8 whole rows of 32 columns per store).
+//  * a workgroup takes 64 of the tile's 128 rows, each wavefront all of them
+//    for 32 columns: 142 registers, so three workgroups run per CU and one's
+//    MFMAs cover another's loads and splits (a whole tile per workgroup, 2 x 2
+//    wavefronts of 64 x 64, ran two at 232 registers), and row blocks past
+//    the tile's rows are left out 32 at a time.  What bounds it then is the
+//    power the matrix cores draw: with both at full load the 64-row form
+//    needs 17% fewer cycles but runs at 1.54 instead of 1.85 GHz, and a
+//    library bf16 product loses the same share from all-zero to random
+//    operands (2247 -> 1602 TFLOP/s).  Taller or wider wavefront tiles (128 x
+//    32 with two workgroups per CU) measured slower.  The tables' XCD runs
+//    matter as much (_xcd_balanced in ops.py).  Both together, whole tiles in
+//    runs of equal length -> halves in runs of equal cost: 12,288 rows x (1 +
+//    3 + 5 + 7), k 2,944-5,376 into 128 columns, 1666 -> 1309 us (142 -> 181
+//    TFLOP/s); the same at 1,024 rows and 4 species 247 -> 153 us; 128 -> 128
+//    shared linears 52 -> 51 us.
 // Tiles, contributions and the XCD-grouped tile order are those of
-// k_seg_linear_bx3s; contribution column 2 is the block's offset in the
-// fragment-order weights.  Per output element the products and their order
+// k_seg_linear_bx3s (entries of 0 rows are skipped); contribution column 2 is
+// the block's offset in the fragment-order weights.  Per output element the products and their order
 // are those of k_seg_linear_bx3s (contributions and k steps in order, the six
 // terms smallest first, each a sum over the same 32 products), so the two
 // kernels give the same bits.
@@ -516,18 +540,18 @@ __device__ __forceinline__ void ft_open(FtLoad& L, const float* __restrict__ x, 
   L.xvec = ((((uintptr_t)L.xa) & 15) == 0) && ((L.k & 3) == 0);
 }
 
-// A (128 rows x 32 k) of step L.s as seg_load_k<128> holds it, but rows past
-// nrows repeat the last row (their outputs are not stored).  VEC (every
-// contribution 16-byte aligned with k % 4 == 0): four unconditional 16-byte
-// loads, a run past k read from the row's start and zeroed -- no branch, so
+// A (64 rows from r0 x 32 k) of step L.s: thread t holds row t / 4, k 8 (t & 3)
+// .. + 7.  Rows past nrows repeat the last row (their outputs are not stored).
+// VEC (every contribution 16-byte aligned with k % 4 == 0): two unconditional
+// 16-byte loads, a run past k read from the row's start and zeroed -- no branch, so
 // the compiler's wait for this step's B (issued before) is exact.
 template <bool VEC>
-__device__ __forceinline__ void ft_load_a(const FtLoad& L, int nrows, int t, f4* v) {
-  const int kk = 32 * L.s + 16 * (t & 1);
-  const int r = min(t >> 1, nrows - 1);
+__device__ __forceinline__ void ft_load_a(const FtLoad& L, int r0, int nrows, int t, f4 (&v)[2]) {
+  const int kk = 32 * L.s + 8 * (t & 3);
+  const int r = r0 + min(t >> 2, nrows - 1);
   const float* row = L.xa + (int64_t)r * L.k;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < 2; ++q) {
     const int left = L.k - (kk + 4 * q);
     if constexpr (VEC) {
       const f4 u = *(const f4*)(left >= 4 ? row + kk + 4 * q : row);
@@ -538,11 +562,11 @@ __device__ __forceinline__ void ft_load_a(const FtLoad& L, int nrows, int t, f4*
   }
 }
 
-// B fragments (three terms) of column blocks jb0 .. jb0 + 3 (clamped to the
+// B fragments (three terms) of column blocks jb0 and jb0 + 1 (clamped to the
 // block's last) at step L.s
-__device__ __forceinline__ void ft_load_b(const FtLoad& L, int jb0, int nb16, int lane, u4v (&d)[3][4]) {
+__device__ __forceinline__ void ft_load_b(const FtLoad& L, int jb0, int nb16, int lane, u4v (&d)[3][2]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < 2; ++j) {
     const int jb = min(jb0 + j, nb16 - 1);
     const unsigned short* p = L.wf + ((int64_t)(jb * L.nks + L.s) * 3) * 512 + 8 * lane;
 #pragma unroll
@@ -551,55 +575,63 @@ __device__ __forceinline__ void ft_load_b(const FtLoad& L, int jb0, int nb16, in
 }
 
 //
-// SPLIT (split k, for launches with too few tiles to fill the chip): work
-// item vi = tile * splits + sp sums steps [sp nks / splits, (sp + 1) nks /
+// SPLIT (split k, for launches with too few tiles to fill the chip, or long k
+// over more weights than the caches hold): item vi = tile * splits + sp sums steps [sp nks / splits, (sp + 1) nks /
 // splits) of the tile's first contribution into its own 128 x 128 partial
 // tile, partials + 16384 vi (row stride 128), with no addend, bias or alpha;
 // k_seg_split_sum adds the partials up (NaN for a tile with more than one
 // contribution).
 template <bool VEC, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_seg_linear_bx3f(
-    const float* __restrict__ x, float* y, const float* addend,
-                                                         const unsigned short* __restrict__ wfrag,
-                                                         const float* __restrict__ bias,
-                                                         const int64_t* __restrict__ tiles,
-                                                         const int64_t* __restrict__ contribs, float alpha,
-                                                         int n_tiles, int per, int splits,
-                                                         float* __restrict__ partials) {
-  constexpr int WM = 4, TR = 128, PL = 128 * SB_STR;   // plane size (bf16)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_seg_linear_bx3f(
+    const float* __restrict__ x, float* y, const float* addend, const unsigned short* __restrict__ wfrag,
+    const float* __restrict__ bias, const int64_t* __restrict__ tiles, const int64_t* __restrict__ contribs,
+    float alpha, int n_tiles, int per, int splits, float* __restrict__ partials) {
+  constexpr int WM = 4, PL = 64 * SB_STR;   // 16-row blocks, plane size (bf16)
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3 * PL];
-  const int vi = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  const int tile = SPLIT ? vi / splits : vi;
-  if (tile >= n_tiles) return;
+  // work item wi: split sp of a tile, half of its rows.  The two halves run
+  // next to each other on one XCD, and all tiles' first k range comes before
+  // their second: tiles that read the same weights start within a few steps
+  // of each other, so what one of them loads the others find in L2.  (With
+  // the splits of a tile side by side, or unsplit, the row tiles of a long-k
+  // block drift apart by more steps than L2 holds: 5,003 rows of 89 species,
+  // k 5,888-10,752 into 256 columns, 4.8 GB of weights: 19.6 GB fetched and
+  // 3,451 us unsplit, 3,281 us in 4 neighbouring splits, 2,710 us this way.)
+  const int half = (int)(blockIdx.x >> 3) & 1;
+  const int wi = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 4);
+  const int sp = SPLIT ? wi / n_tiles : 0, tile = SPLIT ? wi - sp * n_tiles : wi;
+  const int vi = SPLIT ? tile * splits + sp : tile;
+  if (SPLIT ? sp >= splits : tile >= n_tiles) return;
   const int64_t* td = tiles + 8 * (int64_t)tile;
-  const int64_t out_base = td[0];
-  const int rows = (int)td[1], n = (int)td[2], c0 = (int)td[3];
+  const int r0 = 64 * half, rows = min((int)td[1] - r0, 64);
+  if (rows <= 0) return;   // the tile ends in the first half, or a padding entry of the table
+  const int n = (int)td[2], c0 = (int)td[3];
+  const int64_t out_base = td[0] + (int64_t)r0 * n;
   const int64_t bias_off = SPLIT ? -1 : td[4];
   const int cb = (int)td[5];
   int ce = (int)td[6];
   if constexpr (SPLIT) ce = min(ce, cb + 1);   // k_seg_split_sum writes NaN for a tile with more
   const int t = (int)threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int wr = (wv >> 1) * 16 * WM, wc = (wv & 1) * 64;
+  const int wc = wv * 32;   // this wavefront's 32 columns (all 64 rows)
   const int fr = lane & 15, fg = lane >> 4;
   const int nb16 = (n + 15) >> 4, jb0 = (c0 + wc) >> 4;
-  const int soff = (t >> 1) * SB_STR + 16 * (t & 1);   // this thread's k16 run of a k-contiguous plane
+  const int soff = (t >> 2) * SB_STR + 8 * (t & 3);   // this thread's 8 k of a k-contiguous plane
 
-  f4 acc[WM][4];
+  f4 acc[WM][2];
   if (!SPLIT && addend) {
     const bool avec = ((n & 3) == 0) && ((out_base & 3) == 0) && ((((uintptr_t)addend) & 15) == 0);
     const float ia = 1.f / alpha;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = wr + 16 * i + fr, col = c0 + wc + 16 * j + 4 * fg;
+      for (int j = 0; j < 2; ++j) {
+        const int r = 16 * i + fr, col = c0 + wc + 16 * j + 4 * fg;
         acc[i][j] = addend_init(addend, out_base + (int64_t)r * n + col, r < rows, col, n, avec, ia);
       }
   } else {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   }
 
   // skip contributions without k steps
@@ -608,7 +640,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   while (c < ce) {
     ft_open(L, x, wfrag, contribs, c);
     if constexpr (SPLIT) {
-      const int sp = vi - tile * splits;
       L.s = (int)((int64_t)sp * L.nks / splits);
       L.send = (int)((int64_t)(sp + 1) * L.nks / splits);
     }
@@ -642,20 +673,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
       more = false;
     };
-    f4 a0[4], a1[4];
-    u4v b0[3][4], b1[3][4];
-    ft_load_a<VEC>(LA, rows, t, a0);
+    f4 a0[2], a1[2];
+    u4v b0[3][2], b1[3][2];
+    ft_load_a<VEC>(LA, r0, rows, t, a0);
     advance(LA, moreA);
     ft_load_b(LB, jb0, nb16, lane, b0);
     advance(LB, moreB);
-    ft_load_a<VEC>(LA, rows, t, a1);   // (a repeat of the last step when there is no next)
+    ft_load_a<VEC>(LA, r0, rows, t, a1);   // (a repeat of the last step when there is no next)
     advance(LA, moreA);
-    sb_store_k16<false>(As[0], PL, soff, a0, 1.f);
+    sb_store_k8(As[0], PL, soff, a0);
     __syncthreads();
     // step g: MFMAs on LDS buffer `buf` (= g & 1) and fragments cur while A(g
     // + 2) loads into al and B(g + 1) into nxt; then A(g + 1) (in as) split
     // into the other buffer
-    auto step = [&](int buf, const u4v (&cur)[3][4], u4v (&nxt)[3][4], f4 (&al)[4], const f4 (&as)[4]) {
+    auto step = [&](int buf, const u4v (&cur)[3][2], u4v (&nxt)[3][2], f4 (&al)[2], const f4 (&as)[2]) {
       const bool have = moreB;
       // B before A: vector loads complete in issue order, so waiting for
       // this step's B (issued last step) does not wait for the A issued
@@ -663,30 +694,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // a branch makes the compiler wait for every load at the join
       ft_load_b(LB, jb0, nb16, lane, nxt);
       advance(LB, moreB);
-      ft_load_a<VEC>(LA, rows, t, al);
+      ft_load_a<VEC>(LA, r0, rows, t, al);
       advance(LA, moreA);
       __builtin_amdgcn_sched_barrier(0);
       const unsigned short* Ab = As[buf];
 #pragma unroll
       for (int ip = 0; ip < WM / 2; ++ip) {
+        if (ip > 0 && rows <= 32 * ip) break;   // no such rows (uniform)
         bx3_bf8 af[2][3];
 #pragma unroll
         for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
           for (int pl = 0; pl < 3; ++pl)
-            af[ii][pl] = *(const bx3_bf8*)&Ab[pl * PL + (wr + 32 * ip + 16 * ii + fr) * SB_STR + 8 * fg];
+            af[ii][pl] = *(const bx3_bf8*)&Ab[pl * PL + (32 * ip + 16 * ii + fr) * SB_STR + 8 * fg];
 #pragma unroll
         for (int u = 0; u < 6; ++u)   // the six terms a_i b_j, smallest first
 #pragma unroll
           for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < 2; ++j)
               acc[2 * ip + ii][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                   __builtin_bit_cast(bx3_bf8, cur[BX3_TB[u]][j]), af[ii][BX3_TA[u]], acc[2 * ip + ii][j], 0, 0, 0);
       }
       // the next A's split after the MFMAs (interleaving it measured slower)
       __builtin_amdgcn_sched_barrier(0);
-      sb_store_k16<false>(As[buf ^ 1], PL, soff, as, 1.f);
+      sb_store_k8(As[buf ^ 1], PL, soff, as);
       __syncthreads();
       return have;
     };
@@ -694,47 +726,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
-  // the bias of this lane's 16 columns (no loads are outstanding here)
-  f4 bv[4];
+  // the bias of this lane's 8 columns (no loads are outstanding here)
+  f4 bv[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < 2; ++j) {
     bv[j] = f4{0.f, 0.f, 0.f, 0.f};
     if (bias_off >= 0) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) bv[j][q] = bias[bias_off + min(c0 + wc + 16 * j + 4 * fg + q, n - 1)];
     }
   }
-  // acc[i][j][q] = out[row wr + 16 i + fr][column c0 + wc + 16 j + 4 fg + q];
-  // per pair of blocks (2 jp, 2 jp + 1) lanes fr and fr ^ 8 trade one block,
-  // so a store writes 8 whole rows of 32 columns
+  // acc[i][j][q] = out[row 16 i + fr][column c0 + wc + 16 j + 4 fg + q];
+  // lanes fr and fr ^ 8 trade one block, so a store writes 8 whole rows of 32 columns
   const bool vst = SPLIT || (((n & 3) == 0) && ((out_base & 3) == 0) && ((((uintptr_t)y) & 15) == 0));
   const float osc = SPLIT ? 1.f : alpha;
   const bool lo = fr < 8;
   const int jl = lo ? 0 : 1;
+  const int col = c0 + wc + 16 * jl + 4 * fg;
 #pragma unroll
-  for (int jp = 0; jp < 2; ++jp) {
-    const int col = c0 + wc + 32 * jp + 16 * jl + 4 * fg;
+  for (int i = 0; i < WM; ++i) {
+    const f4 v0 = osc * (acc[i][0] + bv[0]), v1 = osc * (acc[i][1] + bv[1]);
+    const f4 give = lo ? v1 : v0;
+    f4 got;
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const f4 v0 = osc * (acc[i][2 * jp] + bv[2 * jp]), v1 = osc * (acc[i][2 * jp + 1] + bv[2 * jp + 1]);
-      const f4 give = lo ? v1 : v0;
-      f4 got;
+    for (int q = 0; q < 4; ++q) got[q] = __shfl_xor(give[q], 8);
+    const f4 s0 = lo ? v0 : got, s1 = lo ? got : v1;   // rows 16 i + (fr & 7), + 8
 #pragma unroll
-      for (int q = 0; q < 4; ++q) got[q] = __shfl_xor(give[q], 8);
-      const f4 s0 = lo ? v0 : got, s1 = lo ? got : v1;   // rows 16 i + (fr & 7), + 8
+    for (int h = 0; h < 2; ++h) {
+      const int r = 16 * i + 8 * h + (fr & 7);
+      if (r >= rows || col >= n) continue;
+      const f4 v = h ? s1 : s0;
+      float* dst = SPLIT ? partials + 16384 * (int64_t)vi + 128 * (r0 + r) + (col - c0)
+                         : y + out_base + (int64_t)r * n + col;
+      if (vst) {
+        *(f4*)dst = v;
+      } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = wr + 16 * i + 8 * h + (fr & 7);
-        if (r >= rows || col >= n) continue;
-        const f4 v = h ? s1 : s0;
-        float* dst = SPLIT ? partials + 16384 * (int64_t)vi + 128 * r + (col - c0) : y + out_base + (int64_t)r * n + col;
-        if (vst) {
-          *(f4*)dst = v;
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (col + q < n) dst[q] = v[q];
-        }
+        for (int q = 0; q < 4; ++q)
+          if (col + q < n) dst[q] = v[q];
       }
     }
   }
@@ -989,6 +1018,7 @@ __global__ __launch_bounds__(KS_THREADS) void k_seg_linear_ks(const float* __res
   KsTask T;
   T.out_base = td[0];
   T.rows = (int)td[1];
+  if (T.rows <= 0) return;   // a padding entry of the table
   T.n = (int)td[2];
   T.cb = (int)td[3];
   T.ce = (int)td[4];
@@ -1123,14 +1153,14 @@ extern "C" int tace_seg_linear_presplit_frag(const float* x, float* y, const flo
                                              const float* bias,
                                              const int64_t* tiles, int64_t n_tiles, const int64_t* contribs,
                                              int32_t aligned, double alpha, void* stream) {
-  if (n_tiles < 0 || n_tiles > 0x7ffffff0) return tace_fail_msg("tace_seg_linear_presplit_frag: bad tile count");
+  if (n_tiles < 0 || n_tiles > 0x7ffffff) return tace_fail_msg("tace_seg_linear_presplit_frag: bad tile count");
   if (n_tiles == 0) return 0;
   if (!x || !y || !w_frag || !tiles || !contribs) return tace_fail_msg("tace_seg_linear_presplit_frag: null pointer");
   if (addend && alpha == 0.0) return tace_fail_msg("tace_seg_linear_presplit_frag: an addend needs alpha != 0");
   if ((((uintptr_t)w_frag) & 15) != 0)
     return tace_fail_msg("tace_seg_linear_presplit_frag: fragment-order weights must be 16-byte aligned");
   const int per = (int)((n_tiles + 7) / 8);
-  const dim3 g((unsigned)(8 * per)), b(256);
+  const dim3 g((unsigned)(16 * per)), b(256);   // two 64-row halves per tile
   if (aligned && (((uintptr_t)x) & 15) == 0)
     hipLaunchKernelGGL((k_seg_linear_bx3f<true, false>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag,
@@ -1149,7 +1179,7 @@ extern "C" int tace_seg_linear_presplit_frag_split(const float* x, float* y, con
                                                    double alpha, void* stream) {
   if (n_tiles < 0 || n_tiles > 0x7ffffff0) return tace_fail_msg("tace_seg_linear_presplit_frag_split: bad tile count");
   if (splits < 2 || splits > 64) return tace_fail_msg("tace_seg_linear_presplit_frag_split: 2..64 splits");
-  if (n_tiles * splits > 0x7ffffff0 || n_tiles > 0x7ffffff)
+  if (n_tiles * splits > 0x7ffffff || n_tiles > 0x7ffffff)
     return tace_fail_msg("tace_seg_linear_presplit_frag_split: too many work items");
   if (n_tiles == 0) return 0;
   if (!x || !y || !w_frag || !tiles || !contribs || !partials)
@@ -1161,7 +1191,7 @@ extern "C" int tace_seg_linear_presplit_frag_split(const float* x, float* y, con
     return tace_fail_msg("tace_seg_linear_presplit_frag_split: partials hold fewer than n_tiles * splits * 16384 floats");
   const int64_t items = n_tiles * splits;
   const int per = (int)((items + 7) / 8);
-  const dim3 g((unsigned)(8 * per)), b(256);
+  const dim3 g((unsigned)(16 * per)), b(256);   // two 64-row halves per item
   if (aligned && (((uintptr_t)x) & 15) == 0)
     hipLaunchKernelGGL((k_seg_linear_bx3f<true, true>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag, bias, tiles, contribs, (float)alpha, (int)n_tiles, per,

@@ -1739,32 +1739,72 @@ SEG_KS_CHUNK = 1024
 # (tace_seg_linear_presplit_frag) when every instruction has a
 # fragment-order block; False: the planes of tace_seg_linear_presplit
 SEG_TILE_FRAG = True
-# fragment-order tile launches of at most SEG_SPLIT_MAX_TILES tiles (too
-# few to fill the GPU) may split each tile's k over several workgroups
+# fragment-order tile launches of at most SEG_SPLIT_MAX_WORK workgroups (too
+# few to fill the GPU) may split each tile's k over several
 # (tace_seg_linear_presplit_frag_split): SEG_SPLIT_SLOTS is the number of
-# tile workgroups the GPU runs at once (two per CU; None: never split), a
-# split takes at least SEG_SPLIT_MIN_STEPS 32-k steps.  Measured: the
-# 1,024-atom alloy's model step 3.24 -> 2.90 ms; the ragged batch's 342-tile
-# launches were slower split (uneven tile heights), hence the tile limit
-SEG_SPLIT_SLOTS = 512
+# workgroups (64 rows of a tile) the GPU runs at once (three per CU; None:
+# never split), a split takes at least SEG_SPLIT_MIN_STEPS 32-k steps.
+# Measured at 1,024 rows, 4 species, k 2,944-5,376 into 128 columns: 7-8
+# splits 153 us, unsplit 239 us; launches of more workgroups than the limit
+# were slower split (342 tiles of uneven heights: 62.4 against 61.6 ms a step)
+SEG_SPLIT_SLOTS = 768
 SEG_SPLIT_MIN_STEPS = 8
-SEG_SPLIT_MAX_TILES = 192
+SEG_SPLIT_MAX_WORK = 384
+# launches whose weights exceed the 256 MB Infinity Cache split long k too,
+# into ranges of about SEG_STREAM_STEPS steps: the row tiles of one weight
+# block then read it at nearly the same time (k_seg_linear_bx3f).  5,003 /
+# 13,000 rows of 89 species, k 5,888-10,752 into 256 columns (4.8 GB of
+# weights), us: 1 split 3451 / 6625, 2 splits 2984 / 6371, 4 splits 2710 /
+# 5789, 8 splits 2723 / 5925; k 1,024-1,792 there: 582, 582, 651, 756; 12,288
+# rows of 2 species, k 2,944-5,376 into 128 columns (27 MB): 1436, 1468, 1414,
+# 1565
+SEG_STREAM_BYTES = 256 << 20
+SEG_STREAM_STEPS = 84
 
 
-def seg_split_count(n_tiles: int, nks_min: int, nks_max: int) -> int:
-    """Splits per tile (1: none) for n_tiles tiles of nks_min .. nks_max
+def seg_split_count(n_work: int, nks_min: int, nks_max: int) -> int:
+    """Splits per tile (1: none) for n_work workgroups of nks_min .. nks_max
     32-k steps: the fewest time units by a model in which the launch runs in
     rounds of SEG_SPLIT_SLOTS workgroups, a workgroup takes one unit per step
     plus one, and the partial sums' launch takes two."""
-    if SEG_SPLIT_SLOTS is None or n_tiles <= 0 or n_tiles > SEG_SPLIT_MAX_TILES:
+    if SEG_SPLIT_SLOTS is None or n_work <= 0 or n_work > SEG_SPLIT_MAX_WORK:
         return 1
     slots = int(SEG_SPLIT_SLOTS)
-    best, best_c = 1, -(-n_tiles // slots) * (nks_max + 1)
+    best, best_c = 1, -(-n_work // slots) * (nks_max + 1)
     for S in range(2, min(64, nks_min // max(1, SEG_SPLIT_MIN_STEPS)) + 1):
-        c = -(-n_tiles * S // slots) * (-(-nks_max // S) + 1) + 2
+        c = -(-n_work * S // slots) * (-(-nks_max // S) + 1) + 2
         if c < best_c:
             best, best_c = S, c
     return best
+
+
+# tables of at least this many entries are cut into runs of equal cost
+# (_xcd_balanced); shorter ones fill the XCDs unevenly whatever the cut
+SEG_BALANCE_MIN = 64
+
+
+def _xcd_balanced(table: np.ndarray, cost: np.ndarray, length: np.ndarray, runs: int = 8) -> np.ndarray:
+    """``table`` for launches in which XCD x works through entries x per ..
+    (x + 1) per - 1: eight contiguous runs (8 / splits where every split of k
+    goes through the table) of equal total cost instead of equal length
+    (neighbours share operands in their XCD's L2, so the runs
+    stay contiguous), in each run the entries of the greatest ``length``
+    (steps: the same for all row tiles of a weight block, so they stay
+    together) first, padded to the longest run with entries of 0 rows that
+    the kernels skip.  Equal lengths
+    left the XCDs with the long-k blocks working while the others were done:
+    of 12,288 rows' k = 2,944-5,376 blocks the busiest XCD had 1.14 times the
+    mean, of a [128 -> 768, 256 x 3] linear 1.5 times (114 -> 75 us)."""
+    cum = np.cumsum(cost)
+    # an entry belongs to the run its cost's midpoint falls in
+    run = np.minimum((cum - 0.5 * cost) * runs // cum[-1], runs - 1).astype(np.int64)
+    counts = np.bincount(run, minlength=runs)
+    per, starts = int(counts.max()), np.concatenate([[0], np.cumsum(counts)])
+    out = np.zeros((runs * per, table.shape[1]), dtype=table.dtype)
+    for x in range(runs):
+        mine = np.arange(starts[x], starts[x + 1])
+        out[x * per:x * per + len(mine)] = table[mine[np.argsort(-length[mine], kind="stable")]]
+    return out
 
 
 class SegLinearPlan:
@@ -1874,8 +1914,14 @@ class SegLinearPlan:
         # to fill the GPU (fragment-order tiles with one contribution each)
         self.splits = 1
         if self.tile_frag and len(t) and ((t[:, 6] - t[:, 5]) == 1).all():
-            nks = (c[t[:, 5], 1] + 31) // 32
-            self.splits = seg_split_count(len(t), int(nks.min()), int(nks.max()))
+            mine = c[t[:, 5]]
+            nks = (mine[:, 1] + 31) // 32
+            self.splits = seg_split_count(int(((t[:, 1] + 63) // 64).sum()), int(nks.min()), int(nks.max()))
+            _, first = np.unique(mine[:, 2], return_index=True)
+            wbytes = 6 * int(((t[first, 2] + 15) // 16 * 16 * nks[first] * 32).sum())
+            if self.splits == 1 and SEG_SPLIT_SLOTS is not None and wbytes > SEG_STREAM_BYTES:
+                q = 1 << max(0, min(3, round(math.log2(int(nks.max()) / SEG_STREAM_STEPS))))
+                self.splits = q if int(nks.min()) >= q * SEG_SPLIT_MIN_STEPS else 1
         self.x_numel, self.y_numel, self.w_numel, self.b_numel = x_numel, y_numel, w_numel, b_numel
         # multiply-adds x 2 of the whole launch (rows x valid columns x summed k
         # of every tile): the algorithmic flops of the GEMMs, padding excluded
@@ -1883,6 +1929,13 @@ class SegLinearPlan:
         if len(t) and len(c):
             ksum = np.concatenate([[0], np.cumsum(c[:, 1])])
             self.flops = int(2 * (t[:, 1] * np.minimum(TN, t[:, 2] - t[:, 3]) * (ksum[t[:, 6]] - ksum[t[:, 5]])).sum())
+        if self.tile_frag and 8 % self.splits == 0 and len(t) >= SEG_BALANCE_MIN:
+            # a tile costs its 32-k steps (and about four for its start and
+            # stores) per 64 rows
+            steps = np.concatenate([[0], np.cumsum((c[:, 1] + 31) // 32)])
+            steps = steps[t[:, 6]] - steps[t[:, 5]] + 4
+            t = _xcd_balanced(t, steps * ((t[:, 1] + 63) // 64), steps, 8 // self.splits)
+            self.n_tiles = len(t)
         self.tiles = torch.from_numpy(np.ascontiguousarray(t)).to(device)
         self.contribs = torch.from_numpy(np.ascontiguousarray(c) if len(c) else np.zeros((1, 4), np.int64)).to(device)
         self.scales = torch.from_numpy(s if len(s) else np.zeros(1)).to(device)
@@ -1917,6 +1970,10 @@ class SegLinearPlan:
                         raise ValueError("seg linear plan: a task is taller than its kernel's tile")
                     if (sel[:, 7] > (128 if R == 128 else 256)).any():
                         raise ValueError("seg linear plan: a task's k exceeds its kernel's limit")
+                    if len(sel) >= SEG_BALANCE_MIN:
+                        # a task costs its columns' 32-k steps and about two for their stores
+                        cost = (sel[:, 4] - sel[:, 3]) * ((sel[:, 7] + 31) // 32 + 2)
+                        sel = _xcd_balanced(sel, cost, cost)
                     self.ks_groups.append((R, len(sel), torch.from_numpy(np.ascontiguousarray(sel)).to(device)))
 
     @staticmethod
