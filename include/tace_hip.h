@@ -593,6 +593,56 @@ int tace_so2_gemm_bf16_kt(const uint16_t* a, int64_t lda, const uint16_t* b_frag
 int tace_edge_pairs(const int32_t* rowptr, const int32_t* eid, const int32_t* src, const int32_t* shifts,
                     int64_t n_nodes, int64_t n_edges, int32_t* work, int32_t* w_rows, int32_t* row_edges,
                     int32_t* row_partner, void* stream);
+/* Positions 0 .. n-1 grouped by key (torch.argsort(stable=True) of the
+ * receivers, and bincount + cumsum): key i is keys[(through ? through[i] : i)
+ * * stride], of key_bytes 4 or 8.  keys32 [n]: the keys (-1 outside [0,
+ * n_keys)); rowptr [n_keys + 1] and order [n]: the positions in key order,
+ * ascending within a key (positions with a key outside the range take no
+ * part).  other (may be NULL): n more keys, other[i * other_stride], checked
+ * against the same range and converted into other32 [n] (an edge list's
+ * senders).  flags (int32 [2], may be NULL): [0] nonzero if some key or other
+ * key is outside the range, [1] if the keys are not ascending.  work:
+ * tace_group_keys_work int32. */
+int64_t tace_group_keys_work(int64_t n, int64_t n_keys);
+int tace_group_keys(int key_bytes, const void* keys, int64_t stride, const int32_t* through, int64_t n, int64_t n_keys,
+                    int32_t* keys32, int32_t* rowptr, int32_t* order, const void* other, int64_t other_stride,
+                    int32_t* other32, int32_t* work, int32_t* flags, void* stream);
+
+/* The gate of n_blocks blocks l = 0 .. n_blocks - 1 (O3Gate with gate_m0,
+ * tace/models/_e3nn/nonlinear.py:27-42, 93-143) on group-major features: x =
+ * [n, (n_blocks + 1) C] (one run of C gates per block, then the l = 0
+ * features) and the blocks [n, 2l + 1, C] of l >= 1; out = cst sigmoid(gate_l)
+ * x_l as blocks [n, 2l + 1, C].  1..4 blocks; _bwd: the input gradient. */
+int tace_gate_fwd(int dtype, const void* x, int64_t n_nodes, int32_t channels, int32_t n_blocks, double cst, void* out,
+                  void* stream);
+int tace_gate_bwd(int dtype, const void* x, const void* g_out, int64_t n_nodes, int32_t channels, int32_t n_blocks,
+                  double cst, void* g_x, void* stream);
+
+/* The scalar readout with 16 hidden values, the element tables and the
+ * per-graph sums (tace/models/_e3nn/readout.py:36-84, blocks.py:250-379,
+ * _e3nn/tace.py:356-418).  Node a's features are row row_of[a] of x [n,
+ * channels]; with h = x w1 (w1 [channels, 16], scaled) its readout is e =
+ * sum_j w2_j silu(h_j); its energy is attrs[a] . e0 + e (attrs[a] . scale) +
+ * attrs[a] . shift, scale and shift dropped for an atom alone in its graph
+ * (ptr [n_graphs + 1], batch [n]) without edges (receiver CSR rowptr [n +
+ * 1]).  Writes hid [n, 16], vals [n, 2], factor [n] (kept for the gradient),
+ * node_energy [n] and energy [n_graphs] (fixed summation order).  _bwd: g_x
+ * rows from g_energy [n_graphs] and g_node [n] (either may be NULL). */
+int tace_energy_head_fwd(int dtype, const void* x, const int64_t* row_of, const void* w1, const void* w2,
+                         int64_t n_nodes, int32_t channels, const void* attrs, int32_t n_species, const void* e0,
+                         const void* scale, const void* shift, const int64_t* batch, const int64_t* ptr,
+                         const int32_t* rowptr, int64_t n_graphs, void* hid, void* vals, void* factor,
+                         void* node_energy, void* energy, void* stream);
+int tace_energy_head_bwd(int dtype, const void* hid, const void* factor, const void* g_energy, const void* g_node,
+                         const int64_t* row_of, const int64_t* batch, const void* w1, int64_t n_nodes,
+                         int32_t channels, void* g_x, void* stream);
+
+/* tace_edge_vec_bwd with the lattice's share: g_lat [n_nodes, 9] receives
+ * sum over the edges e node n sends of shifts[e] (x) g_vec[e] (row-major),
+ * whose sums over a graph's nodes are the gradient of its lattice. */
+int tace_edge_vec_lat_bwd(int dtype, const void* g_vec, const void* shifts, const int32_t* rowptr, const int32_t* eid,
+                          const int32_t* s_rowptr, const int32_t* s_slot, int64_t n_nodes, void* g_pos, void* g_lat,
+                          void* stream);
 /* exclusive prefix sum: out[0] = 0, out[i+1] = out[i] + counts[i], i < n */
 int tace_scan_i32(const int32_t* counts, int64_t n, int32_t* out, void* stream);
 

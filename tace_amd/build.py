@@ -59,7 +59,7 @@ def build(verbose: bool = True, force: bool = True, jobs: int = 0) -> str:
     # the longest translation units first
     srcs = [os.path.join(CSRC, n) for n in ("tece_rotin.hip", "tece_rotout.hip", "tece_ace.hip", "linear.hip",
                                             "tace_hip.hip", "tece_score.hip", "tece_wigner.hip", "mlp.hip",
-                                            "so2_gemm.hip")] + generate()
+                                            "so2_gemm.hip", "nodewise.hip", "group.hip")] + generate()
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     jobs = jobs or min(16, os.cpu_count() or 4)

@@ -240,30 +240,59 @@ __global__ __launch_bounds__(256) void k_edge_vec_fwd(const T* __restrict__ pos,
     vec[3 * e + c] = pos[3 * j + c] - pos[3 * i + c] + (s0 * L[c] + s1 * L[3 + c] + s2 * L[6 + c]);
 }
 
-// gpos[n] = sum_{e: dst(e)=n} g[e] - sum_{e: src(e)=n} g[e], both in CSR order
-template <typename T>
-__global__ __launch_bounds__(256) void k_edge_vec_bwd(const T* __restrict__ g, const int* __restrict__ rowptr,
-                                                      const int* __restrict__ eid, const int* __restrict__ s_rowptr,
-                                                      const int* __restrict__ s_slot, int n, T* __restrict__ gpos) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= n) return;
-  T x = T(0), y = T(0), z = T(0);
-  for (int k = rowptr[a]; k < rowptr[a + 1]; ++k) {
-    const int e = eid ? eid[k] : k;
-    x += g[3 * e];
-    y += g[3 * e + 1];
-    z += g[3 * e + 2];
+// gpos[n] = sum_{e: dst(e)=n} g[e] - sum_{e: src(e)=n} g[e], and with LAT
+// glat[n] = sum_{e: src(e)=n} S[e] (x) g[e].  16 lanes per node, lane q taking
+// every 16th edge of its CSR ranges, then a tree over the lanes (a fixed
+// order).  The gathers' latency bounds it: with a thread per node the edges
+// of a node came one after the other (41 us at 1,024 nodes of 45 edges, 99 us
+// at 12,288 of 87; now 5.5 and 22 us).  The lattice's share per sender needs
+// no sort of the edges by graph: as a row sum over the edges of each graph (one
+// workgroup per graph) it took 2.57 ms for 64 crystals of 360k edges, now 13 us.
+template <typename T, bool LAT>
+__global__ __launch_bounds__(256) void k_edge_vec_bwd(const T* __restrict__ g, const T* __restrict__ shift,
+                                                      const int* __restrict__ rowptr, const int* __restrict__ eid,
+                                                      const int* __restrict__ s_rowptr,
+                                                      const int* __restrict__ s_slot, int n, T* __restrict__ gpos,
+                                                      T* __restrict__ glat) {
+  const int a = (int)(blockIdx.x * 16 + (threadIdx.x >> 4)), q = (int)(threadIdx.x & 15);
+  if (a >= n) return;   // all 16 lanes of a node leave together
+  T p[3] = {T(0), T(0), T(0)}, m[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) m[i] = T(0);
+  for (int k = rowptr[a] + q; k < rowptr[a + 1]; k += 16) {
+    const int64_t e = eid ? eid[k] : k;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) p[c] += g[3 * e + c];
   }
-  for (int k = s_rowptr[a]; k < s_rowptr[a + 1]; ++k) {
+  for (int k = s_rowptr[a] + q; k < s_rowptr[a + 1]; k += 16) {
     const int sl = s_slot[k];
-    const int e = eid ? eid[sl] : sl;
-    x -= g[3 * e];
-    y -= g[3 * e + 1];
-    z -= g[3 * e + 2];
+    const int64_t e = eid ? eid[sl] : sl;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const T v = g[3 * e + c];
+      p[c] -= v;
+      if constexpr (LAT) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) m[3 * r + c] += shift[3 * e + r] * v;
+      }
+    }
   }
-  gpos[3 * a] = x;
-  gpos[3 * a + 1] = y;
-  gpos[3 * a + 2] = z;
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) p[c] += __shfl_xor(p[c], o, 64);
+    if constexpr (LAT) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) m[i] += __shfl_xor(m[i], o, 64);
+    }
+  }
+  if (q < 3) gpos[3 * (int64_t)a + q] = q == 0 ? p[0] : q == 1 ? p[1] : p[2];
+  if constexpr (LAT) {
+    if (q == 0) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) glat[9 * (int64_t)a + i] = m[i];
+    }
+  }
 }
 
 // ------------------------------------------------------ edge featurisation --
@@ -1333,22 +1362,48 @@ int tace_edge_vec_fwd(int dtype, const void* pos, const void* lattice, const int
   return check_launch("tace_edge_vec_fwd");
 }
 
+static int edge_vec_bwd(const char* who, int dtype, const void* g_vec, const void* shifts, const int32_t* rowptr,
+                        const int32_t* eid, const int32_t* s_rowptr, const int32_t* s_slot, int64_t n_nodes,
+                        void* g_pos, void* g_lat, hipStream_t s) {
+  const dim3 g((unsigned)((n_nodes + 15) / 16)), b(256);
+  if (dtype == TACE_F32) {
+    if (g_lat)
+      hipLaunchKernelGGL((k_edge_vec_bwd<float, true>), g, b, 0, s, (const float*)g_vec, (const float*)shifts, rowptr,
+                         eid, s_rowptr, s_slot, (int)n_nodes, (float*)g_pos, (float*)g_lat);
+    else
+      hipLaunchKernelGGL((k_edge_vec_bwd<float, false>), g, b, 0, s, (const float*)g_vec, (const float*)nullptr, rowptr,
+                         eid, s_rowptr, s_slot, (int)n_nodes, (float*)g_pos, (float*)nullptr);
+  } else {
+    if (g_lat)
+      hipLaunchKernelGGL((k_edge_vec_bwd<double, true>), g, b, 0, s, (const double*)g_vec, (const double*)shifts,
+                         rowptr, eid, s_rowptr, s_slot, (int)n_nodes, (double*)g_pos, (double*)g_lat);
+    else
+      hipLaunchKernelGGL((k_edge_vec_bwd<double, false>), g, b, 0, s, (const double*)g_vec, (const double*)nullptr,
+                         rowptr, eid, s_rowptr, s_slot, (int)n_nodes, (double*)g_pos, (double*)nullptr);
+  }
+  return check_launch(who);
+}
+
 int tace_edge_vec_bwd(int dtype, const void* g_vec, const int32_t* rowptr, const int32_t* eid,
                       const int32_t* s_rowptr, const int32_t* s_slot, int64_t n_nodes, void* g_pos, void* stream) {
-  if (n_nodes < 0 || n_nodes > INT32_MAX) return fail("tace_edge_vec_bwd: bad sizes");
+  if (n_nodes < 0 || n_nodes > INT32_MAX - 16) return fail("tace_edge_vec_bwd: bad sizes");
   if (n_nodes == 0) return 0;
   if (!g_vec || !rowptr || !s_rowptr || !s_slot || !g_pos) return fail("tace_edge_vec_bwd: null pointer");
-  const dim3 g((unsigned)((n_nodes + 255) / 256)), b(256);
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == TACE_F32)
-    hipLaunchKernelGGL(k_edge_vec_bwd<float>, g, b, 0, s, (const float*)g_vec, rowptr, eid, s_rowptr, s_slot,
-                       (int)n_nodes, (float*)g_pos);
-  else if (dtype == TACE_F64)
-    hipLaunchKernelGGL(k_edge_vec_bwd<double>, g, b, 0, s, (const double*)g_vec, rowptr, eid, s_rowptr, s_slot,
-                       (int)n_nodes, (double*)g_pos);
-  else
-    return fail("tace_edge_vec_bwd: dtype must be TACE_F32 or TACE_F64");
-  return check_launch("tace_edge_vec_bwd");
+  if (dtype != TACE_F32 && dtype != TACE_F64) return fail("tace_edge_vec_bwd: dtype must be TACE_F32 or TACE_F64");
+  return edge_vec_bwd("tace_edge_vec_bwd", dtype, g_vec, nullptr, rowptr, eid, s_rowptr, s_slot, n_nodes, g_pos,
+                      nullptr, (hipStream_t)stream);
+}
+
+int tace_edge_vec_lat_bwd(int dtype, const void* g_vec, const void* shifts, const int32_t* rowptr, const int32_t* eid,
+                          const int32_t* s_rowptr, const int32_t* s_slot, int64_t n_nodes, void* g_pos, void* g_lat,
+                          void* stream) {
+  if (n_nodes < 0 || n_nodes > INT32_MAX - 16) return fail("tace_edge_vec_lat_bwd: bad sizes");
+  if (n_nodes == 0) return 0;
+  if (!g_vec || !shifts || !rowptr || !s_rowptr || !s_slot || !g_pos || !g_lat)
+    return fail("tace_edge_vec_lat_bwd: null pointer");
+  if (dtype != TACE_F32 && dtype != TACE_F64) return fail("tace_edge_vec_lat_bwd: dtype must be TACE_F32 or TACE_F64");
+  return edge_vec_bwd("tace_edge_vec_lat_bwd", dtype, g_vec, shifts, rowptr, eid, s_rowptr, s_slot, n_nodes, g_pos,
+                      g_lat, (hipStream_t)stream);
 }
 
 int64_t tace_nl_workspace_bytes(int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff) {

@@ -199,8 +199,11 @@ class EdgePlan:
         """(s_rowptr int32 [N+1], s_slot int32 [E]): receiver-sorted slots grouped
         by sender, stable -- the fixed order of the grad_x segmented sum."""
         if self._sender is None:
-            slot_src = self.src if self.eid is None else self.src[self.eid.long()]
-            self._sender = group_by_key(slot_src, self.n_nodes)
+            if self.src.is_cuda:
+                self._sender = _group_keys(self.src, self.n_nodes, through=self.eid)[1:3]
+            else:
+                slot_src = self.src if self.eid is None else self.src[self.eid.long()]
+                self._sender = group_by_key(slot_src, self.n_nodes)
         return self._sender
 
     def edge_pairs(self, shifts: torch.Tensor) -> "EdgePairs":
@@ -214,6 +217,16 @@ class EdgePlan:
     def from_edge_index(edge_index: torch.Tensor, n_nodes: int) -> "EdgePlan":
         src, dst = edge_index[0], edge_index[1]
         E = int(src.shape[0])
+        if (E and dst.is_cuda and src.dtype == dst.dtype and dst.dtype in (torch.int64, torch.int32)
+                and max(E, n_nodes) < 2 ** 31 - 8192):
+            # one grouping kernel sequence checks, converts and groups the
+            # edges; the host reads its two flags (the only wait)
+            flags = torch.empty(2, dtype=torch.int32, device=dst.device)
+            _, rowptr, order, src32 = _group_keys(dst, n_nodes, other=src, flags=flags)
+            bad, unsorted = flags.tolist()
+            if bad:
+                raise ValueError("edge_index refers to nodes outside [0, n_nodes)")
+            return EdgePlan(n_nodes, E, rowptr, src32, order if unsorted else None)
         if E and (int(torch.minimum(src.min(), dst.min())) < 0
                   or int(torch.maximum(src.max(), dst.max())) >= n_nodes):
             raise ValueError("edge_index refers to nodes outside [0, n_nodes)")
@@ -1319,10 +1332,9 @@ def scatter_add_rows(out: torch.Tensor, index: torch.Tensor, src: torch.Tensor) 
 
 def group_by_key(keys: torch.Tensor, n_keys: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """(rowptr int32 [n_keys+1], order int32 [E]) of keys in [0, n_keys): the
-    positions grouped by key, in position order within a key (a stable sort
-    of 32-bit keys, half the radix passes of 64-bit ones), and each key's
-    range from a binary search of the sorted keys (no atomics, no host
-    synchronisation)."""
+    positions grouped by key, in position order within a key, and each key's
+    range (no host synchronisation): ``tace_group_keys`` on the GPU, a stable
+    sort and a binary search of the sorted keys elsewhere."""
     if n_keys >= 2 ** 31:
         raise ValueError("group_by_key: more than 2^31 keys")
     k32 = keys.to(torch.int32)
@@ -1397,6 +1409,29 @@ def tece_score(q: Sequence[torch.Tensor], k: Sequence[torch.Tensor], radial_proj
     """Radial-rotary complex QK score [E, heads] of query / key in the SO(2)
     block layout (tscale = attention scale x temperature)."""
     if tscale.requires_grad:
+def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor] = None,
+                other: Optional[torch.Tensor] = None, flags: Optional[torch.Tensor] = None):
+    """``tace_group_keys`` on 1-D GPU keys (any stride; ``through``: int32
+    positions the keys are read at): (keys int32, rowptr int32 [n_keys + 1],
+    order int32, ``other`` as int32 or None); ``flags`` int32 [2] receives
+    (some key out of range, keys not ascending)."""
+    n, dev = int((keys if through is None else through).shape[0]), keys.device
+    k32, order = torch.empty(2, n, dtype=torch.int32, device=dev)
+    rowptr = torch.empty(n_keys + 1, dtype=torch.int32, device=dev)
+    L = N.lib()
+    work = torch.empty(L.tace_group_keys_work(n, n_keys), dtype=torch.int32, device=dev)
+    o32 = torch.empty(n, dtype=torch.int32, device=dev) if other is not None else None
+    if through is not None:
+        _req(through, "through", torch.int32, (n,))
+    if other is not None and (other.shape != keys.shape or other.dtype != keys.dtype):
+        raise ValueError("group keys: the second keys differ from the first in shape or dtype")
+    N.check(L.tace_group_keys(keys.element_size(), keys.data_ptr(), keys.stride(0), N.ptr(through), n, n_keys,
+                              k32.data_ptr(), rowptr.data_ptr(), order.data_ptr(), N.ptr(other),
+                              0 if other is None else other.stride(0), N.ptr(o32), work.data_ptr(), N.ptr(flags),
+                              N.stream_ptr(dev)), "tace_group_keys")
+    return k32, rowptr, order, o32
+
+
         raise ValueError("tece_score: the temperature gradient is not computed (parameters must be frozen)")
     C = q[0].shape[1] // (lmax + 1)
     return _TeceScore.apply(radial_proj.contiguous(), tscale.contiguous(), int(lmax), int(heads), C,
@@ -1405,6 +1440,9 @@ def tece_score(q: Sequence[torch.Tensor], k: Sequence[torch.Tensor], radial_proj
 
 class _GraphSoftmax(torch.autograd.Function):
     @staticmethod
+    if (keys.is_cuda and keys.dim() == 1 and keys.dtype in (torch.int64, torch.int32)
+            and max(n_keys, keys.shape[0]) < 2 ** 31 - 8192):
+        return _group_keys(keys, n_keys)[1:3]
     def forward(ctx, s, plan: EdgePlan):
         a = launch_softmax_fwd(s, plan)
         ctx.save_for_backward(a)
