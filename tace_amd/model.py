@@ -1640,7 +1640,9 @@ class TensorModel(torch.nn.Module):
         if dst32 is None:
             dst32 = ei[1].to(torch.int32)
         egraph = None if (num_graphs == 1 and not ops.MODE.export) else batch[ei[0]].to(torch.int32)
-        vec = ops.edge_vectors(pos_s, lat_s, shifts, plan, dst32, egraph)
+        ptr = data["ptr"]
+        lat_ptr = ptr if ptr.dtype == torch.int64 and lat_s.shape[0] == num_graphs else None
+        vec = ops.edge_vectors(pos_s, lat_s, shifts, plan, dst32, egraph, lat_ptr)
         E, e_node = self.readout_fn.energy(data, plan, vec, pairs=pairs)
         out: Dict[str, Optional[torch.Tensor]] = dict(energy=E, node_energy=e_node, forces=None, virials=None,
                                                       stress=None, edge_forces=None, atomic_virials=None,

@@ -643,7 +643,7 @@ def edge_rtp_scatter(x, y, h, W, alpha: float, plan: EdgePlan, var: TpVariant, C
 # ------------------------------------------------------------ edge vectors ----
 class _EdgeVectors(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, pos, lattice, shifts, plan: EdgePlan, dst: torch.Tensor, edge_graph):
+    def forward(ctx, pos, lattice, shifts, plan: EdgePlan, dst: torch.Tensor, edge_graph, ptr=None):
         E = plan.n_edges
         dt = pos.dtype
         _req(pos, "positions", dt, (plan.n_nodes, 3))
@@ -654,7 +654,7 @@ class _EdgeVectors(torch.autograd.Function):
                                           dst.data_ptr(), shifts.data_ptr(), N.ptr(edge_graph), E, vec.data_ptr(),
                                           N.stream_ptr(pos.device)), "tace_edge_vec_fwd")
         ctx.save_for_backward(shifts)
-        ctx.plan, ctx.edge_graph, ctx.nlat = plan, edge_graph, lattice.shape[0]
+        ctx.plan, ctx.edge_graph, ctx.nlat, ctx.ptr = plan, edge_graph, lattice.shape[0], ptr
         return vec
 
     @staticmethod
@@ -667,6 +667,16 @@ class _EdgeVectors(torch.autograd.Function):
             # no edge: every receiver and sender sum is empty (and the empty
             # per-edge tensors have no device pointer for the kernel)
             gpos = torch.zeros(plan.n_nodes, 3, dtype=g.dtype, device=g.device)
+        elif ctx.needs_input_grad[1] and ctx.ptr is not None and plan.n_edges:
+            # the lattice's share summed per sender, then over each graph's nodes
+            s_rowptr, s_slot = plan.sender_csr()
+            gpos = torch.empty(plan.n_nodes, 3, dtype=g.dtype, device=g.device)
+            gnode = torch.empty(plan.n_nodes, 9, dtype=g.dtype, device=g.device)
+            N.check(N.lib().tace_edge_vec_lat_bwd(N.dtype_code(g.dtype), g.data_ptr(), shifts.data_ptr(),
+                                                  plan.rowptr.data_ptr(), N.ptr(plan.eid), s_rowptr.data_ptr(),
+                                                  s_slot.data_ptr(), plan.n_nodes, gpos.data_ptr(), gnode.data_ptr(),
+                                                  N.stream_ptr(g.device)), "tace_edge_vec_lat_bwd")
+            glat = _graph_sum(gnode, ctx.ptr).view(-1, 3, 3)
         elif ctx.needs_input_grad[0]:
             s_rowptr, s_slot = plan.sender_csr()
             gpos = torch.empty(plan.n_nodes, 3, dtype=g.dtype, device=g.device)
@@ -674,20 +684,23 @@ class _EdgeVectors(torch.autograd.Function):
                                               N.ptr(plan.eid), s_rowptr.data_ptr(), s_slot.data_ptr(),
                                               plan.n_nodes, gpos.data_ptr(), N.stream_ptr(g.device)),
                     "tace_edge_vec_bwd")
-        if ctx.needs_input_grad[1]:
+        if ctx.needs_input_grad[1] and glat is None:
             outer = (shifts.unsqueeze(2) * g.unsqueeze(1)).reshape(-1, 9)
             if ctx.edge_graph is None:
                 glat = outer.sum(0).view(1, 3, 3)
             else:
                 glat = scatter_add_rows(torch.zeros(ctx.nlat, 9, dtype=g.dtype, device=g.device),
                                         ctx.edge_graph.long(), outer).view(-1, 3, 3)
-        return gpos, glat, None, None, None, None
+        return gpos, glat, None, None, None, None, None
 
 
-def edge_vectors(pos, lattice, shifts, plan: EdgePlan, dst: torch.Tensor, edge_graph=None) -> torch.Tensor:
+def edge_vectors(pos, lattice, shifts, plan: EdgePlan, dst: torch.Tensor, edge_graph=None, ptr=None) -> torch.Tensor:
     """vec[e] = pos[dst] - pos[src] + shifts[e] . lattice[edge_graph[e]]
     (``tace/models/adapter.py:334-340``) with a deterministic CSR backward.
-    ``dst`` int32 [E] in edge-id order; ``edge_graph`` int32 [E] or None (one graph)."""
+    ``dst`` int32 [E] in edge-id order; ``edge_graph`` int32 [E] or None (one
+    graph).  ``ptr`` (int64 [graphs + 1], optional): the graphs' node ranges,
+    when edge_graph is the graph of each edge's sender and lattice has one row
+    per graph; the lattice gradient is then summed per sender first."""
     if MODE.double:
         # adapter.py:334-340 as torch operations (differentiable to any order)
         L = lattice[edge_graph.long()] if edge_graph is not None else lattice[0].expand(plan.n_edges, 3, 3)
@@ -696,8 +709,10 @@ def edge_vectors(pos, lattice, shifts, plan: EdgePlan, dst: torch.Tensor, edge_g
         dst = dst.to(torch.int32)
     if edge_graph is not None and edge_graph.dtype != torch.int32:
         edge_graph = edge_graph.to(torch.int32)
+    if ptr is not None and ptr.numel() - 1 != lattice.shape[0]:
+        raise ValueError("edge_vectors: ptr and lattice name different numbers of graphs")
     return _EdgeVectors.apply(pos.contiguous(), lattice.contiguous(), shifts.contiguous(), plan, dst.contiguous(),
-                              None if edge_graph is None else edge_graph.contiguous())
+                              None if edge_graph is None else edge_graph.contiguous(), ptr)
 
 
 # ---------------------------------------------------------------- uuu ----
