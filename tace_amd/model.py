@@ -658,7 +658,20 @@ class _GateFn(torch.autograd.Function):
     (e3nn's elementwise product with sqrt(2l+1) W3j(l,0,l) is exactly that)."""
 
     @staticmethod
+    def native(lin: GMLayout, lout: GMLayout, C: int) -> bool:
+        """The layouts of ``tace_gate_fwd``: gated blocks of C channels l = 0,
+        1, .. up to l = 3, the gates and the l = 0 features in block 0."""
+        n = len(lout.blocks)
+        return (n <= 4 and [(m, d) for _, m, d in lout.blocks] == [(C, 2 * l + 1) for l in range(n)]
+                and [(m, d) for _, m, d in lin.blocks] == [((n + 1) * C, 1)] + [(C, 2 * l + 1) for l in range(1, n)])
+
+    @staticmethod
     def forward(ctx, x, lin: GMLayout, lout: GMLayout, C: int):
+        ctx.kernel = x.is_cuda and x.is_contiguous() and _GateFn.native(lin, lout, C)
+        if ctx.kernel:
+            ctx.save_for_backward(x)
+            ctx.lay = (lin, lout, C)
+            return ops.launch_gate_fwd(x, C, len(lout.blocks), SIGMOID_CST)
         Z = x.shape[0]
         ng = len(lout.blocks)
         X0 = lin.block(x, 0).view(Z, -1)
@@ -672,9 +685,12 @@ class _GateFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gout):
-        x, g = ctx.saved_tensors
         lin, lout, C = ctx.lay
         gout = gout.contiguous()
+        if ctx.kernel:
+            (x,) = ctx.saved_tensors
+            return ops.launch_gate_bwd(x, gout, C, len(lout.blocks), SIGMOID_CST), None, None, None
+        x, g = ctx.saved_tensors
         Z = x.shape[0]
         ng = len(lout.blocks)
         gx = torch.empty_like(x)
@@ -1306,6 +1322,17 @@ class TACE(torch.nn.Module):
             dtype=torch.get_default_dtype()))
         self.scale_shift.register_buffer("shift", torch.zeros(len(stats), len(zs), dtype=torch.get_default_dtype()))
 
+    def _head_fits(self, x, attrs, plan, sp) -> bool:
+        """Whether the readout, the element tables and the per-graph sums run
+        on ``ops.EnergyHead``: frozen parameters, one hidden layer of 16, and a
+        receiver CSR over exactly these nodes."""
+        lin = self.energy_readouts[0].linear2
+        return (x.is_cuda and not (ops.MODE.double or ops.MODE.export) and x.dtype in (torch.float32, torch.float64)
+                and attrs.dtype == x.dtype and not attrs.requires_grad and _frozen(self.energy_readouts[0])
+                and len(lin) == 2 and lin[0].weight.numel() == 16 * x.shape[1] and lin[1].weight.numel() == 16
+                and x.shape[1] <= 512 and 0 < x.shape[0] == attrs.shape[0] and sp.inv is not None
+                and isinstance(plan, ops.EdgePlan) and plan.n_nodes == x.shape[0])
+
     def energy(self, data, plan: ops.EdgePlan, edge_vector, exchange=None, pairs: Optional[ops.EdgePairs] = None):
         """Energy branch of ``readout_fn`` (``tace.py:356-418``) + ``ScaleShift``
         (``blocks.py:289-379``), fidelity 0.  ``exchange``: LAMMPS ML-IAP data
@@ -1318,6 +1345,14 @@ class TACE(torch.nn.Module):
         num_graphs = ptr.numel() - 1
         sp = SpeciesPlan(attrs, exchange, pairs, natural=ops.MODE.export, counts=_opt(data, "_species_counts"))
         x = self.representation(attrs, plan, edge_vector, sp, data["edge_index"])
+        if self._head_fits(x, attrs, plan, sp):
+            l1, l2 = self.energy_readouts[0].linear2
+            w1 = l1.weight.detach().view(x.shape[1], 16) * l1.lay.ins[0][5]
+            w2 = l2.weight.detach() * (l2.lay.ins[0][5] * SILU_CST)
+            tab = [t[0].to(x.dtype).contiguous() for t in (self.atomic_energy_layer.atomic_energy, self.scale_shift.scale,
+                                                            self.scale_shift.shift)]
+            return ops.EnergyHead.apply(x.contiguous(), sp.inv, w1, w2, attrs.contiguous(), *tab, batch.contiguous(),
+                                        ptr.contiguous(), plan.rowptr)
         # E0(Z_n) (OneHotToAtomicEnergy, blocks.py:250-286) as a masked row sum (a
         # [N, S] x [S, 1] product would be a library GEMM launch)
         e_base = (attrs * self.atomic_energy_layer.atomic_energy[0]).sum(-1)

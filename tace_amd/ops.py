@@ -836,6 +836,71 @@ def uuu_tp(x1, x2, var: TpVariant, C: int, layout: int = 0, w: Optional[torch.Te
     return _UUU.apply(x1.contiguous(), x2.contiguous(), None if w is None else w.contiguous(), var, C, int(layout))
 
 
+# ------------------------------------------------------------ gate, readout ----
+def launch_gate_fwd(x: torch.Tensor, C: int, n_blocks: int, cst: float) -> torch.Tensor:
+    """``tace_gate_fwd`` on group-major x [n, C (n_blocks + n_blocks^2)]."""
+    n = x.shape[0]
+    _req(x, "x", x.dtype, (n, C * (n_blocks + n_blocks * n_blocks)))
+    out = torch.empty(n, C * n_blocks * n_blocks, dtype=x.dtype, device=x.device)
+    tok = _t0("gate_fwd")
+    N.check(N.lib().tace_gate_fwd(N.dtype_code(x.dtype), x.data_ptr(), n, C, n_blocks, cst, out.data_ptr(),
+                                  N.stream_ptr(x.device)), "tace_gate_fwd")
+    _t1(tok, (n, C, n_blocks))
+    return out
+
+
+def launch_gate_bwd(x: torch.Tensor, g: torch.Tensor, C: int, n_blocks: int, cst: float) -> torch.Tensor:
+    n = x.shape[0]
+    _req(g, "g_out", x.dtype, (n, C * n_blocks * n_blocks))
+    gx = torch.empty_like(x)
+    tok = _t0("gate_bwd")
+    N.check(N.lib().tace_gate_bwd(N.dtype_code(x.dtype), x.data_ptr(), g.data_ptr(), n, C, n_blocks, cst,
+                                  gx.data_ptr(), N.stream_ptr(x.device)), "tace_gate_bwd")
+    _t1(tok, (n, C, n_blocks))
+    return gx
+
+
+class EnergyHead(torch.autograd.Function):
+    """``tace_energy_head_*``: (energy [B], node energies [n]) of last-layer
+    features x [n, C] in rows row_of; every other argument is a constant.
+    w1 [C, 16] and w2 [16] carry their scales."""
+
+    @staticmethod
+    def forward(ctx, x, row_of, w1, w2, attrs, e0, scale, shift, batch, ptr, rowptr):
+        n, C = x.shape
+        dt, dev, S, B = x.dtype, x.device, attrs.shape[1], ptr.numel() - 1
+        _req(x, "x", dt, (n, C))
+        for t, nm, shp in ((w1, "w1", (C, 16)), (w2, "w2", (16,)), (attrs, "attrs", (n, S)), (e0, "e0", (S,)),
+                           (scale, "scale", (S,)), (shift, "shift", (S,))):
+            _req(t, nm, dt, shp)
+        for t, nm in ((row_of, "row_of"), (batch, "batch")):
+            _req(t, nm, torch.int64, (n,))
+        _req(ptr, "ptr", torch.int64, (B + 1,))
+        _req(rowptr, "rowptr", torch.int32, (n + 1,))
+        hid, vals, fac, en, E = (torch.empty(s, dtype=dt, device=dev) for s in ((n, 16), (n, 2), (n,), (n,), (B,)))
+        N.check(N.lib().tace_energy_head_fwd(N.dtype_code(dt), x.data_ptr(), row_of.data_ptr(), w1.data_ptr(),
+                                             w2.data_ptr(), n, C, attrs.data_ptr(), S, e0.data_ptr(),
+                                             scale.data_ptr(), shift.data_ptr(), batch.data_ptr(), ptr.data_ptr(),
+                                             rowptr.data_ptr(), B, hid.data_ptr(), vals.data_ptr(), fac.data_ptr(),
+                                             en.data_ptr(), E.data_ptr(), N.stream_ptr(dev)), "tace_energy_head_fwd")
+        ctx.save_for_backward(hid, fac, row_of, batch, w1)
+        ctx.set_materialize_grads(False)
+        return E, en
+
+    @staticmethod
+    def backward(ctx, gE, gn):
+        if gE is None and gn is None:
+            return (None,) * 11
+        hid, fac, row_of, batch, w1 = ctx.saved_tensors
+        n, C = hid.shape[0], w1.shape[0]
+        gE, gn = (None if g is None else g.contiguous() for g in (gE, gn))
+        gx = torch.empty(n, C, dtype=hid.dtype, device=hid.device)
+        N.check(N.lib().tace_energy_head_bwd(N.dtype_code(hid.dtype), hid.data_ptr(), fac.data_ptr(), N.ptr(gE),
+                                             N.ptr(gn), row_of.data_ptr(), batch.data_ptr(), w1.data_ptr(), n, C,
+                                             gx.data_ptr(), N.stream_ptr(hid.device)), "tace_energy_head_bwd")
+        return (gx,) + (None,) * 10
+
+
 # ---------------------------------------------------------------- TECE ops ----
 class _EdgeWigner(torch.autograd.Function):
     @staticmethod
@@ -1345,6 +1410,29 @@ def scatter_add_rows(out: torch.Tensor, index: torch.Tensor, src: torch.Tensor) 
     return rows_accumulate(out.view(n, -1), src.reshape(E, -1).contiguous(), rp, slot).view(out.shape)
 
 
+def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor] = None,
+                other: Optional[torch.Tensor] = None, flags: Optional[torch.Tensor] = None):
+    """``tace_group_keys`` on 1-D GPU keys (any stride; ``through``: int32
+    positions the keys are read at): (keys int32, rowptr int32 [n_keys + 1],
+    order int32, ``other`` as int32 or None); ``flags`` int32 [2] receives
+    (some key out of range, keys not ascending)."""
+    n, dev = int((keys if through is None else through).shape[0]), keys.device
+    k32, order = torch.empty(2, n, dtype=torch.int32, device=dev)
+    rowptr = torch.empty(n_keys + 1, dtype=torch.int32, device=dev)
+    L = N.lib()
+    work = torch.empty(L.tace_group_keys_work(n, n_keys), dtype=torch.int32, device=dev)
+    o32 = torch.empty(n, dtype=torch.int32, device=dev) if other is not None else None
+    if through is not None:
+        _req(through, "through", torch.int32, (n,))
+    if other is not None and (other.shape != keys.shape or other.dtype != keys.dtype):
+        raise ValueError("group keys: the second keys differ from the first in shape or dtype")
+    N.check(L.tace_group_keys(keys.element_size(), keys.data_ptr(), keys.stride(0), N.ptr(through), n, n_keys,
+                              k32.data_ptr(), rowptr.data_ptr(), order.data_ptr(), N.ptr(other),
+                              0 if other is None else other.stride(0), N.ptr(o32), work.data_ptr(), N.ptr(flags),
+                              N.stream_ptr(dev)), "tace_group_keys")
+    return k32, rowptr, order, o32
+
+
 def group_by_key(keys: torch.Tensor, n_keys: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """(rowptr int32 [n_keys+1], order int32 [E]) of keys in [0, n_keys): the
     positions grouped by key, in position order within a key, and each key's
@@ -1352,6 +1440,9 @@ def group_by_key(keys: torch.Tensor, n_keys: int) -> Tuple[torch.Tensor, torch.T
     sort and a binary search of the sorted keys elsewhere."""
     if n_keys >= 2 ** 31:
         raise ValueError("group_by_key: more than 2^31 keys")
+    if (keys.is_cuda and keys.dim() == 1 and keys.dtype in (torch.int64, torch.int32)
+            and max(n_keys, keys.shape[0]) < 2 ** 31 - 8192):
+        return _group_keys(keys, n_keys)[1:3]
     k32 = keys.to(torch.int32)
     srt, order = torch.sort(k32, stable=True)
     bounds = torch.arange(n_keys + 1, dtype=torch.int32, device=keys.device)
@@ -1424,29 +1515,6 @@ def tece_score(q: Sequence[torch.Tensor], k: Sequence[torch.Tensor], radial_proj
     """Radial-rotary complex QK score [E, heads] of query / key in the SO(2)
     block layout (tscale = attention scale x temperature)."""
     if tscale.requires_grad:
-def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor] = None,
-                other: Optional[torch.Tensor] = None, flags: Optional[torch.Tensor] = None):
-    """``tace_group_keys`` on 1-D GPU keys (any stride; ``through``: int32
-    positions the keys are read at): (keys int32, rowptr int32 [n_keys + 1],
-    order int32, ``other`` as int32 or None); ``flags`` int32 [2] receives
-    (some key out of range, keys not ascending)."""
-    n, dev = int((keys if through is None else through).shape[0]), keys.device
-    k32, order = torch.empty(2, n, dtype=torch.int32, device=dev)
-    rowptr = torch.empty(n_keys + 1, dtype=torch.int32, device=dev)
-    L = N.lib()
-    work = torch.empty(L.tace_group_keys_work(n, n_keys), dtype=torch.int32, device=dev)
-    o32 = torch.empty(n, dtype=torch.int32, device=dev) if other is not None else None
-    if through is not None:
-        _req(through, "through", torch.int32, (n,))
-    if other is not None and (other.shape != keys.shape or other.dtype != keys.dtype):
-        raise ValueError("group keys: the second keys differ from the first in shape or dtype")
-    N.check(L.tace_group_keys(keys.element_size(), keys.data_ptr(), keys.stride(0), N.ptr(through), n, n_keys,
-                              k32.data_ptr(), rowptr.data_ptr(), order.data_ptr(), N.ptr(other),
-                              0 if other is None else other.stride(0), N.ptr(o32), work.data_ptr(), N.ptr(flags),
-                              N.stream_ptr(dev)), "tace_group_keys")
-    return k32, rowptr, order, o32
-
-
         raise ValueError("tece_score: the temperature gradient is not computed (parameters must be frozen)")
     C = q[0].shape[1] // (lmax + 1)
     return _TeceScore.apply(radial_proj.contiguous(), tscale.contiguous(), int(lmax), int(heads), C,
@@ -1455,9 +1523,6 @@ def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor]
 
 class _GraphSoftmax(torch.autograd.Function):
     @staticmethod
-    if (keys.is_cuda and keys.dim() == 1 and keys.dtype in (torch.int64, torch.int32)
-            and max(n_keys, keys.shape[0]) < 2 ** 31 - 8192):
-        return _group_keys(keys, n_keys)[1:3]
     def forward(ctx, s, plan: EdgePlan):
         a = launch_softmax_fwd(s, plan)
         ctx.save_for_backward(a)

@@ -1,0 +1,167 @@
+"""The gate, the energy readout, the edge-vector gradient and the key grouping kernels (GPU)."""
+
+import pytest
+import torch
+
+from tace_amd import model as pm
+from tace_amd import ops
+from tace_amd.so3 import Irrep, Irreps
+
+pytestmark = pytest.mark.gpu
+
+# a handful of roundings per output (exp to 1 ulp, products, sums of at most 7 terms)
+EPS = {torch.float32: 2e-6, torch.float64: 4e-15}
+
+
+def _rel(got, want):
+    return ((got.double() - want).abs().max() / want.abs().max().clamp_min(1e-300)).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("L,C,n,off", [(0, 64, 5, 0), (1, 5, 257, 0), (2, 128, 1, 0), (3, 128, 70, 0), (3, 33, 19, 0),
+                                       (3, 64, 31, 1), (2, 256, 0, 0)])
+def test_gate_matches_torch(cuda, dtype, L, C, n, off):
+    """Gate kernels against the same expressions in float64: channel counts
+    off the vector width, a misaligned input (off), no nodes."""
+    lout = pm.GMLayout(Irreps([(C, Irrep(l, (-1) ** l)) for l in range(L + 1)]))
+    lin = pm.GMLayout(Irreps([((L + 2) * C, Irrep(0, 1))] + [(C, Irrep(l, (-1) ** l)) for l in range(1, L + 1)]))
+    assert pm._GateFn.native(lin, lout, C)
+    g = torch.Generator().manual_seed(n + L)
+    x64 = 3 * torch.randn(n, lin.dim, generator=g, dtype=torch.float64)
+    go64 = torch.randn(n, lout.dim, generator=g, dtype=torch.float64)
+    buf = torch.empty(n * lin.dim + off, dtype=dtype, device=cuda)
+    x = buf[off:].view(n, lin.dim).copy_(x64).requires_grad_(True)
+    go = go64.to(dtype).to(cuda)
+    out = pm._GateFn.apply(x, lin, lout, C)
+    (gx,) = torch.autograd.grad(out, x, go)
+    assert out.shape == (n, lout.dim) and gx.shape == x.shape
+    if n == 0:
+        return
+    xr = x.detach().double().cpu().requires_grad_(True)
+    gate = torch.sigmoid(lin.block(xr, 0).view(n, -1)[:, :(L + 1) * C]) * pm.SIGMOID_CST
+    want = torch.cat([(s * gate[:, k * C:(k + 1) * C].unsqueeze(1)).reshape(-1)
+                      for k, s in enumerate(pm._gated_blocks(xr, lin, lout, C))]).view(n, -1)
+    (gw,) = torch.autograd.grad(want, xr, go.double().cpu())
+    assert _rel(out.detach().cpu(), want.detach()) < EPS[dtype]
+    assert _rel(gx.cpu(), gw) < EPS[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("C,S,sizes", [(64, 1, [1]), (128, 4, [1, 30, 1]), (200, 89, [5, 64, 65, 1, 0, 700]),
+                                       (512, 2, [3000]), (40, 70, [2, 2])])
+def test_energy_head_matches_torch(cuda, dtype, C, S, sizes):
+    """Readout, element tables and graph sums against float64: atoms alone
+    with and without edges, an empty graph, more species than lanes."""
+    g = torch.Generator().manual_seed(C)
+    n = sum(sizes)
+    mk = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64).to(dtype)
+    x, w1, w2, e0, sc, sh = mk(n, C), mk(C, 16) / C ** 0.5, mk(16), mk(S), mk(S), mk(S)
+    attrs = torch.nn.functional.one_hot(torch.randint(0, S, (n,), generator=g), S).to(dtype)
+    row_of = torch.randperm(n, generator=g)
+    batch = torch.repeat_interleave(torch.arange(len(sizes)), torch.tensor(sizes))
+    ptr = torch.tensor([0] + sizes).cumsum(0)
+    deg = torch.randint(0, 3, (n,), generator=g)
+    rowptr = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)]).to(torch.int32)
+    gE, gn = mk(len(sizes)), mk(n)
+    d = lambda t: t.to(cuda)
+    xg = d(x).requires_grad_(True)
+    E, en = ops.EnergyHead.apply(xg, d(row_of), d(w1), d(w2), d(attrs), d(e0), d(sc), d(sh), d(batch), d(ptr), d(rowptr))
+    got = torch.autograd.grad([E, en], xg, [d(gE), d(gn)], retain_graph=True)[0]
+    only_e = torch.autograd.grad(E, xg, d(gE), retain_graph=True)[0]
+    only_n = torch.autograd.grad(en, xg, d(gn))[0]
+    xr = x.double().requires_grad_(True)
+    e = torch.nn.functional.silu(xr[row_of] @ w1.double()) @ w2.double()
+    keep = 1.0 - ((ptr[1:] - ptr[:-1])[batch] == 1).double() * (deg == 0).double()
+    a = attrs.double()
+    en_w = a @ e0.double() + (e * (a @ sc.double()) + a @ sh.double()) * keep
+    E_w = torch.zeros(len(sizes), dtype=torch.float64).index_add(0, batch, en_w)
+    want = torch.autograd.grad([E_w, en_w], xr, [gE.double(), gn.double()], retain_graph=True)[0]
+    # sums of C products (and of the graph's nodes) in another order
+    tol = (C + n) ** 0.5 * EPS[dtype]
+    assert _rel(E.detach().cpu(), E_w.detach()) < tol and _rel(en.detach().cpu(), en_w.detach()) < tol
+    assert _rel(got.cpu(), want) < tol
+    assert _rel((only_e + only_n).cpu(), want) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("sorted_edges", [True, False])
+def test_edge_vector_gradient_with_lattices(cuda, dtype, sorted_edges):
+    """Position and lattice gradients of edge_vectors with ``ptr`` against
+    autograd: nodes without edges, with 1, 15, 16, 17 and 100, a graph
+    without edges."""
+    g = torch.Generator().manual_seed(1)
+    sizes = [7, 1, 130, 2]
+    n = sum(sizes)
+    ptr = torch.tensor([0] + sizes).cumsum(0)
+    batch = torch.repeat_interleave(torch.arange(4), torch.tensor(sizes))
+    src, dst = [], []
+    for i, k in enumerate([0, 1, 15, 16, 17, 100] + [0] * (n - 6)):
+        lo, hi = (0, 7) if i < 7 else (8, 138)
+        if i >= 8 and i < 138:
+            k = i % 20
+        src.append(torch.randint(lo, hi, (k,), generator=g))
+        dst.append(torch.full((k,), i))
+    ei = torch.stack([torch.cat(src), torch.cat(dst)])
+    if not sorted_edges:
+        ei = ei[:, torch.randperm(ei.shape[1], generator=g)]
+    E = ei.shape[1]
+    pos, lat = torch.randn(n, 3, generator=g, dtype=dtype), torch.randn(4, 3, 3, generator=g, dtype=dtype)
+    sh = torch.randint(-2, 3, (E, 3), generator=g).to(dtype)
+    go = torch.randn(E, 3, generator=g, dtype=dtype)
+    plan = ops.EdgePlan.from_edge_index(ei.to(cuda), n)
+    assert (plan.eid is None) == sorted_edges
+    p, l = pos.to(cuda).requires_grad_(True), lat.to(cuda).requires_grad_(True)
+    eg = batch[ei[0]].to(cuda)
+    v = ops.edge_vectors(p, l, sh.to(cuda), plan, ei[1].to(cuda), eg, ptr.to(cuda))
+    got = torch.autograd.grad(v, [p, l], go.to(cuda))
+    pr, lr = pos.double().requires_grad_(True), lat.double().requires_grad_(True)
+    w = pr[ei[1]] - pr[ei[0]] + torch.einsum("ei,eij->ej", sh.double(), lr[batch[ei[0]]])
+    want = torch.autograd.grad(w, [pr, lr], go.double())
+    for a, b in zip(got, want):
+        assert _rel(a.cpu(), b) < 20 * EPS[dtype]
+    with pytest.raises(ValueError, match="numbers of graphs"):
+        ops.edge_vectors(p, l, sh.to(cuda), plan, ei[1].to(cuda), eg, ptr[:3].to(cuda))
+
+
+@pytest.mark.parametrize("n,n_keys,skew", [(0, 3, 0), (1, 1, 0), (300, 7, 0), (8192, 4096, 0), (8193, 4096, 0),
+                                           (8192, 4097, 0), (30000, 50, 0), (30000, 9000, 1), (12345, 2, 0),
+                                           (50000, 5, 1), (8192, 10, 1)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_group_keys_equals_stable_sort(cuda, n, n_keys, skew, dtype):
+    """Both forms of the grouping (one workgroup, several launches), ranges
+    longer than the ranked ones, strided keys, keys read through positions."""
+    g = torch.Generator().manual_seed(n + n_keys)
+    keys = torch.randint(0, n_keys, (n,), generator=g)
+    if skew:   # most positions in one range
+        keys[torch.rand(n, generator=g) < 0.8] = n_keys // 2
+    wide = torch.stack([keys, torch.zeros_like(keys)], 1).to(dtype).to(cuda)
+    perm = torch.randperm(n, generator=g)
+    for k, through, ref in ((wide[:, 0], None, keys), (wide[:, 0].contiguous(), perm.to(torch.int32).to(cuda), keys[perm])):
+        flags = torch.empty(2, dtype=torch.int32, device=cuda)
+        k32, rp, order, _ = ops._group_keys(k, n_keys, through=through, flags=flags)
+        assert torch.equal(k32.cpu(), ref.to(torch.int32))
+        assert torch.equal(order.cpu().long(), torch.argsort(ref, stable=True))
+        assert torch.equal(rp.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64),
+                                                       torch.bincount(ref, minlength=n_keys).cumsum(0)]))
+        assert flags.tolist() == [0, int(bool((ref[1:] < ref[:-1]).any()))]
+
+
+@pytest.mark.parametrize("n", [50, 20000])
+def test_edge_plan_refuses_nodes_out_of_range(cuda, n):
+    """Negative and too large ids in either row are refused (the kernels skip
+    them; nothing is indexed with them); int32 and column-major edge lists are
+    taken."""
+    g = torch.Generator().manual_seed(n)
+    ei = torch.randint(0, 40, (2, n), generator=g)
+    for row, bad in ((0, -1), (0, 40), (1, -3), (1, 2 ** 40)):
+        e = ei.clone()
+        e[row, n // 2] = bad
+        with pytest.raises(ValueError, match="outside"):
+            ops.EdgePlan.from_edge_index(e.to(cuda), 40)
+    want = ops.EdgePlan.from_edge_index(ei, 40)   # the torch form, on the CPU
+    for e in (ei.to(cuda), ei.to(torch.int32).to(cuda), ei.t().contiguous().to(cuda).t()):
+        plan = ops.EdgePlan.from_edge_index(e, 40)
+        for a, b in ((plan.rowptr, want.rowptr), (plan.src, want.src), (plan.eid, want.eid)):
+            assert torch.equal(a.cpu(), b)
+        for a, b in zip(plan.sender_csr(), want.sender_csr()):
+            assert torch.equal(a.cpu(), b)
