@@ -593,6 +593,23 @@ int tace_so2_gemm_bf16_kt(const uint16_t* a, int64_t lda, const uint16_t* b_frag
 int tace_edge_pairs(const int32_t* rowptr, const int32_t* eid, const int32_t* src, const int32_t* shifts,
                     int64_t n_nodes, int64_t n_edges, int32_t* work, int32_t* w_rows, int32_t* row_edges,
                     int32_t* row_partner, void* stream);
+/* y [m, n] = x [m, k] @ B (+ bias [n]) in float32 on the bf16 MFMA (three
+ * terms per operand, six products): the fragment-order tile kernel of
+ * tace_seg_linear_presplit_frag without tables.  w_frag: B [k, n] in the
+ * three-term fragment order (tace_layout_operands kind 1 or
+ * tace_bf16x3_split_blocks layout 1), 16-byte aligned; x and y row-major. */
+int tace_gemm_bx3(const float* x, const uint16_t* w_frag, const float* bias, float* y, int64_t m, int32_t n, int32_t k,
+                  void* stream);
+/* Several GEMM operands B [k, n] laid out from float32 weights in one launch.
+ * table: 20 x int64 per operand on the device: kind (0 bf16 in MFMA fragment
+ * order, 1024 ceil(k/32) ceil(n/16) bytes; 1 its three terms, three times
+ * that; 2 float32 row-major), k, n, byte offset in out (a multiple of 16),
+ * number of segments (1..4), axis (0: segments stacked along n, 1: along k),
+ * trans (B[kk][c] = W[c][kk], else W[kk][c]), row stride of every W, then per
+ * segment the device address of W, its length along the axis and its scale as
+ * a double's bits.  Values are scaled in float32, then rounded or split. */
+int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, void* stream);
+
 /* Positions 0 .. n-1 grouped by key (torch.argsort(stable=True) of the
  * receivers, and bincount + cumsum): key i is keys[(through ? through[i] : i)
  * * stride], of key_bytes 4 or 8.  keys32 [n]: the keys (-1 outside [0,

@@ -527,16 +527,21 @@ struct FtLoad {   // the contribution and step whose operands load next
   bool xvec;
 };
 
+struct FtDense {   // the sizes of a launch without tables: one [m, k] x [k, n] product
+  int64_t m;
+  int n, k;
+};
+
 __device__ __forceinline__ void ft_open(FtLoad& L, const float* __restrict__ x, const unsigned short* __restrict__ wfrag,
-                                        const int64_t* __restrict__ contribs, int c) {
+                                        const int64_t* __restrict__ contribs, int c, const FtDense& dense) {
   const int64_t* cd = contribs + 4 * (int64_t)c;
   L.c = c;
   L.s = 0;
-  L.xa = x + cd[0];
-  L.k = (int)cd[1];
+  L.xa = contribs ? x + cd[0] : x;
+  L.k = contribs ? (int)cd[1] : dense.k;
   L.nks = (L.k + 31) >> 5;
   L.send = L.nks;
-  L.wf = wfrag + cd[2];
+  L.wf = contribs ? wfrag + cd[2] : wfrag;
   L.xvec = ((((uintptr_t)L.xa) & 15) == 0) && ((L.k & 3) == 0);
 }
 
@@ -585,7 +590,7 @@ template <bool VEC, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_seg_linear_bx3f(
     const float* __restrict__ x, float* y, const float* addend, const unsigned short* __restrict__ wfrag,
     const float* __restrict__ bias, const int64_t* __restrict__ tiles, const int64_t* __restrict__ contribs,
-    float alpha, int n_tiles, int per, int splits, float* __restrict__ partials) {
+    float alpha, int n_tiles, int per, int splits, float* __restrict__ partials, FtDense dense) {
   constexpr int WM = 4, PL = 64 * SB_STR;   // 16-row blocks, plane size (bf16)
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3 * PL];
   // work item wi: split sp of a tile, half of its rows.  The two halves run
@@ -602,13 +607,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const int vi = SPLIT ? tile * splits + sp : tile;
   if (SPLIT ? sp >= splits : tile >= n_tiles) return;
   const int64_t* td = tiles + 8 * (int64_t)tile;
-  const int r0 = 64 * half, rows = min((int)td[1] - r0, 64);
+  const int r0 = 64 * half;
+  int rows, n, c0, cb = 0, ce = 1;
+  int64_t out_base, bias_off = -1;
+  if (tiles) {
+    rows = min((int)td[1] - r0, 64);
+    n = (int)td[2];
+    c0 = (int)td[3];
+    out_base = td[0] + (int64_t)r0 * n;
+    if constexpr (!SPLIT) bias_off = td[4];
+    cb = (int)td[5];
+    ce = (int)td[6];
+  } else {
+    // one [m, k] x [k, n] product: the column tiles of a row tile in turn
+    const int ct = (dense.n + 127) >> 7, rt = tile / ct;
+    rows = (int)min(dense.m - 128 * (int64_t)rt - r0, (int64_t)64);
+    n = dense.n;
+    c0 = 128 * (tile - rt * ct);
+    out_base = (128 * (int64_t)rt + r0) * n;
+    if (bias) bias_off = 0;
+    x += 128 * (int64_t)rt * dense.k;
+  }
   if (rows <= 0) return;   // the tile ends in the first half, or a padding entry of the table
-  const int n = (int)td[2], c0 = (int)td[3];
-  const int64_t out_base = td[0] + (int64_t)r0 * n;
-  const int64_t bias_off = SPLIT ? -1 : td[4];
-  const int cb = (int)td[5];
-  int ce = (int)td[6];
   if constexpr (SPLIT) ce = min(ce, cb + 1);   // k_seg_split_sum writes NaN for a tile with more
   const int t = (int)threadIdx.x, lane = t & 63, wv = t >> 6;
   const int wc = wv * 32;   // this wavefront's 32 columns (all 64 rows)
@@ -638,7 +658,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   int c = cb;
   FtLoad L;
   while (c < ce) {
-    ft_open(L, x, wfrag, contribs, c);
+    ft_open(L, x, wfrag, contribs, c, dense);
     if constexpr (SPLIT) {
       L.s = (int)((int64_t)sp * L.nks / splits);
       L.send = (int)((int64_t)(sp + 1) * L.nks / splits);
@@ -665,7 +685,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
       }
       for (int cc = C.c + 1; cc < ce; ++cc) {
         FtLoad D;
-        ft_open(D, x, wfrag, contribs, cc);
+        ft_open(D, x, wfrag, contribs, cc, dense);
         if (D.send > 0) {
           C = D;
           return;
@@ -1121,7 +1141,81 @@ __global__ __launch_bounds__(256) void k_split_blocks(const float* __restrict__ 
   }
 }
 
+// Several GEMM operands laid out in one launch, each from up to four scaled
+// weight matrices stacked along its columns or its rows.  An operand is 20 x
+// int64: kind (0 bf16 in MFMA fragment order, 1 three bf16 terms in fragment
+// order, 2 float32 row-major [k, n]), k, n, byte offset in out (16-byte
+// aligned), segments, axis (0: stacked along n, 1: along k), trans (B[kk][c] =
+// W[c][kk], else W[kk][c]), row stride of every W, then per segment its
+// address, its length along the axis and its scale (a double's bits).  A
+// thread makes the eight values of one lane's fragment (or one float), so its
+// stores are 16 bytes; blockIdx.y picks the operand.
+struct OpDesc {
+  int64_t d[20];
+
+  __device__ __forceinline__ float at(int kk, int c) const {
+    int a = d[5] == 0 ? c : kk, first = 0;   // the index in its segment
+    const float* W = (const float*)d[8];
+    float sc = (float)__longlong_as_double(d[10]);
+#pragma unroll
+    for (int s = 1; s < 4; ++s) {
+      first += (int)d[6 + 3 * s];   // the lengths of the segments before s
+      if (s < (int)d[4] && (d[5] == 0 ? c : kk) >= first) {
+        a = (d[5] == 0 ? c : kk) - first;
+        W = (const float*)d[8 + 3 * s];
+        sc = (float)__longlong_as_double(d[10 + 3 * s]);
+      }
+    }
+    if (d[5] == 0) c = a;
+    else kk = a;
+    // trans: W's rows are B's columns
+    return bx3_scale2(bx3_f2{W[d[6] ? (int64_t)c * d[7] + kk : (int64_t)kk * d[7] + c], 0.f}, sc).x;
+  }
+};
+
+__global__ __launch_bounds__(256) void k_layout_operands(const int64_t* __restrict__ table,
+                                                         unsigned char* __restrict__ out) {
+  OpDesc o;   // uniform: in scalar registers
+#pragma unroll
+  for (int i = 0; i < 20; ++i) o.d[i] = table[20 * (int64_t)blockIdx.y + i];
+  const int kind = (int)o.d[0], k = (int)o.d[1], n = (int)o.d[2];
+  unsigned char* dst = out + o.d[3];
+  if (kind == 2) {
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < (int64_t)k * n; e += (int64_t)gridDim.x * 256)
+      ((float*)dst)[e] = o.at((int)(e / n), (int)(e % n));
+    return;
+  }
+  const int nks = (k + 31) >> 5, nb = (n + 15) >> 4;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < (int64_t)nks * nb * 64; e += (int64_t)gridDim.x * 256) {
+    const int lane = (int)(e & 63);
+    const int64_t run = e >> 6;   // column block x k step
+    const int s = (int)(run % nks), cb = (int)(run / nks);
+    const int c = 16 * cb + (lane & 15), k0 = 32 * s + 8 * (lane >> 4);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = c < n && k0 + j < k ? o.at(k0 + j, c) : 0.f;
+    bx3_bf8 h[3];
+    bx3_split8(v, h);
+    if (kind == 0) {
+      *(bx3_bf8*)(dst + 1024 * run + 16 * lane) = h[0];
+    } else {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *(bx3_bf8*)(dst + 1024 * (3 * run + p) + 16 * lane) = h[p];
+    }
+  }
+}
+
 }  // namespace
+
+extern "C" int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, void* stream) {
+  if (n_operands < 0 || n_operands > 65535) return tace_fail_msg("tace_layout_operands: 0..65535 operands");
+  if (n_operands == 0) return 0;
+  if (!table || !out || (((uintptr_t)out) & 15) != 0)
+    return tace_fail_msg("tace_layout_operands: null or misaligned pointer");
+  hipLaunchKernelGGL(k_layout_operands, dim3(64, (unsigned)n_operands), dim3(256), 0, (hipStream_t)stream, table,
+                     (unsigned char*)out);
+  return tace_check_launch("tace_layout_operands");
+}
 
 extern "C" int tace_bf16x3_split_blocks(const float* w, const int64_t* blocks, const double* scales,
                                         int64_t n_blocks, uint16_t* planes, int64_t plane_stride, void* stream) {
@@ -1164,11 +1258,11 @@ extern "C" int tace_seg_linear_presplit_frag(const float* x, float* y, const flo
   if (aligned && (((uintptr_t)x) & 15) == 0)
     hipLaunchKernelGGL((k_seg_linear_bx3f<true, false>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag,
-                       bias, tiles, contribs, (float)alpha, (int)n_tiles, per, 1, nullptr);
+                       bias, tiles, contribs, (float)alpha, (int)n_tiles, per, 1, nullptr, FtDense{0, 0, 0});
   else
     hipLaunchKernelGGL((k_seg_linear_bx3f<false, false>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag,
-                       bias, tiles, contribs, (float)alpha, (int)n_tiles, per, 1, nullptr);
+                       bias, tiles, contribs, (float)alpha, (int)n_tiles, per, 1, nullptr, FtDense{0, 0, 0});
   return tace_check_launch("tace_seg_linear_presplit_frag");
 }
 
@@ -1195,15 +1289,36 @@ extern "C" int tace_seg_linear_presplit_frag_split(const float* x, float* y, con
   if (aligned && (((uintptr_t)x) & 15) == 0)
     hipLaunchKernelGGL((k_seg_linear_bx3f<true, true>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag, bias, tiles, contribs, (float)alpha, (int)n_tiles, per,
-                       (int)splits, partials);
+                       (int)splits, partials, FtDense{0, 0, 0});
   else
     hipLaunchKernelGGL((k_seg_linear_bx3f<false, true>), g, b, 0, (hipStream_t)stream, x, y, addend,
                        (const unsigned short*)w_frag, bias, tiles, contribs, (float)alpha, (int)n_tiles, per,
-                       (int)splits, partials);
+                       (int)splits, partials, FtDense{0, 0, 0});
   if (int rc = tace_check_launch("tace_seg_linear_presplit_frag_split")) return rc;
   hipLaunchKernelGGL(k_seg_split_sum, dim3((unsigned)(16 * n_tiles)), dim3(256), 0, (hipStream_t)stream, y, addend, bias,
                      tiles, (const float*)partials, (int)splits, (float)alpha);
   return tace_check_launch("tace_seg_linear_presplit_frag_split");
+}
+
+extern "C" int tace_gemm_bx3(const float* x, const uint16_t* w_frag, const float* bias, float* y, int64_t m, int32_t n,
+                             int32_t k, void* stream) {
+  if (m < 0 || n <= 0 || k <= 0) return tace_fail_msg("tace_gemm_bx3: bad sizes");
+  const int64_t items = ((m + 127) / 128) * ((n + 127) / 128);
+  if (items > 0x7ffffff) return tace_fail_msg("tace_gemm_bx3: too many tiles");
+  if (m == 0) return 0;
+  if (!x || !w_frag || !y) return tace_fail_msg("tace_gemm_bx3: null pointer");
+  if ((((uintptr_t)w_frag) & 15) != 0) return tace_fail_msg("tace_gemm_bx3: the weights must be 16-byte aligned");
+  const int per = (int)((items + 7) / 8);
+  const dim3 g((unsigned)(16 * per)), b(256);   // two 64-row halves per tile
+  const unsigned short* wf = (const unsigned short*)w_frag;
+  const FtDense d{m, n, k};
+  if ((k & 3) == 0 && (((uintptr_t)x) & 15) == 0)
+    hipLaunchKernelGGL((k_seg_linear_bx3f<true, false>), g, b, 0, (hipStream_t)stream, x, y, nullptr, wf, bias, nullptr,
+                       nullptr, 1.f, (int)items, per, 1, nullptr, d);
+  else
+    hipLaunchKernelGGL((k_seg_linear_bx3f<false, false>), g, b, 0, (hipStream_t)stream, x, y, nullptr, wf, bias, nullptr,
+                       nullptr, 1.f, (int)items, per, 1, nullptr, d);
+  return tace_check_launch("tace_gemm_bx3");
 }
 
 extern "C" int32_t tace_seg_linear_ks_rows(int32_t k) { return k < 0 ? 0 : k <= 128 ? 128 : k <= 256 ? 64 : 0; }

@@ -1274,6 +1274,34 @@ def so2_gemm_bf16(a: torch.Tensor, b_frag: torch.Tensor, n: int, k: int,
     return out
 
 
+def layout_operands(table: torch.Tensor, nbytes: int) -> torch.Tensor:
+    """The operands of ``tace_layout_operands``' table [n, 20] (int64, on the
+    GPU, whose addresses the caller keeps alive) in one new buffer of bytes."""
+    _req(table, "table", torch.int64, (table.shape[0], 20))
+    out = torch.empty(nbytes, dtype=torch.uint8, device=table.device)
+    N.check(N.lib().tace_layout_operands(table.data_ptr(), table.shape[0], out.data_ptr(), N.stream_ptr(table.device)),
+            "tace_layout_operands")
+    return out
+
+
+def gemm_bx3(x: torch.Tensor, frag: torch.Tensor, n: int, k: int, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [m, k] @ B [k, n] (+ bias [n]) in float32 on ``tace_gemm_bx3``; frag:
+    B's three bf16 terms in fragment order (int16)."""
+    m = x.shape[0]
+    _req(x, "x", torch.float32, (m, k))
+    if frag.dtype != torch.int16 or not frag.is_contiguous() or not frag.is_cuda \
+            or frag.numel() < 1536 * ((k + 31) // 32) * ((n + 15) // 16):
+        raise ValueError("gemm_bx3: the weights are not the three-term fragment order of a [k, n] matrix")
+    if bias is not None:
+        _req(bias, "bias", torch.float32, (n,))
+    out = torch.empty(m, n, dtype=torch.float32, device=x.device)
+    tok = _t0("gemm_bx3")
+    N.check(N.lib().tace_gemm_bx3(x.data_ptr(), frag.data_ptr(), N.ptr(bias), out.data_ptr(), m, n, k,
+                                  N.stream_ptr(x.device)), "tace_gemm_bx3")
+    _t1(tok, (m, n, k))
+    return out
+
+
 def rows_accumulate(out: torch.Tensor, rows: torch.Tensor, rowptr: torch.Tensor, slot: Optional[torch.Tensor] = None,
                     target: Optional[torch.Tensor] = None, run: int = 1) -> torch.Tensor:
     """out[target[s]] += sum of rows[slot[k]], k in [rowptr[s], rowptr[s+1])

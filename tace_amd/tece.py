@@ -18,6 +18,7 @@ features come and go in the model's group-major, species-sorted layout.
 from __future__ import annotations
 
 import math
+import struct
 from typing import List, Optional
 
 import torch
@@ -439,11 +440,40 @@ def _so2_route(k: int, n: int, bias: bool):
     return "kt" if k % 64 == 0 else "lds"
 
 
+# float32 SO(2) GEMMs on tace_gemm_bx3 (three bf16 terms per operand, float32
+# accuracy); False: the library.  The 24 products of a 39k-edge layer (k, n =
+# 96-1152, forward and backward): 2.87 ms on the library, 1.92 ms here, with
+# the layer's error against float64 as it was (8.7e-7, 8.2e-7)
+F32_GEMM = True
+
+
+class _Operand:
+    """One right GEMM operand [k, n] of the fused operator: ``frag``, its copy
+    in MFMA fragment order (bf16 or three bf16 terms, None in float64), and
+    ``plain()``, the matrix itself for the library."""
+
+    def __init__(self, k: int, n: int, plain):
+        self.k, self.n, self.frag = k, n, None
+        self._plain, self._made = plain, None
+
+    def plain(self) -> torch.Tensor:
+        if self._made is None:
+            self._made = self._plain()
+        return self._made
+
+
 class _FusedParams:
-    """Everything the fused TECE operator needs from the frozen modules,
-    prepared once per forward: the SO(2) linears as W^T (forward GEMM
-    operand) and W (input-gradient operand) in the mixing precision, the
-    biases, the radial projection, the attention scale and the radial MLP."""
+    """Everything the fused TECE operator needs from the frozen modules, laid
+    out once per forward: the SO(2) linears as W^T (forward GEMM operand) and
+    W (input-gradient operand), the biases, the radial projection, the
+    attention scale and the radial MLP.
+
+    In float32 one launch (``tace_layout_operands``) reads every weight and
+    writes all operands, in the fragment order of the mixing precision's GEMM
+    kernel; made by torch operations they took about 130 launches a forward.
+    Only the table of addresses and sizes is kept between calls (on the
+    convolution, for the addresses it was made from); the weights are read
+    every time."""
 
     def __init__(self, conv: "TeceConvolution", mlp, dtype):
         self.lmax, self.H, self.A, self.C = conv.lmax, conv.H, conv.A, conv.C
@@ -451,71 +481,104 @@ class _FusedParams:
         self.bf16 = self.mixing is not None
         op = self.mixing or dtype
         L = self.lmax
+        gemms, floats = [], []   # (operand, segments, stacked along k); (name, shape, segments, trans, row stride)
 
-        def pair(W):
-            W = W.detach().to(dtype)
-            return W.t().to(op).contiguous(), W.to(op).contiguous()
+        def pair(*fcs):
+            """(W^T, W) operands of linears sharing an input, stacked along their outputs."""
+            out, cin = sum(f.weight.shape[0] for f in fcs), fcs[0].weight.shape[1]
 
-        def so2(lin):
-            f0 = lin.m0_rlinear
-            mats = [pair(f0.weight * f0.alpha)] + [pair(lin.ms_clinear[m - 1].fc.weight * lin.ms_clinear[m - 1].fc.alpha)
-                                                   for m in range(1, L + 1)]
-            return [a for a, _ in mats], [b for _, b in mats], f0.bias.detach().to(dtype).contiguous()
+            def stacked():
+                return torch.cat([f.weight.detach() * f.alpha for f in fcs]).to(dtype)
+            T = _Operand(cin, out, lambda: stacked().t().to(op).contiguous())
+            N = _Operand(out, cin, lambda: stacked().to(op).contiguous())
+            segs = [(f.weight, f.weight.shape[0], f.alpha) for f in fcs]
+            gemms.extend([(T, segs, False), (N, segs, True)])
+            return T, N
 
-        self.k_T, self.k_N, self.k_b = so2(conv.key_proj)
-        self.q_T, self.q_N, self.q_b = so2(conv.query_proj)
-        self.d_T, self.d_N, self.d_b = so2(conv.linear_down)
-        lc, lg, lu = conv.linear_coefs, conv.linear_glu, conv.linear_up
-        f0 = [lc.m0_rlinear, lg.m0_rlinear, lu.m0_rlinear]
-        sh = [pair(torch.cat([f.weight * f.alpha for f in f0]))]
-        for m in range(1, L + 1):
-            fg, fu = lg.ms_clinear[m - 1].fc, lu.ms_clinear[m - 1].fc
-            sh.append(pair(torch.cat([fg.weight * fg.alpha, fu.weight * fu.alpha])))
-        self.s_T, self.s_N = [a for a, _ in sh], [b for _, b in sh]
-        self.s_b = torch.cat([f.bias for f in f0]).detach().to(dtype).contiguous()
+        def so2(*lins):
+            mats = [pair(*[lin.m0_rlinear for lin in lins])]
+            mats += [pair(*[lin.ms_clinear[m - 1].fc for lin in lins if lin.mmax >= m]) for m in range(1, L + 1)]
+            return [a for a, _ in mats], [b for _, b in mats]
+
+        self.k_T, self.k_N = so2(conv.key_proj)
+        self.q_T, self.q_N = so2(conv.query_proj)
+        self.d_T, self.d_N = so2(conv.linear_down)
+        shared = (conv.linear_coefs, conv.linear_glu, conv.linear_up)
+        self.s_T, self.s_N = so2(*shared)
+        self.k_b, self.q_b, self.d_b = (lin.m0_rlinear.bias.detach().to(dtype).contiguous()
+                                        for lin in (conv.key_proj, conv.query_proj, conv.linear_down))
         rp = conv.radial_proj
-        Wrp = (rp.weight * rp.alpha).detach().to(dtype)
-        self.rp_T, self.rp_N, self.rp_b = Wrp.t().contiguous(), Wrp.contiguous(), rp.bias.detach().to(dtype)
+        self.rp_b = rp.bias.detach().to(dtype)
         T = conv.tmin + (conv.tmax - conv.tmin) * torch.sigmoid(conv.temperature_logit.detach())
         self.tscale = (T * conv.attention_scale).to(dtype).contiguous()
         lins = [m for m in mlp.mlp if hasattr(m, "alpha")]
-        self.mlp_flat = torch.cat([(m.weight * m.alpha).detach().reshape(-1) for m in lins[:-1]]).to(dtype).contiguous()
         self.mlp_layers = len(lins) - 1
         self.mlp_W = lins[-1].weight.detach().to(dtype).contiguous()
         self.mlp_alpha = float(lins[-1].alpha)
-        self.mlp_WT_scaled = (lins[-1].weight * lins[-1].alpha).detach().to(dtype).t().contiguous()
-        # fragment-order copies of the bf16 GEMM operands (by id of the operand;
-        # each entry keeps its operand alive)
-        self._frag = {}
+        biases = [lin.m0_rlinear.bias for lin in shared]
+        nr, no = rp.weight.shape[1], rp.weight.shape[0]
+        floats = [("s_b", [(v, v.numel(), 1.0) for v in biases], 1, sum(v.numel() for v in biases), False, 1, 1),
+                  ("mlp_flat", [(m.weight, m.weight.numel(), m.alpha) for m in lins[:-1]], 1,
+                   sum(m.weight.numel() for m in lins[:-1]), False, 1, 1),
+                  ("rp_T", [(rp.weight, no, rp.alpha)], nr, no, False, 1, nr),
+                  ("rp_N", [(rp.weight, no, rp.alpha)], no, nr, True, 0, nr)]
+        params = [w for _, segs, _ in gemms[::2] for w, _, _ in segs] + [w for f in floats for w, _, _ in f[1]]
+        if dtype == torch.float32 and all(p.is_cuda and p.dtype == dtype and p.is_contiguous() for p in params):
+            self._layout(conv, gemms, floats, params)
+            return
+        self.s_b = torch.cat([v.detach() for v in biases]).to(dtype).contiguous()
+        Wrp = (rp.weight * rp.alpha).detach().to(dtype)
+        self.rp_T, self.rp_N = Wrp.t().contiguous(), Wrp.contiguous()
+        self.mlp_flat = torch.cat([(m.weight * m.alpha).detach().reshape(-1) for m in lins[:-1]]).to(dtype).contiguous()
 
-    def _so2(self, x, B, b=None, kernel="lds"):
-        """x @ B (+ b) on ``tace_so2_gemm_bf16`` or, kernel "kt", its k-tiled
-        variant (bf16 operands, float32 sums, bias in the epilogue); B's
-        fragment-order copy is made on first use."""
-        f = self._frag.get(id(B))
-        if f is None:
-            f = self._frag[id(B)] = (ops.bf16_fragment_order(B), B)
-        return ops.so2_gemm_bf16(x, f[0], B.shape[1], B.shape[0], b, ktiled=kernel == "kt")
+    def _layout(self, conv, gemms, floats, params):
+        """All operands in one launch; see the class."""
+        dev = params[0].device
+        key = (self.bf16, str(dev)) + tuple(p.data_ptr() for p in params)
+        kept = conv.__dict__.get("_operand_table")
+        if kept is None or kept[0] != key:
+            rows, places, at = [], [], 0
 
-    def mm(self, x, WT, b=None):
-        """x @ WT (+ b): bf16 operands with float32 accumulation and output
+            def add(kind, k, n, segs, along_k, trans, ld, nbytes):
+                nonlocal at
+                row = [kind, k, n, at, len(segs), int(along_k), trans, ld]
+                for w, length, alpha in segs:
+                    row += [w.data_ptr(), length, struct.unpack("q", struct.pack("d", alpha))[0]]
+                rows.append(row + [0] * (20 - len(row)))
+                places.append((at, nbytes))
+                at += (nbytes + 15) // 16 * 16
+            for o, segs, along_k in gemms:
+                size = 1024 * ((o.k + 31) // 32) * ((o.n + 15) // 16)
+                cin = o.n if along_k else o.k
+                add(0 if self.bf16 else 1, o.k, o.n, segs, along_k, int(not along_k), cin, size * (1 if self.bf16 else 3))
+            for _nm, segs, k, n, along_k, trans, ld in floats:
+                add(2, k, n, segs, along_k, trans, ld, 4 * k * n)
+            kept = (key, torch.tensor(rows, dtype=torch.int64, device=dev), places, at)
+            conv.__dict__["_operand_table"] = kept
+        _, table, places, nbytes = kept
+        buf = ops.layout_operands(table, nbytes)
+        for (o, _, _), (at, size) in zip(gemms, places):
+            o.frag = buf[at:at + size].view(torch.bfloat16 if self.bf16 else torch.int16)
+        for (nm, _, k, n, *_), (at, size) in zip(floats, places[len(gemms):]):
+            v = buf[at:at + size].view(torch.float32)
+            setattr(self, nm, v.view(k, n) if k > 1 else v)
+
+    def mm(self, x, B: _Operand, b=None):
+        """x @ B (+ b): bf16 operands with float32 accumulation and output
         under bf16 mixing, else in the features' precision."""
         if self.bf16:
-            r = _so2_route(WT.shape[0], WT.shape[1], b is not None) if SO2_GEMM else None
+            r = _so2_route(B.k, B.n, b is not None) if SO2_GEMM else None
             if r is not None and x.dtype == torch.bfloat16:
-                return self._so2(x, WT, b, r)
+                frag = B.frag if B.frag is not None else ops.bf16_fragment_order(B.plain())
+                return ops.so2_gemm_bf16(x, frag, B.n, B.k, b, ktiled=r == "kt")
             if b is None:
-                return torch.mm(x, WT, out_dtype=torch.float32)
-            return torch.addmm(b, x, WT, out_dtype=torch.float32)
-        return torch.mm(x, WT) if b is None else torch.addmm(b, x, WT)
+                return torch.mm(x, B.plain(), out_dtype=torch.float32)
+            return torch.addmm(b, x, B.plain(), out_dtype=torch.float32)
+        if F32_GEMM and B.frag is not None:
+            return ops.gemm_bx3(x, B.frag, B.n, B.k, b)
+        return torch.mm(x, B.plain()) if b is None else torch.addmm(b, x, B.plain())
 
-    def mm_grad(self, g, WN):
-        if self.bf16:
-            r = _so2_route(WN.shape[0], WN.shape[1], False) if SO2_GEMM else None
-            if r is not None and g.dtype == torch.bfloat16:
-                return self._so2(g, WN, None, r)
-            return torch.mm(g, WN, out_dtype=torch.float32)
-        return torch.mm(g, WN)
+    mm_grad = mm
 
 
 def _fused_chunk_fwd(P: _FusedParams, x_lc, R, W, rs, rd, plan: ops.EdgePlan, out_map, save: bool,
@@ -587,7 +650,7 @@ def _fused_chunk_bwd(P: _FusedParams, x_lc, R, W, rs, rd, plan: ops.EdgePlan, ou
     if gw.dtype == torch.float32 and gw.shape[1] % 4 == 0:
         gh = ops.launch_mlp_out_bwd_f32(gw, P.mlp_W, P.mlp_alpha)
     else:
-        gh = torch.mm(gw, P.mlp_WT_scaled)
+        gh = torch.mm(gw, P.mlp_W.t()).mul_(P.mlp_alpha)
     gR = torch.add(gR, ops.launch_mlp_hidden_bwd(R, gh, P.mlp_flat, P.mlp_layers), out=gR_out)
     return gR, gW
 

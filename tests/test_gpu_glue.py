@@ -165,3 +165,42 @@ def test_edge_plan_refuses_nodes_out_of_range(cuda, n):
             assert torch.equal(a.cpu(), b)
         for a, b in zip(plan.sender_csr(), want.sender_csr()):
             assert torch.equal(a.cpu(), b)
+
+
+@pytest.mark.parametrize("m,k,n,bias", [(1, 32, 16, True), (63, 96, 384, True), (64, 33, 70, False), (129, 384, 96, True),
+                                        (300, 768, 1152, True), (5001, 250, 129, False), (0, 64, 64, False)])
+def test_gemm_bx3_and_layout_match_float64(cuda, m, k, n, bias):
+    """Operands laid out from stacked, scaled weights (W^T and W, float32 and
+    bf16, row-major floats) and the float32 product against float64: edges of
+    the 64-row halves, the 128-column tiles, 32-k steps and 16-byte rows."""
+    g = torch.Generator().manual_seed(m + k)
+    cut = [n // 3, n - n // 3]
+    W = [torch.randn(c, k, generator=g).to(cuda) for c in cut]
+    alpha = [0.3, 1.7]
+    seg = [v for w, c, a in zip(W, cut, alpha) for v in (w.data_ptr(), c, torch.tensor([a]).double().view(torch.int64).item())]
+    pad = lambda r: r + [0] * (20 - len(r))
+    nb = lambda a, b: 1024 * ((a + 31) // 32) * ((b + 15) // 16)
+    sizes = [3 * nb(k, n), 3 * nb(n, k), nb(k, n), nb(n, k), 4 * n * k]
+    offs = [sum((s + 15) // 16 * 16 for s in sizes[:i]) for i in range(6)]
+    rows = [pad([1, k, n, offs[0], 2, 0, 1, k] + seg), pad([1, n, k, offs[1], 2, 1, 0, k] + seg),
+            pad([0, k, n, offs[2], 2, 0, 1, k] + seg), pad([0, n, k, offs[3], 2, 1, 0, k] + seg),
+            pad([2, n, k, offs[4], 2, 1, 0, k] + seg)]
+    buf = ops.layout_operands(torch.tensor(rows, dtype=torch.int64, device=cuda), offs[5])
+    full = torch.cat([w * torch.tensor(a, dtype=torch.float32) for w, a in zip(W, alpha)])   # [n, k]
+    view = lambda i, dt: buf[offs[i]:offs[i] + sizes[i]].view(dt)
+    assert torch.equal(view(4, torch.float32).view(n, k), full)
+    assert torch.equal(view(2, torch.bfloat16), ops.bf16_fragment_order(full.t().to(torch.bfloat16)))
+    assert torch.equal(view(3, torch.bfloat16), ops.bf16_fragment_order(full.to(torch.bfloat16)))
+    x, go = torch.randn(m, k, generator=g).to(cuda), torch.randn(m, n, generator=g).to(cuda)
+    b = torch.randn(n, generator=g).to(cuda) if bias else None
+    y = ops.gemm_bx3(x, view(0, torch.int16), n, k, b)
+    gx = ops.gemm_bx3(go, view(1, torch.int16), k, n)
+    assert y.shape == (m, n) and gx.shape == (m, k)
+    if m == 0:
+        return
+    want = x.double() @ full.double().t() + (b.double() if bias else 0.0)
+    # 2^-24 of the running sum at each of its 6 k / 32 accumulations, and 2^-23 of each product left out
+    tol = lambda kk: 2.0 ** -24 * (6 * kk / 32) ** 0.5 + 2.0 ** -23
+    assert ((y.double() - want).norm() / want.norm()).item() < tol(k)
+    want = go.double() @ full.double()
+    assert ((gx.double() - want).norm() / want.norm()).item() < tol(n)
