@@ -15,6 +15,7 @@
 #include <stdint.h>
 
 #include "../../include/tace_hip.h"
+#include "scan.h"
 
 int tace_fail_msg(const char* msg);   // tace_hip.hip
 int tace_check_launch(const char* what);
@@ -65,44 +66,8 @@ __global__ __launch_bounds__(256) void k_group_count(Keys<K> in, int n, int n_ke
   if (key >= 0) place[i] = atomicAdd(cnt + key, 1);
 }
 
-// exclusive scan of cnt[0..m) into out[0..m], one workgroup, 4096 counts at a time
 __global__ __launch_bounds__(1024) void k_group_scan(const int* __restrict__ cnt, int m, int* __restrict__ out) {
-  __shared__ int wsum[16];
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
-  int base = 0;
-  for (int b = 0; b < m; b += 4096) {
-    int v[4], s = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = b + 4 * t + q;
-      v[q] = i < m ? cnt[i] : 0;
-      s += v[q];
-    }
-    int inc = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int u = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += u;
-    }
-    if (lane == 63) wsum[w] = inc;
-    __syncthreads();
-    int before = 0, total = 0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      if (k < w) before += wsum[k];
-      total += wsum[k];
-    }
-    int run = base + before + inc - s;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = b + 4 * t + q;
-      if (i < m) out[i] = run;
-      run += v[q];
-    }
-    base += total;
-    __syncthreads();
-  }
-  if (t == 0) out[m] = base;
+  scan_1024(cnt, m, out);
 }
 
 __global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ k32, const int* __restrict__ place,

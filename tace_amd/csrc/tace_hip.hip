@@ -54,6 +54,7 @@ int tace_fail_msg(const char* msg) { return fail(msg); }
 int tace_check_launch(const char* what) { return check_launch(what); }
 
 #include "common.h"
+#include "scan.h"
 #include "gen/registry.inc"
 #include "gen/sh.inc"
 
@@ -592,28 +593,9 @@ __global__ void k_edge_rows(const int* __restrict__ partner, const int* __restri
   }
 }
 
-// exclusive scan of cnt[0..m) into out[0..m]; single block of 1024 threads
+// exclusive scan of cnt[0..m) into out[0..m], one workgroup of 1024 threads
 __global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ cnt, int m, int* __restrict__ out) {
-  __shared__ long long part[1024];
-  const int t = threadIdx.x;
-  const int chunk = (m + 1023) / 1024;
-  const int b = t * chunk, e = min(m, b + chunk);
-  long long s = 0;
-  for (int i = b; i < e; ++i) s += cnt[i];
-  part[t] = s;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    long long v = (t >= o) ? part[t - o] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
-  }
-  long long run = part[t] - s;
-  for (int i = b; i < e; ++i) {
-    out[i] = (int)run;
-    run += cnt[i];
-  }
-  if (t == 1023) out[m] = (int)part[1023];
+  scan_1024(cnt, m, out);
 }
 
 __global__ void k_nl_scatter(const int* __restrict__ abin, int n, const int* __restrict__ bstart,
@@ -709,12 +691,93 @@ static __device__ __forceinline__ bool nl_pair(const double* __restrict__ pos, c
   return r2 < g.rc2;
 }
 
+// A wavefront's search for receiver a (whose bin, lin, counts from its
+// structure's first bin b0): the 64 lanes load 64 of the neighbouring bins'
+// ranges at once, a prefix sum over them numbers the candidates of all those
+// bins, and each lane tests one candidate of 64, so the lanes are full and a
+// round of loads serves 64 candidates.  (Bin after bin, a round served the 10
+// to 25 atoms of one bin and waited for its range first: 128 crystals of 8-200
+// atoms, 13k receivers, 27 to some hundred bins each: 175 us a pass, now 77;
+// 12,288 atoms of water 84 -> 37; 1,024 of fcc 24 -> 12.)  Hits are counted by ballot
+// and take their slots by rank, so the edge order is the serial one.  Returns
+// the number of edges.
+template <bool FILL>
+static __device__ __forceinline__ int nl_wave(const double* __restrict__ pos, const NlGeom& g, int b0, int lin, int a,
+                                              const int* __restrict__ aimg, const int* __restrict__ bstart,
+                                              const int* __restrict__ batoms, int base, int* __restrict__ src,
+                                              int* __restrict__ shift) {
+  const int lane = (int)(threadIdx.x & 63);
+  const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
+  const int ba[3] = {lin / (g.nb[1] * g.nb[2]), (lin / g.nb[2]) % g.nb[1], lin % g.nb[2]};
+  const int oa[3] = {aimg[3 * a], aimg[3 * a + 1], aimg[3 * a + 2]};
+  int lo[3], m[3];
+  for (int k = 0; k < 3; ++k) {
+    int l = ba[k] - g.reach[k], h = ba[k] + g.reach[k];
+    if (!g.pbc[k]) {
+      l = l < 0 ? 0 : l;
+      h = h >= g.nb[k] ? g.nb[k] - 1 : h;
+    }
+    lo[k] = l;
+    m[k] = h - l + 1;
+  }
+  const int nbin = m[0] * m[1] * m[2];
+  int cnt = 0;
+  for (int c0 = 0; c0 < nbin; c0 += 64) {
+    const int c = c0 + lane;
+    int q0 = 0, num = 0, sx = 0, sy = 0, sz = 0;
+    if (c < nbin) {
+      const int bx = lo[0] + c / (m[1] * m[2]), by = lo[1] + (c / m[2]) % m[1], bz = lo[2] + c % m[2];
+      const int wx = ((bx % g.nb[0]) + g.nb[0]) % g.nb[0], wy = ((by % g.nb[1]) + g.nb[1]) % g.nb[1],
+                wz = ((bz % g.nb[2]) + g.nb[2]) % g.nb[2];
+      sx = (bx - wx) / g.nb[0];
+      sy = (by - wy) / g.nb[1];
+      sz = (bz - wz) / g.nb[2];
+      const int bl = b0 + (wx * g.nb[1] + wy) * g.nb[2] + wz;
+      q0 = bstart[bl];
+      num = bstart[bl + 1] - q0;
+    }
+    int inc = num;   // inclusive prefix sum over the bins
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += u;
+    }
+    const int total = __shfl(inc, 63, 64);
+    for (int t0 = 0; t0 < total; t0 += 64) {
+      const int i = t0 + lane;
+      // the bin of candidate i: the number of bins whose prefix is <= i
+      int p = 0;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1)
+        if (__shfl(inc, p + o - 1, 64) <= i) p += o;
+      const int pb = p < 63 ? p : 63;   // (p = 64 only past the last candidate)
+      const int q = __shfl(q0, pb, 64) + i - (__shfl(inc, pb, 64) - __shfl(num, pb, 64));
+      const int tx = __shfl(sx, pb, 64), ty = __shfl(sy, pb, 64), tz = __shfl(sz, pb, 64);
+      int S[3] = {0, 0, 0};
+      int b = 0;
+      bool hit = false;
+      if (i < total) {
+        b = batoms[q];
+        hit = nl_pair(pos, aimg, g, a, ax, ay, az, oa, tx, ty, tz, b, S);
+      }
+      const unsigned long long mask = __ballot(hit);
+      if (FILL && hit) {
+        const int slot = base + cnt + __popcll(mask & ((1ull << lane) - 1ull));
+        src[slot] = b;
+        shift[3 * slot] = S[0];
+        shift[3 * slot + 1] = S[1];
+        shift[3 * slot + 2] = S[2];
+      }
+      cnt += __popcll(mask);
+    }
+  }
+  return cnt;
+}
+
 // For receiver a: every source b and shift S with |r_a - r_b + S.cell|^2 < rc^2,
 // (b, S) != (a, 0) (nl_pair: the distance exactly as the brute-force oracle
 // evaluates it for edge (i=b, j=a, S)).  WAVE = false: one thread per receiver;
-// WAVE = true: one wavefront per receiver (four per workgroup), the 64 lanes
-// over each bin's candidates, counts by ballot and fill slots by the rank of
-// the lane's hit among the wave's hits, so the edge order is the serial one.
+// WAVE = true: one wavefront per receiver (four per workgroup; nl_wave).
 // A structure of n atoms gives only n / 64 wavefronts with a thread per
 // receiver; below NL_WAVE_MAX atoms the wavefront form fills the GPU.
 constexpr int NL_WAVE_MAX = 32768;
@@ -728,6 +791,11 @@ __global__ __launch_bounds__(256) void k_nl_edges(const double* __restrict__ pos
   const int lane = WAVE ? (int)(threadIdx.x & 63) : 0;
   const int a = WAVE ? (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) : (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (a >= n) return;
+  if constexpr (WAVE) {
+    const int c = nl_wave<FILL>(pos, g, 0, abin[a], a, aimg, bstart, batoms, FILL ? rowptr[a] : 0, src, shift);
+    if (!FILL && lane == 0) counts[a] = c;
+    return;
+  }
   const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
   const int lin = abin[a];
   const int ba[3] = {lin / (g.nb[1] * g.nb[2]), (lin / g.nb[2]) % g.nb[1], lin % g.nb[2]};
@@ -754,48 +822,29 @@ __global__ __launch_bounds__(256) void k_nl_edges(const double* __restrict__ pos
         const int sz = (bz - wz) / g.nb[2];
         const int bl = (wx * g.nb[1] + wy) * g.nb[2] + wz;
         const int q1 = bstart[bl + 1];
-        for (int q0 = bstart[bl]; q0 < q1; q0 += (WAVE ? 64 : 1)) {
-          const int q = q0 + lane;
-          int S[3] = {0, 0, 0};
-          int b = 0;
-          bool hit = false;
-          if (q < q1) {
-            b = batoms[q];
-            hit = nl_pair(pos, aimg, g, a, ax, ay, az, oa, sx, sy, sz, b, S);
+        for (int q = bstart[bl]; q < q1; ++q) {
+          const int b = batoms[q];
+          int S[3];
+          if (!nl_pair(pos, aimg, g, a, ax, ay, az, oa, sx, sy, sz, b, S)) continue;
+          if (FILL) {
+            const int slot = base + cnt;
+            src[slot] = b;
+            shift[3 * slot] = S[0];
+            shift[3 * slot + 1] = S[1];
+            shift[3 * slot + 2] = S[2];
           }
-          if (WAVE) {
-            const unsigned long long m = __ballot(hit);
-            if (FILL && hit) {
-              const int slot = base + cnt + __popcll(m & ((1ull << lane) - 1ull));
-              src[slot] = b;
-              shift[3 * slot] = S[0];
-              shift[3 * slot + 1] = S[1];
-              shift[3 * slot + 2] = S[2];
-            }
-            cnt += __popcll(m);
-          } else if (hit) {
-            if (FILL) {
-              const int slot = base + cnt;
-              src[slot] = b;
-              shift[3 * slot] = S[0];
-              shift[3 * slot + 1] = S[1];
-              shift[3 * slot + 2] = S[2];
-            }
-            ++cnt;
-          }
+          ++cnt;
         }
       }
     }
   }
-  if (!FILL && lane == 0) counts[a] = cnt;
+  if (!FILL) counts[a] = cnt;
 }
 
 // WAVE = false: one thread per receiver (large structures: enough receivers
-// to fill the GPU).  WAVE = true: one wavefront per receiver, the 64 lanes
-// over each bin's candidates; counts by ballot, fill slots by the rank of the
-// lane's hit among the wave's hits -- the candidate order, and so the edge
-// order, is the serial one (small structures, where a thread per receiver
-// would leave the GPU idle behind a few long serial loops).
+// to fill the GPU).  WAVE = true: one wavefront per receiver (nl_wave; small
+// structures, where a thread per receiver would leave the GPU idle behind a
+// few long serial loops).
 template <bool FILL, bool WAVE>
 __global__ __launch_bounds__(256) void k_nlb_edges(const double* __restrict__ pos, int n, NlBatch B,
                                                    const int* __restrict__ abin, const int* __restrict__ aimg,
@@ -808,6 +857,11 @@ __global__ __launch_bounds__(256) void k_nlb_edges(const double* __restrict__ po
   const int s = nlb_struct_of(B, a);
   const NlGeom& g = B.geo[s];
   const int b0 = B.boff[s];
+  if constexpr (WAVE) {
+    const int c = nl_wave<FILL>(pos, g, b0, abin[a] - b0, a, aimg, bstart, batoms, FILL ? rowptr[a] : 0, src, shift);
+    if (!FILL && lane == 0) counts[a] = c;
+    return;
+  }
   const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
   const int lin = abin[a] - b0;
   const int ba[3] = {lin / (g.nb[1] * g.nb[2]), (lin / g.nb[2]) % g.nb[1], lin % g.nb[2]};
@@ -834,40 +888,23 @@ __global__ __launch_bounds__(256) void k_nlb_edges(const double* __restrict__ po
         const int sz = (bz - wz) / g.nb[2];
         const int bl = b0 + (wx * g.nb[1] + wy) * g.nb[2] + wz;
         const int q1 = bstart[bl + 1];
-        for (int q0 = bstart[bl]; q0 < q1; q0 += (WAVE ? 64 : 1)) {
-          const int q = q0 + lane;
-          int S[3] = {0, 0, 0};
-          int b = 0;
-          bool hit = false;
-          if (q < q1) {
-            b = batoms[q];
-            hit = nl_pair(pos, aimg, g, a, ax, ay, az, oa, sx, sy, sz, b, S);
+        for (int q = bstart[bl]; q < q1; ++q) {
+          const int b = batoms[q];
+          int S[3];
+          if (!nl_pair(pos, aimg, g, a, ax, ay, az, oa, sx, sy, sz, b, S)) continue;
+          if (FILL) {
+            const int slot = base + cnt;
+            src[slot] = b;
+            shift[3 * slot] = S[0];
+            shift[3 * slot + 1] = S[1];
+            shift[3 * slot + 2] = S[2];
           }
-          if (WAVE) {
-            const unsigned long long m = __ballot(hit);
-            if (FILL && hit) {
-              const int slot = base + cnt + __popcll(m & ((1ull << lane) - 1ull));
-              src[slot] = b;
-              shift[3 * slot] = S[0];
-              shift[3 * slot + 1] = S[1];
-              shift[3 * slot + 2] = S[2];
-            }
-            cnt += __popcll(m);
-          } else if (hit) {
-            if (FILL) {
-              const int slot = base + cnt;
-              src[slot] = b;
-              shift[3 * slot] = S[0];
-              shift[3 * slot + 1] = S[1];
-              shift[3 * slot + 2] = S[2];
-            }
-            ++cnt;
-          }
+          ++cnt;
         }
       }
     }
   }
-  if (!FILL && lane == 0) counts[a] = cnt;
+  if (!FILL) counts[a] = cnt;
 }
 
 // --------------------------------------------------------------- C ABI --
