@@ -593,6 +593,10 @@ int tace_so2_gemm_bf16_kt(const uint16_t* a, int64_t lda, const uint16_t* b_frag
 int tace_edge_pairs(const int32_t* rowptr, const int32_t* eid, const int32_t* src, const int32_t* shifts,
                     int64_t n_nodes, int64_t n_edges, int32_t* work, int32_t* w_rows, int32_t* row_edges,
                     int32_t* row_partner, void* stream);
+/* edge_index [2, n_edges] int64 (senders, receivers) and the receivers as
+ * int32 of a receiver CSR rowptr [n_nodes + 1], src [n_edges]. */
+int tace_edge_index(const int32_t* rowptr, const int32_t* src, int64_t n_nodes, int64_t n_edges, int64_t* edge_index,
+                    int32_t* dst32, void* stream);
 /* y [m, n] = x [m, k] @ B (+ bias [n]) in float32 on the bf16 MFMA (three
  * terms per operand, six products): the fragment-order tile kernel of
  * tace_seg_linear_presplit_frag without tables.  w_frag: B [k, n] in the

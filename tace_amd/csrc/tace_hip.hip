@@ -907,6 +907,21 @@ __global__ __launch_bounds__(256) void k_nlb_edges(const double* __restrict__ po
   if (!FILL) counts[a] = cnt;
 }
 
+// The edge list of a receiver CSR in the form callers pass around: ei [2, E]
+// int64 (senders, receivers) and the receivers as int32.  A wavefront per
+// receiver; one launch for what took eight (a difference, a scan, a repeat,
+// two conversions, a stack): 361k edges in 5.5 us.
+__global__ __launch_bounds__(256) void k_edge_index(const int* __restrict__ rowptr, const int* __restrict__ src, int n,
+                                                    int64_t E, int64_t* __restrict__ ei, int* __restrict__ dst32) {
+  const int a = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (a >= n) return;
+  for (int k = rowptr[a] + (int)(threadIdx.x & 63); k < rowptr[a + 1]; k += 64) {
+    ei[k] = src[k];
+    ei[E + k] = a;
+    dst32[k] = a;
+  }
+}
+
 // --------------------------------------------------------------- C ABI --
 extern "C" {
 
@@ -1473,8 +1488,7 @@ int tace_nl_count(const double* pos, int64_t n_atoms, const double* cell, const 
   int* bfill = bstart + nbins + 1;
   int* batoms = bfill + nbins;
   int* unsorted = batoms + n;
-  launch_fill<int>(bcount, (size_t)nbins, 0, s);
-  launch_fill<int>(bfill, (size_t)nbins, 0, s);
+  launch_fill<int>(bcount, (size_t)(3 * nbins + 1), 0, s);   // bcount, bstart, bfill
   const dim3 ga((n + 255) / 256), ba(256);
   hipLaunchKernelGGL(k_nl_bin, ga, ba, 0, s, pos, n, g, abin, aimg, bcount);
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, bcount, (int)nbins, bstart);
@@ -1596,8 +1610,7 @@ int tace_nl_batch_count(const double* pos, int64_t n_atoms, int32_t n_structs, c
   int* bfill = bstart + nb + 1;
   int* batoms = bfill + nb;
   int* unsorted = batoms + n;
-  launch_fill<int>(bcount, (size_t)nb, 0, s);
-  launch_fill<int>(bfill, (size_t)nb, 0, s);
+  launch_fill<int>(bcount, (size_t)(3 * (int64_t)nb + 1), 0, s);   // bcount, bstart, bfill
   const dim3 ga((n + 255) / 256), ba(256);
   hipLaunchKernelGGL(k_nlb_bin, ga, ba, 0, s, pos, n, B, abin, aimg, bcount);
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, bcount, nb, bstart);
@@ -1635,6 +1648,17 @@ int tace_nl_batch_fill(const double* pos, int64_t n_atoms, int32_t n_structs, co
     hipLaunchKernelGGL((k_nlb_edges<true, false>), dim3((n + 255) / 256), dim3(256), 0, s, pos, n, B, abin, aimg,
                        bstart, batoms, nullptr, rowptr, src, shifts);
   return check_launch("tace_nl_batch_fill");
+}
+
+int tace_edge_index(const int32_t* rowptr, const int32_t* src, int64_t n_nodes, int64_t n_edges, int64_t* edge_index,
+                    int32_t* dst32, void* stream) {
+  if (n_nodes < 0 || n_nodes > INT32_MAX - 4 || n_edges < 0 || n_edges > INT32_MAX)
+    return fail("tace_edge_index: bad sizes");
+  if (n_nodes == 0 || n_edges == 0) return 0;
+  if (!rowptr || !src || !edge_index || !dst32) return fail("tace_edge_index: null pointer");
+  hipLaunchKernelGGL(k_edge_index, dim3((unsigned)((n_nodes + 3) / 4)), dim3(256), 0, (hipStream_t)stream, rowptr, src,
+                     (int)n_nodes, n_edges, edge_index, dst32);
+  return check_launch("tace_edge_index");
 }
 
 static int rows_accumulate(int dtype, const void* rows, int64_t n_rows, int64_t width, const int32_t* rowptr,

@@ -57,15 +57,13 @@ def device_graph(p64: torch.Tensor, sizes: Sequence[int], cells, pbcs, cutoff: f
     (``edge_index[1]`` non-decreasing), node ids batch-global.  Returns
     edge_index (int64), integer edge_shifts (int32) and the receiver CSR plan
     the model's kernels take (``_edge_plan``, ``_dst32``)."""
-    from .ops import EdgePlan, neighbour_list_batch
+    from .ops import EdgePlan, edge_index_of, neighbour_list_batch
 
     n_tot = int(p64.shape[0])
     rowptr, src, shifts = neighbour_list_batch(p64, sizes, cells, pbcs, cutoff)
-    E = src.shape[0]
-    counts = (rowptr[1:] - rowptr[:-1]).to(torch.int64)
-    dst = torch.repeat_interleave(torch.arange(n_tot, device=p64.device), counts, output_size=E)
-    return dict(edge_index=torch.stack([src.to(torch.int64), dst]), edge_shifts=shifts,
-                _edge_plan=EdgePlan(n_tot, E, rowptr, src, None), _dst32=dst.to(torch.int32), _shifts32=shifts)
+    ei, dst = edge_index_of(rowptr, src)
+    return dict(edge_index=ei, edge_shifts=shifts, _edge_plan=EdgePlan(n_tot, src.shape[0], rowptr, src, None),
+                _dst32=dst, _shifts32=shifts)
 
 
 def gpu_graph(structs: List[Dict], atomic_numbers: Sequence[int], cutoff: float, dtype=torch.float32,
@@ -111,22 +109,21 @@ def resident_graph(pos64: torch.Tensor, cell, pbc, node_attrs: torch.Tensor, cut
                    dtype=torch.float32) -> Dict[str, torch.Tensor]:
     """One periodic structure already resident on the GPU (float64 positions)
     -> model input dict, neighbour list rebuilt by the HIP cell list."""
-    from .ops import EdgePlan, neighbour_list
+    from .ops import EdgePlan, edge_index_of, neighbour_list
 
     n = pos64.shape[0]
     dev = pos64.device
     rowptr, src, sh = neighbour_list(pos64, cell, pbc, cutoff)
-    counts = (rowptr[1:] - rowptr[:-1]).to(torch.int64)
-    dst = torch.repeat_interleave(torch.arange(n, device=dev), counts, output_size=int(src.shape[0]))
+    ei, dst32 = edge_index_of(rowptr, src)
     # ptr [0, n] by a fill kernel, the lattice from a cache (host-to-device
     # copies of pageable memory wait for the GPU to go idle)
     ptr = torch.zeros(2, dtype=torch.int64, device=dev)
     ptr[1:] = n
     d = dict(positions=pos64.to(dtype), node_attrs=node_attrs,
-             edge_index=torch.stack([src.to(torch.int64), dst]), edge_shifts=sh.to(dtype),
+             edge_index=ei, edge_shifts=sh.to(dtype),
              lattice=_device_cell(cell, dtype, dev), batch=torch.zeros(n, dtype=torch.int64, device=dev), ptr=ptr)
     d["_edge_plan"] = EdgePlan(n, int(src.shape[0]), rowptr, src, None)
-    d["_shifts32"] = sh
+    d["_dst32"], d["_shifts32"] = dst32, sh
     return d
 
 

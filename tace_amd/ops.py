@@ -2389,6 +2389,19 @@ def neighbour_list(positions: torch.Tensor, cell, pbc, cutoff: float):
     return rowptr, src, shifts
 
 
+def edge_index_of(rowptr: torch.Tensor, src: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(edge_index int64 [2, E], receivers int32 [E]) of a receiver CSR
+    (``tace_edge_index``)."""
+    n, E = rowptr.shape[0] - 1, src.shape[0]
+    _req(rowptr, "rowptr", torch.int32, (n + 1,))
+    _req(src, "src", torch.int32, (E,))
+    ei = torch.empty(2, E, dtype=torch.int64, device=src.device)
+    dst = torch.empty(E, dtype=torch.int32, device=src.device)
+    N.check(N.lib().tace_edge_index(rowptr.data_ptr(), src.data_ptr(), n, E, ei.data_ptr(), dst.data_ptr(),
+                                    N.stream_ptr(src.device)), "tace_edge_index")
+    return ei, dst
+
+
 def neighbour_list_batch(positions: torch.Tensor, sizes: Sequence[int], cells, pbcs, cutoff: float,
                          mode: int = 0):
     """The cell-list neighbour search for a batch of structures in one pass

@@ -204,3 +204,18 @@ def test_gemm_bx3_and_layout_match_float64(cuda, m, k, n, bias):
     assert ((y.double() - want).norm() / want.norm()).item() < tol(k)
     want = go.double() @ full.double()
     assert ((gx.double() - want).norm() / want.norm()).item() < tol(n)
+
+
+@pytest.mark.parametrize("n,most", [(1, 0), (1, 200), (5, 63), (7, 64), (300, 129)])
+def test_edge_index_of_csr(cuda, n, most):
+    """Senders and receivers of a receiver CSR: empty receivers, runs below,
+    at and above a wavefront, a last group of receivers that is not full."""
+    g = torch.Generator().manual_seed(n + most)
+    counts = torch.randint(0, most + 1, (n,), generator=g)
+    counts[n // 2] = most
+    rowptr = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).to(torch.int32)
+    src = torch.randint(0, n, (int(counts.sum()),), generator=g, dtype=torch.int32)
+    ei, dst = ops.edge_index_of(rowptr.to(cuda), src.to(cuda))
+    want = torch.repeat_interleave(torch.arange(n), counts)
+    assert ei.dtype == torch.int64 and dst.dtype == torch.int32
+    assert torch.equal(ei.cpu(), torch.stack([src.to(torch.int64), want])) and torch.equal(dst.cpu().to(torch.int64), want)
