@@ -1989,44 +1989,37 @@ class SegLinearPlan:
         # when every instruction has a fragment-order block
         self.tile_frag = bool(self.split_weights and frag is not None and SEG_TILE_FRAG
                               and all(len(c) > 6 and c[6] >= 0 for c in ins))
+        # the ranges as arrays: every tile of a block over all species at once
+        rng = np.array([(-1 if sp is None else sp, a, b) for sp, a, b in ranges if b > a], dtype=np.int64).reshape(-1, 3)
         for ob, (s_o, n, d, boff) in enumerate(out_blocks):
             mine = [c for c in ins if c[0] == ob]
             if (self.split_weights and frag is not None and SEG_KS_MIN_N is not None and n >= SEG_KS_MIN_N
                     and len(mine) <= 1 and all(c[2] <= 256 and c[6] >= 0 for c in mine)):
-                tasks += self._ks_tasks(Z, s_o, n, d, boff, mine, ranges, frag[0], b_stride)
+                tasks.append(self._ks_tasks(Z, s_o, n, d, boff, mine, rng, frag[0], b_stride))
                 continue
             c0s = np.arange(0, n, TN, dtype=np.int64)
-            for (sp, a, b) in ranges:
-                if b <= a:
-                    continue
-                r0 = np.arange(a * d, b * d, TM, dtype=np.int64)
-                rows = np.minimum(b * d - r0, TM)
-                R, Cc = np.meshgrid(r0, c0s, indexing="ij")
-                Rows = np.broadcast_to(rows[:, None], R.shape)
-                T = R.size
-                t = np.zeros((T, 8), dtype=np.int64)
-                t[:, 0] = Z * s_o + R.ravel() * n
-                t[:, 1] = Rows.ravel()
-                t[:, 2] = n
-                t[:, 3] = Cc.ravel()
-                t[:, 4] = -1 if boff is None else boff + (0 if sp is None else sp * b_stride)
-                k_each = len(mine)
-                t[:, 5] = nc + np.arange(T, dtype=np.int64) * k_each
-                t[:, 6] = t[:, 5] + k_each
-                nc += T * k_each
-                tiles.append(t)
-                if k_each:
-                    c = np.zeros((T, k_each, 4), dtype=np.int64)
-                    for j, (_, s_i, k, w_off, trans, sc, *_f) in enumerate(mine):
-                        c[:, j, 0] = Z * s_i + R.ravel() * k
-                        c[:, j, 1] = k
-                        if self.tile_frag:
-                            c[:, j, 2] = _f[0] + (0 if sp is None else sp * frag[0])
-                        else:
-                            c[:, j, 2] = w_off + (0 if sp is None else sp * w_stride)
-                        c[:, j, 3] = int(trans)
-                    contribs.append(c.reshape(-1, 4))
-                    scales.append(np.tile(np.array([m[5] for m in mine], dtype=np.float64), T))
+            r0, rows, sp = (np.repeat(v, len(c0s)) for v in self._row_tiles(rng, d, TM))
+            T = len(r0)
+            t = np.zeros((T, 8), dtype=np.int64)
+            t[:, 0] = Z * s_o + r0 * n
+            t[:, 1] = rows
+            t[:, 2] = n
+            t[:, 3] = np.tile(c0s, T // max(1, len(c0s)))
+            t[:, 4] = -1 if boff is None else boff + sp * b_stride
+            k_each = len(mine)
+            t[:, 5] = nc + np.arange(T, dtype=np.int64) * k_each
+            t[:, 6] = t[:, 5] + k_each
+            nc += T * k_each
+            tiles.append(t)
+            if k_each:
+                c = np.zeros((T, k_each, 4), dtype=np.int64)
+                for j, (_, s_i, k, w_off, trans, sc, *_f) in enumerate(mine):
+                    c[:, j, 0] = Z * s_i + r0 * k
+                    c[:, j, 1] = k
+                    c[:, j, 2] = _f[0] + sp * frag[0] if self.tile_frag else w_off + sp * w_stride
+                    c[:, j, 3] = int(trans)
+                contribs.append(c.reshape(-1, 4))
+                scales.append(np.tile(np.array([m[5] for m in mine], dtype=np.float64), T))
         t = np.concatenate(tiles) if tiles else np.zeros((0, 8), dtype=np.int64)
         c = np.concatenate(contribs) if contribs else np.zeros((0, 4), dtype=np.int64)
         s = np.concatenate(scales) if scales else np.zeros(0, dtype=np.float64)
@@ -2086,7 +2079,7 @@ class SegLinearPlan:
         self.contribs = torch.from_numpy(np.ascontiguousarray(c) if len(c) else np.zeros((1, 4), np.int64)).to(device)
         self.scales = torch.from_numpy(s if len(s) else np.zeros(1)).to(device)
         # short-k tasks (tace_seg_linear_presplit_ks), checked like the tiles
-        k_t = np.asarray(tasks, dtype=np.int64).reshape(-1, 10)
+        k_t = np.concatenate(tasks) if tasks else np.zeros((0, 10), dtype=np.int64)
         if len(k_t):
             if (k_t[:, 0] + (k_t[:, 1] - 1) * k_t[:, 2] + k_t[:, 4]).max() > y_numel:
                 raise ValueError("seg linear plan: output task out of range")
@@ -2131,27 +2124,36 @@ class SegLinearPlan:
             raise ValueError(f"seg linear plan: no short-k task kernel for k = {k}")
         return R
 
-    def _ks_tasks(self, Z, s_o, n, d, boff, mine, ranges, f_stride, b_stride):
+    @staticmethod
+    def _row_tiles(rng: np.ndarray, d: int, R: int):
+        """(first row, rows, species or 0) of the R-row tiles of every range
+        (species or -1, a, b) of a block with d rows per node, range by range."""
+        lo, hi = rng[:, 1] * d, rng[:, 2] * d
+        num = (hi - lo + R - 1) // R
+        own = np.repeat(np.arange(len(rng)), num)
+        r0 = lo[own] + R * (np.arange(len(own)) - np.repeat(np.cumsum(num) - num, num))
+        return r0, np.minimum(hi[own] - r0, R), np.maximum(rng[own, 0], 0)
+
+    def _ks_tasks(self, Z, s_o, n, d, boff, mine, rng, f_stride, b_stride) -> np.ndarray:
         """Tasks of one output block (one contribution with k <= 128, or
         none): column chunk-major, so that the workgroups running at one time
         on an XCD share a chunk's weight columns in its L2."""
-        out = []
         R = self._ks_rows(mine[0][2] if mine else 0)   # the task height for this k
-        for cb in range(0, n, SEG_KS_CHUNK):
-            ce = min(n, cb + SEG_KS_CHUNK)
-            for (sp, a, b) in ranges:
-                if b <= a:
-                    continue
-                for r0 in range(a * d, b * d, R):
-                    rows = min(b * d - r0, R)
-                    bo = -1 if boff is None else boff + (0 if sp is None else sp * b_stride)
-                    if mine:
-                        s_i, k, f_off = mine[0][1], mine[0][2], mine[0][6]
-                        out.append((Z * s_o + r0 * n, rows, n, cb, ce, bo, Z * s_i + r0 * k, k,
-                                    f_off + (0 if sp is None else sp * f_stride), 0))
-                    else:
-                        out.append((Z * s_o + r0 * n, rows, n, cb, ce, bo, 0, 0, 0, 0))
-        return out
+        r0, rows, sp = self._row_tiles(rng, d, R)
+        cb = np.arange(0, n, SEG_KS_CHUNK, dtype=np.int64)
+        t = np.zeros((len(cb), len(r0), 10), dtype=np.int64)
+        t[:, :, 0] = Z * s_o + r0 * n
+        t[:, :, 1] = rows
+        t[:, :, 2] = n
+        t[:, :, 3] = cb[:, None]
+        t[:, :, 4] = np.minimum(n, cb + SEG_KS_CHUNK)[:, None]
+        t[:, :, 5] = -1 if boff is None else boff + sp * b_stride
+        if mine:
+            s_i, k, f_off = mine[0][1], mine[0][2], mine[0][6]
+            t[:, :, 6] = Z * s_i + r0 * k
+            t[:, :, 7] = k
+            t[:, :, 8] = f_off + sp * f_stride
+        return t.reshape(-1, 10)
 
 
 def _addend_ptr(addend: Optional[torch.Tensor], y: torch.Tensor):
@@ -2389,6 +2391,19 @@ def neighbour_list(positions: torch.Tensor, cell, pbc, cutoff: float):
     return rowptr, src, shifts
 
 
+def _stacked(items, dtype, shape, one) -> np.ndarray:
+    """One array [len(items), *shape] of per-structure values: made in one
+    step where they all have that shape (128 cells and flags: 0.1 against 1.2
+    ms item by item), else each one brought to it by ``one``."""
+    try:
+        a = np.asarray(items, dtype=dtype)
+        if a.shape == (len(items),) + shape:
+            return np.ascontiguousarray(a)
+    except (TypeError, ValueError, RuntimeError):   # items of different shapes, tensors
+        pass
+    return np.ascontiguousarray(np.stack([one(np.asarray(v, dtype=dtype)) for v in items]))
+
+
 def edge_index_of(rowptr: torch.Tensor, src: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """(edge_index int64 [2, E], receivers int32 [E]) of a receiver CSR
     (``tace_edge_index``)."""
@@ -2422,8 +2437,8 @@ def neighbour_list_batch(positions: torch.Tensor, sizes: Sequence[int], cells, p
     if positions.shape[0] != n_tot:
         raise ValueError(f"positions has {positions.shape[0]} rows, sizes sum to {n_tot}")
     sizes_np = np.ascontiguousarray(np.asarray(sizes, dtype=np.int64))
-    cells_np = np.ascontiguousarray(np.stack([np.asarray(c, dtype=np.float64).reshape(3, 3) for c in cells]))
-    pbcs_np = np.ascontiguousarray(np.stack([np.broadcast_to(np.asarray(p, dtype=np.int32), (3,)) for p in pbcs]))
+    cells_np = _stacked(cells, np.float64, (3, 3), lambda c: c.reshape(3, 3))
+    pbcs_np = _stacked(pbcs, np.int32, (3,), lambda p: np.broadcast_to(p, (3,)))
     na, nb = ctypes.c_int64(0), ctypes.c_int64(0)
     need = L.tace_nl_batch_plan(ns, sizes_np.ctypes.data, cells_np.ctypes.data, pbcs_np.ctypes.data, float(cutoff),
                                 None, 0, ctypes.byref(na), ctypes.byref(nb))

@@ -92,3 +92,33 @@ def test_seg_linear_streamed_weights_split(cuda, steps, want, monkeypatch):
     assert torch.equal(got, run())
     # k = 1100 products of unit variance in another order: 2^-24 sqrt(k) each way
     assert ((got - ref).abs().max() / ref.abs().max()).item() < 4e-6
+
+
+@pytest.mark.parametrize("d,R", [(1, 64), (3, 64), (7, 128)])
+def test_row_tiles_of_every_range(d, R):
+    """Range by range, in order: no tile crosses a range, the last of each holds its remainder."""
+    counts, rng, at = [1, 63, 64, 65, 0, 200], [], 0
+    for s, c in enumerate(counts):
+        rng.append((s if s else -1, at, at + c))
+        at += c
+    want = [(r, min(b * d - r, R), max(s, 0)) for s, a, b in rng for r in range(a * d, b * d, R)]
+    got = ops.SegLinearPlan._row_tiles(np.array(rng, dtype=np.int64), d, R)
+    assert [tuple(map(int, v)) for v in zip(*got)] == want
+    assert all(len(v) == 0 for v in ops.SegLinearPlan._row_tiles(np.zeros((0, 3), np.int64), d, R))
+
+
+def test_stacked_values_of_structures():
+    """The quick form and the item by item one give the same array and refuse the same items."""
+    cell = lambda c: c.reshape(3, 3)
+    flag = lambda p: np.broadcast_to(p, (3,))
+    c = np.arange(18, dtype=np.float64).reshape(2, 3, 3)
+    for items in (list(c), list(c.reshape(2, 9)), c.tolist(), [c[0], c[1].ravel()], list(torch.from_numpy(c)), c):
+        assert np.array_equal(ops._stacked(items, np.float64, (3, 3), cell), c)
+    want = np.array([[1, 1, 0], [1, 1, 1]], dtype=np.int32)
+    for items in ([(True, True, False), True], [[1, 1, 0], [1]], want.tolist(), list(torch.from_numpy(want))):
+        got = ops._stacked(items, np.int32, (3,), flag)
+        assert got.dtype == np.int32 and np.array_equal(got, want)
+    for items, dtype, shape, one in (([], np.float64, (3, 3), cell), ([np.zeros((3, 2))], np.float64, (3, 3), cell),
+                                     ([1.0], np.float64, (3, 3), cell), ([np.ones((3, 1))], np.int32, (3,), flag)):
+        with pytest.raises(ValueError):
+            ops._stacked(items, dtype, shape, one)
