@@ -316,15 +316,14 @@ int tace_seg_linear_presplit(const float* x, float* y, const float* addend, cons
                              double alpha, void* stream);
 /* The same linears' tiles with one contribution of k <= 256 (the input
  * gradients of the product-basis contractions, linear.py:377-482, and any
- * block with no contribution), as n_tasks row tiles of up to task_rows rows,
+ * block with no contribution), as n_tasks row tiles of up to 64 rows
+ * (tace_seg_linear_ks_rows(k): the height for k, 0 when not supported),
  * each over a column range, with the weights split in MFMA fragment order
- * (tace_bf16x3_split_blocks layout 1).  task_rows is 128 (every task's k <=
- * 128) or 64 (k <= 256): tace_seg_linear_ks_rows(k) gives the height for k
- * (0: not supported); one call takes tasks of one height.  A task whose k
- * exceeds its height's limit (128 for 128-row tasks, 256 for 64-row tasks)
- * gets NaN in every output of its tile:
+ * (tace_bf16x3_split_blocks layout 1).  k_max is 128 or 256: every task's k is
+ * at most that, and a task whose k exceeds it gets NaN in every output of its
+ * tile:
  *   tasks int64 [n_tasks, 10]: out_base (offset of the tile's row 0, column 0
- *         in y), rows (1..task_rows), n (block width = row stride of y), cb, ce (its
+ *         in y), rows (1..64), n (block width = row stride of y), cb, ce (its
  *         columns [cb, ce), ce <= n), bias_off (-1 none), x_base (offset of
  *         the tile's row 0 in x), k (0..256, the row stride of x; 0: no
  *         contribution), w_off (the block's offset in w_frag), unused.
@@ -346,7 +345,7 @@ int tace_seg_linear_presplit_frag(const float* x, float* y, const float* addend,
                                   double alpha, void* stream);
 int tace_seg_linear_presplit_ks(const float* x, float* y, const float* addend, const uint16_t* w_frag,
                                 const float* bias,
-                                const int64_t* tasks, int64_t n_tasks, int32_t task_rows, double alpha, void* stream);
+                                const int64_t* tasks, int64_t n_tasks, int32_t k_max, double alpha, void* stream);
 /* tace_seg_linear_presplit_frag with k split over `splits` (2..64)
  * workgroups per tile, for launches with too few tiles to fill the GPU (the
  * small systems' per-species linears, linear.py:377-482): every tile has at

@@ -834,14 +834,15 @@ __global__ __launch_bounds__(256) void k_seg_split_sum(float* y, const float* ad
 // x [128, n] with n up to ~5,400 columns per output block.  A 128 x 128 tile
 // of the kernel above does four 32-k steps after staging A and B through LDS
 // with two barriers per step, then writes its outputs one float per lane.
-// Here a workgroup owns one R-row tile of one contribution with k <= KM (R =
-// 128 for k <= 128, R = 64 for k <= 256) and a range of columns:
+// Here a workgroup owns one R-row tile of one contribution with k <= KM
+// and a range of columns:
 //  * A is split once into the three bf16 planes in LDS (k-contiguous rows of
-//    128 + 8 bf16: 272-byte rows, so the 16 rows of a fragment read fall on
-//    distinct banks); one barrier, none after it;
-//  * KS_GROUPS groups of four wavefronts take the range's 128-column tiles in
+//    KM + 8 bf16, so the 16 rows of a fragment read fall on distinct banks),
+//    its loads all in flight together; one barrier, none after it;
+//  * GROUPS groups of four wavefronts take the range's 128-column tiles in
 //    turn; a wavefront owns all R rows of 32 columns, so each B fragment
-//    is loaded by one wavefront only;
+//    is loaded by one wavefront only; a tile of at most 32 rows (a species'
+//    last one) multiplies two row blocks instead of four;
 //  * B comes from weights pre-split in MFMA fragment order (k_split_blocks,
 //    layout 1): the three terms of one 16-column x 32-k fragment are three
 //    contiguous 1 KB runs in lane order, so a fragment is one fully
@@ -863,14 +864,24 @@ __global__ __launch_bounds__(256) void k_seg_split_sum(float* y, const float* ad
 // tile's row 0 in x), k (0..KM, the row stride of x; 0 = no contribution:
 // the tile is alpha * bias or zero), w_off (the block's offset in the
 // fragment-order weights), unused.
-// Two instantiations: R = 128 rows per task for k <= 128, R = 64 for k <= 256
-// (the A planes take 3 R (KM + 8) bf16 of LDS, ~100 KB either way).  Groups of
-// four wavefronts per workgroup and the column stride between one group's
-// consecutive tiles:
-constexpr int KS_GROUPS = 2, KS_THREADS = 256 * KS_GROUPS, KS_CSTEP = 128 * KS_GROUPS;
-template <int R, int KM>
+//
+// Two shapes, both of 64 rows: k <= 128 in one group (52 KB of LDS, three
+// workgroups per CU), k <= 256 in two groups (101 KB, one).  Large launches
+// are bound by power and by the writes: 5,184 rows of the 593 x 128 columns of
+// a product basis run the MFMAs at 1.36 PFLOP/s without the stores (442 us)
+// and take 671 us with them (1.6 GB: the two add up, the card is at its power
+// limit), 709 us with 128 rows per workgroup and one workgroup per CU, whose
+// operands came in and went out behind nothing.  Small ones gain from the
+// smaller workgroups: 64 rows 41 -> 18 us, 400 rows 88 -> 55, 1,024 rows
+// 170 -> 164, 3,000 rows of 89 species 584 -> 538.  For k <= 256, 32 rows in
+// three workgroups per CU read B twice as often: 3,180 us became 3,431 (6,656
+// rows, 89 species, 256 channels; 3,258 before the loads in flight and the
+// plain stores).
+template <int R_, int KM_, int GROUPS>
 struct KsShape {
-  static constexpr int RB = R / 16, STR = KM + 8, PL = R * STR;
+  static constexpr int R = R_, KM = KM_, RB = R / 16, STR = KM + 8, PL = R * STR;
+  static constexpr int WAVES = GROUPS == 1 ? 3 : 2;   // wavefronts per SIMD
+  static constexpr int THREADS = 256 * GROUPS, CSTEP = 128 * GROUPS;
 };
 
 struct KsTask {
@@ -893,19 +904,18 @@ __device__ __forceinline__ void ks_load_b(const KsTask& T, int c, int ks, int wq
 }
 
 // step KS of a column tile: MFMAs on cur while the next step's fragments
-// (or the next tile's first) load into nxt
-template <int R, int KM, int NKS, int KS>
+// (or the next tile's first) load into nxt; RB: 16-row blocks that hold rows
+template <class S, int RB, int NKS, int KS>
 __device__ __forceinline__ void ks_step(const unsigned short* __restrict__ As, const KsTask& T, int c, int wq,
-                                        int lane, int fr, int fg, f4 (&acc)[R / 16][2], const u4v (&cur)[3][2],
+                                        int lane, int fr, int fg, f4 (&acc)[RB][2], const u4v (&cur)[3][2],
                                         u4v (&nxt)[3][2]) {
   if (KS + 1 < NKS) ks_load_b(T, c, KS + 1, wq, lane, nxt);
-  else ks_load_b(T, c + KS_CSTEP, 0, wq, lane, nxt);
+  else ks_load_b(T, c + S::CSTEP, 0, wq, lane, nxt);
   // the loads go out before this step's MFMAs (the scheduler would sink them
   // to the end of the step, where nothing hides their latency)
   __builtin_amdgcn_sched_barrier(0);
-  typedef KsShape<R, KM> S;
 #pragma unroll
-  for (int ip = 0; ip < S::RB / 2; ++ip) {   // row blocks in pairs: four independent accumulators per term
+  for (int ip = 0; ip < RB / 2; ++ip) {   // row blocks in pairs: four independent accumulators per term
     bx3_bf8 af[2][3];
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii)
@@ -926,34 +936,43 @@ __device__ __forceinline__ void ks_step(const unsigned short* __restrict__ As, c
 }
 
 // steps KS.. of a column tile; step KS reads buffer (KS + PAR) & 1
-template <int R, int KM, int NKS, int PAR, int KS>
+template <class S, int RB, int NKS, int PAR, int KS>
 __device__ __forceinline__ void ks_steps(const unsigned short* __restrict__ As, const KsTask& T, int c, int wq,
-                                         int lane, int fr, int fg, f4 (&acc)[R / 16][2], u4v (&b0)[3][2],
+                                         int lane, int fr, int fg, f4 (&acc)[RB][2], u4v (&b0)[3][2],
                                          u4v (&b1)[3][2]) {
   if constexpr (KS < NKS) {
-    if constexpr (((KS + PAR) & 1) == 0) ks_step<R, KM, NKS, KS>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
-    else ks_step<R, KM, NKS, KS>(As, T, c, wq, lane, fr, fg, acc, b1, b0);
-    ks_steps<R, KM, NKS, PAR, KS + 1>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
+    if constexpr (((KS + PAR) & 1) == 0) ks_step<S, RB, NKS, KS>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
+    else ks_step<S, RB, NKS, KS>(As, T, c, wq, lane, fr, fg, acc, b1, b0);
+    ks_steps<S, RB, NKS, PAR, KS + 1>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
   }
 }
 
-// this wavefront's 128 x 32 part of column tile c
-template <int R, int KM, int NKS, int PAR>
+// lane l of each row of 16 takes lane l ^ 8's value (a rotation by 8)
+__device__ __forceinline__ f4 ks_swap8(const f4 v) {
+  f4 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    r[q] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[q]), 0x128, 0xf, 0xf, false));
+  return r;
+}
+
+// this wavefront's 16 RB x 32 part of column tile c
+template <class S, int RB, int NKS, int PAR>
 __device__ __forceinline__ void ks_tile(const unsigned short* __restrict__ As, const KsTask& T, float* y,
                                         const float* __restrict__ bias, float alpha, bool vst, int c, int wq,
                                         int lane, int fr, int fg, u4v (&b0)[3][2], u4v (&b1)[3][2]) {
+  const bool has_bias = T.bias_off >= 0;
   // the bias of this lane's 8 columns, loaded before the MFMAs: a load
   // waited for in the stores would wait for the B fragments loaded after it
   f4 bv[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) bv[j] = f4{0.f, 0.f, 0.f, 0.f};
-  if (T.bias_off >= 0) {
+  if (has_bias) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) bv[j][q] = bias[T.bias_off + min(c + 32 * wq + 16 * j + 4 * fg + q, T.ce - 1)];
   }
-  constexpr int RB = R / 16;
   f4 acc[RB][2];
   if (T.addend) {
     const bool avec = ((T.n & 3) == 0) && ((T.out_base & 3) == 0) && ((((uintptr_t)T.addend) & 15) == 0);
@@ -971,7 +990,7 @@ __device__ __forceinline__ void ks_tile(const unsigned short* __restrict__ As, c
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   }
-  ks_steps<R, KM, NKS, PAR, 0>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
+  ks_steps<S, RB, NKS, PAR, 0>(As, T, c, wq, lane, fr, fg, acc, b0, b1);
   // acc[i][j][q] = out[row 16 i + fr][column c + 32 wq + 16 j + 4 fg + q].
   // Lanes fr and fr ^ 8 trade one block, so that a store writes 8 whole rows
   // of the 32 columns (128 contiguous bytes each) instead of 16 half rows:
@@ -980,57 +999,61 @@ __device__ __forceinline__ void ks_tile(const unsigned short* __restrict__ As, c
   const bool lo = fr < 8;
   const int jl = lo ? 0 : 1;   // this lane's 16-column half, in both stores
   const int col = c + 32 * wq + 16 * jl + 4 * fg;
+  // whole 32 columns, 16-byte stores: no test but the row's, one 32-bit lane offset
+  const bool whole = vst && c + 32 * wq + 32 <= T.ce;
+  const unsigned off = (unsigned)(fr & 7) * (unsigned)T.n + (unsigned)col;
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
-    const f4 v0 = alpha * (acc[i][0] + bv[0]), v1 = alpha * (acc[i][1] + bv[1]);
-    const f4 give = lo ? v1 : v0;
-    f4 got;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) got[q] = __shfl_xor(give[q], 8);
+    f4 v0 = acc[i][0], v1 = acc[i][1];
+    if (has_bias) {
+      v0 += bv[0];
+      v1 += bv[1];
+    }
+    v0 *= alpha;
+    v1 *= alpha;
+    const f4 got = ks_swap8(lo ? v1 : v0);
     const f4 s0 = lo ? v0 : got, s1 = lo ? got : v1;   // rows 16 i + (fr & 7), + 8
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int r = 16 * i + 8 * h + (fr & 7);
-      if (r >= T.rows || col >= T.ce) continue;
       const f4 v = h ? s1 : s0;
-      float* dst = y + T.out_base + (int64_t)r * T.n + col;
-      if (vst) {
-        *(f4*)dst = v;
-      } else {
+      float* yr = y + T.out_base + (int64_t)(16 * i + 8 * h) * T.n;
+      if (whole) {
+        if (r < T.rows) *(f4*)(yr + off) = v;
+      } else if (r < T.rows && col < T.ce) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (col + q < T.ce) dst[q] = v[q];
+          if (col + q < T.ce) yr[off + q] = v[q];
       }
     }
   }
 }
 
-template <int R, int KM, int NKS>
+template <class S, int RB, int NKS>
 __device__ __forceinline__ void ks_columns(const unsigned short* __restrict__ As, const KsTask& T,
                                            float* y, const float* __restrict__ bias, float alpha, int grp,
                                            int wq, int lane, int fr, int fg) {
   int c0 = T.cb + 128 * grp;
   if (c0 >= T.ce) return;
   // 16-byte stores when every 4-column group of every row is 16-byte aligned
-  // (ce and cb are then multiples of 4 too)
-  const bool vst = ((T.n & 3) == 0) && ((T.out_base & 3) == 0) && ((((uintptr_t)y) & 15) == 0);
+  const bool vst = ((T.n & 3) == 0) && ((T.out_base & 3) == 0) && ((T.cb & 3) == 0) && ((((uintptr_t)y) & 15) == 0);
   u4v b0[3][2], b1[3][2];
   if (NKS > 0) ks_load_b(T, c0, 0, wq, lane, b0);
-  for (; c0 < T.ce; c0 += 2 * KS_CSTEP) {
-    ks_tile<R, KM, NKS, 0>(As, T, y, bias, alpha, vst, c0, wq, lane, fr, fg, b0, b1);
-    if (c0 + KS_CSTEP < T.ce)
-      ks_tile<R, KM, NKS, NKS & 1>(As, T, y, bias, alpha, vst, c0 + KS_CSTEP, wq, lane, fr, fg, b0, b1);
+  for (; c0 < T.ce; c0 += 2 * S::CSTEP) {
+    ks_tile<S, RB, NKS, 0>(As, T, y, bias, alpha, vst, c0, wq, lane, fr, fg, b0, b1);
+    if (c0 + S::CSTEP < T.ce)
+      ks_tile<S, RB, NKS, NKS & 1>(As, T, y, bias, alpha, vst, c0 + S::CSTEP, wq, lane, fr, fg, b0, b1);
   }
 }
 
-template <int R, int KM>
-__global__ __launch_bounds__(KS_THREADS) void k_seg_linear_ks(const float* __restrict__ x, float* y,
+template <class S>
+__global__ __launch_bounds__(S::THREADS, S::WAVES) void k_seg_linear_ks(const float* __restrict__ x, float* y,
                                                        const float* addend,
                                                        const unsigned short* __restrict__ wfrag,
                                                        const float* __restrict__ bias,
                                                        const int64_t* __restrict__ tasks, float alpha, int n_tasks,
                                                        int per) {
-  typedef KsShape<R, KM> S;
+  constexpr int R = S::R, KM = S::KM;
   __shared__ __attribute__((aligned(16))) unsigned short As[3 * S::PL];
   const int task = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (task >= n_tasks) return;
@@ -1049,13 +1072,13 @@ __global__ __launch_bounds__(KS_THREADS) void k_seg_linear_ks(const float* __res
   T.addend = addend;
   T.nks = (k + 31) >> 5;
   T.nb16 = (T.n + 15) >> 4;
-  const int t = (int)threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = (int)threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int grp = wv >> 2, wq = wv & 3;
   const int fr = lane & 15, fg = lane >> 4;
   if (k < 0 || k > KM) {
     // outside this instantiation's k range: NaN outputs instead of a product
     // of a truncated A tile (the host table builder never makes such tasks)
-    for (int u = t; u < T.rows * (T.ce - T.cb); u += KS_THREADS) {
+    for (int u = t; u < T.rows * (T.ce - T.cb); u += S::THREADS) {
       const int r = u / (T.ce - T.cb), c = T.cb + (u - r * (T.ce - T.cb));
       y[T.out_base + (int64_t)r * T.n + c] = __builtin_nanf("");
     }
@@ -1068,22 +1091,50 @@ __global__ __launch_bounds__(KS_THREADS) void k_seg_linear_ks(const float* __res
     const float* __restrict__ xa = x + x_base;
     const bool xvec = ((((uintptr_t)xa) & 15) == 0) && ((k & 3) == 0);
     const int kq = T.nks * 4;   // 8-k units per row
-    for (int u = t; u < R * kq; u += KS_THREADS) {
-      const int r = u / kq, kk = (u - r * kq) * 8;
-      const bool ok = r < T.rows;
-      const float* p = xa + (int64_t)r * k + kk;
-      const f4 a0 = seg_ld4(p, ok && xvec && kk + 4 <= k, ok && kk < k, k - kk);
-      const f4 a1 = seg_ld4(p + 4, ok && xvec && kk + 8 <= k, ok && kk + 4 < k, k - kk - 4);
+    constexpr int NU = R * KM / 8 / S::THREADS;   // units per thread at most
+    auto put = [&](int r, int kk, const f4& a0, const f4& a1) {
       const float v[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
       bx3_bf8 tt[3];
       bx3_split8(v, tt);
 #pragma unroll
       for (int pl = 0; pl < 3; ++pl) *(bx3_bf8*)&As[pl * S::PL + r * S::STR + kk] = tt[pl];
+    };
+    if (xvec && (k & 7) == 0 && k > 0) {
+      // every load in flight before the first split: unconditional, the row
+      // clamped to the last one (its outputs are not stored) and the 8-k unit
+      // into the row (zeros past k: an infinity there would meet zero weights)
+      f4 a[NU][2];
+#pragma unroll
+      for (int i = 0; i < NU; ++i) {
+        const int u = min(t + S::THREADS * i, R * kq - 1), r = u / kq, kk = (u - r * kq) * 8;
+        const float* p = xa + (int64_t)min(r, T.rows - 1) * k + min(kk, k - 8);
+        a[i][0] = *(const f4*)p;
+        a[i][1] = *(const f4*)(p + 4);
+      }
+#pragma unroll
+      for (int i = 0; i < NU; ++i) {
+        const int u = t + S::THREADS * i, r = u / kq, kk = (u - r * kq) * 8;
+        if (u >= R * kq) continue;
+        if (kk >= k) a[i][0] = a[i][1] = f4{0.f, 0.f, 0.f, 0.f};
+        put(r, kk, a[i][0], a[i][1]);
+      }
+    } else {
+      for (int u = t; u < R * kq; u += S::THREADS) {
+        const int r = u / kq, kk = (u - r * kq) * 8;
+        const bool ok = r < T.rows;
+        const float* p = xa + (int64_t)r * k + kk;
+        put(r, kk, seg_ld4(p, ok && xvec && kk + 4 <= k, ok && kk < k, k - kk),
+            seg_ld4(p + 4, ok && xvec && kk + 8 <= k, ok && kk + 4 < k, k - kk - 4));
+      }
     }
   }
   __syncthreads();
 
-#define KS_C(n) ks_columns<R, KM, (n) <= KM / 32 ? (n) : 0>(As, T, y, bias, alpha, grp, wq, lane, fr, fg)
+#define KS_C(n)                                                                                                       \
+  do {                                                                                                                \
+    if (T.rows > 32) ks_columns<S, S::RB, (n) <= KM / 32 ? (n) : 0>(As, T, y, bias, alpha, grp, wq, lane, fr, fg);     \
+    else ks_columns<S, 2, (n) <= KM / 32 ? (n) : 0>(As, T, y, bias, alpha, grp, wq, lane, fr, fg);                     \
+  } while (0)
   switch (T.nks) {
     case 1: KS_C(1); break;
     case 2: KS_C(2); break;
@@ -1093,7 +1144,7 @@ __global__ __launch_bounds__(KS_THREADS) void k_seg_linear_ks(const float* __res
     case 6: KS_C(6); break;
     case 7: KS_C(7); break;
     case 8: KS_C(8); break;
-    default: ks_columns<R, KM, 0>(As, T, y, bias, alpha, grp, wq, lane, fr, fg); break;   // k = 0: bias or zeros
+    default: ks_columns<S, S::RB, 0>(As, T, y, bias, alpha, grp, wq, lane, fr, fg); break;   // k = 0: bias or zeros
   }
 #undef KS_C
 }
@@ -1321,14 +1372,20 @@ extern "C" int tace_gemm_bx3(const float* x, const uint16_t* w_frag, const float
   return tace_check_launch("tace_gemm_bx3");
 }
 
-extern "C" int32_t tace_seg_linear_ks_rows(int32_t k) { return k < 0 ? 0 : k <= 128 ? 128 : k <= 256 ? 64 : 0; }
+extern "C" int32_t tace_seg_linear_ks_rows(int32_t k) { return k >= 0 && k <= 256 ? 64 : 0; }
+
+template <class S>
+static void launch_ks(const float* x, float* y, const float* addend, const uint16_t* w_frag, const float* bias,
+                      const int64_t* tasks, double alpha, int64_t n_tasks, int per, void* stream) {
+  hipLaunchKernelGGL(k_seg_linear_ks<S>, dim3((unsigned)(8 * per)), dim3(S::THREADS), 0, (hipStream_t)stream, x, y,
+                     addend, (const unsigned short*)w_frag, bias, tasks, (float)alpha, (int)n_tasks, per);
+}
 
 extern "C" int tace_seg_linear_presplit_ks(const float* x, float* y, const float* addend, const uint16_t* w_frag,
                                            const float* bias,
-                                           const int64_t* tasks, int64_t n_tasks, int32_t task_rows, double alpha,
+                                           const int64_t* tasks, int64_t n_tasks, int32_t k_max, double alpha,
                                            void* stream) {
-  if (task_rows != 128 && task_rows != 64)
-    return tace_fail_msg("tace_seg_linear_presplit_ks: tasks of 128 rows (k <= 128) or 64 rows (k <= 256)");
+  if (k_max != 128 && k_max != 256) return tace_fail_msg("tace_seg_linear_presplit_ks: k_max 128 or 256");
   if (n_tasks < 0 || n_tasks > 0x7ffffff0) return tace_fail_msg("tace_seg_linear_presplit_ks: bad task count");
   if (n_tasks == 0) return 0;
   if (!x || !y || !w_frag || !tasks) return tace_fail_msg("tace_seg_linear_presplit_ks: null pointer");
@@ -1336,12 +1393,8 @@ extern "C" int tace_seg_linear_presplit_ks(const float* x, float* y, const float
   if ((((uintptr_t)w_frag) & 15) != 0)
     return tace_fail_msg("tace_seg_linear_presplit_ks: the fragment-order weights must be 16-byte aligned");
   const int per = (int)((n_tasks + 7) / 8);
-  if (task_rows == 128)
-    hipLaunchKernelGGL((k_seg_linear_ks<128, 128>), dim3((unsigned)(8 * per)), dim3(KS_THREADS), 0, (hipStream_t)stream,
-                       x, y, addend, (const unsigned short*)w_frag, bias, tasks, (float)alpha, (int)n_tasks, per);
-  else
-    hipLaunchKernelGGL((k_seg_linear_ks<64, 256>), dim3((unsigned)(8 * per)), dim3(KS_THREADS), 0, (hipStream_t)stream,
-                       x, y, addend, (const unsigned short*)w_frag, bias, tasks, (float)alpha, (int)n_tasks, per);
+  if (k_max == 128) launch_ks<KsShape<64, 128, 1>>(x, y, addend, w_frag, bias, tasks, alpha, n_tasks, per, stream);
+  else launch_ks<KsShape<64, 256, 2>>(x, y, addend, w_frag, bias, tasks, alpha, n_tasks, per, stream);
   return tace_check_launch("tace_seg_linear_presplit_ks");
 }
 

@@ -1879,8 +1879,10 @@ def radial_mlp_hidden(radial: torch.Tensor, mats: Sequence[torch.Tensor]) -> tor
 # contribution with k <= 256 (or none) go to tace_seg_linear_presplit_ks
 # (pre-split plans only; None: every tile to the tile kernel)
 SEG_KS_MIN_N = 256
-# columns per tace_seg_linear_presplit_ks task
-SEG_KS_CHUNK = 1024
+# columns per tace_seg_linear_presplit_ks task of k <= 128 (one group of
+# wavefronts: 512 fill the GPU sooner, 200 rows 44 -> 34 us, and cost nothing
+# at 5,184) and of k <= 256 (two groups: 512 cost 8% at 3,000 rows of 89 species)
+SEG_KS_CHUNK = {128: 512, 256: 1024}
 # pre-split plans' tiles read the weights in fragment order
 # (tace_seg_linear_presplit_frag) when every instruction has a
 # fragment-order block; False: the planes of tace_seg_linear_presplit
@@ -2097,28 +2099,25 @@ class SegLinearPlan:
                     raise ValueError("seg linear plan: fragment-order weights of a task out of range")
             self.flops += int(2 * (k_t[:, 1] * (k_t[:, 4] - k_t[:, 3]) * k_t[:, 7]).sum())
         self.n_ks = len(k_t)
-        # one launch per task height (128 rows: k <= 128, 64 rows: k <= 256)
+        # one launch per kernel: tasks of k <= 128, of k <= 256
         self.ks_groups = []
-        if len(k_t):
-            by_k = {int(k): self._ks_rows(int(k)) for k in np.unique(k_t[:, 7])}
-            hts = np.array([by_k[int(k)] for k in k_t[:, 7]], dtype=np.int64)
-            for R in (128, 64):
-                sel = k_t[hts == R]
-                if len(sel):
-                    if (sel[:, 1] > R).any():
-                        raise ValueError("seg linear plan: a task is taller than its kernel's tile")
-                    if (sel[:, 7] > (128 if R == 128 else 256)).any():
-                        raise ValueError("seg linear plan: a task's k exceeds its kernel's limit")
-                    if len(sel) >= SEG_BALANCE_MIN:
-                        # a task costs its columns' 32-k steps and about two for their stores
-                        cost = (sel[:, 4] - sel[:, 3]) * ((sel[:, 7] + 31) // 32 + 2)
-                        sel = _xcd_balanced(sel, cost, cost)
-                    self.ks_groups.append((R, len(sel), torch.from_numpy(np.ascontiguousarray(sel)).to(device)))
+        for k_max in (128, 256) if len(k_t) else ():
+            sel = k_t[(k_t[:, 7] <= k_max) & ((k_t[:, 7] > 128) == (k_max > 128))]
+            if not len(sel):
+                continue
+            R = self._ks_rows(k_max)
+            if (sel[:, 1] > R).any():
+                raise ValueError("seg linear plan: a task is taller than its kernel's tile")
+            if len(sel) >= SEG_BALANCE_MIN:
+                # a task costs its columns' 32-k steps and about two for their stores
+                cost = (sel[:, 4] - sel[:, 3]) * ((sel[:, 7] + 31) // 32 + 2)
+                sel = _xcd_balanced(sel, cost, cost)
+            self.ks_groups.append((k_max, len(sel), torch.from_numpy(np.ascontiguousarray(sel)).to(device)))
 
     @staticmethod
     def _ks_rows(k: int) -> int:
         """Task height of ``tace_seg_linear_presplit_ks`` for contributions of
-        width k (k = 0: a block without contribution, 128 rows)."""
+        width k (k = 0: a block without contribution)."""
         R = N.lib().tace_seg_linear_ks_rows(int(k))
         if R <= 0:
             raise ValueError(f"seg linear plan: no short-k task kernel for k = {k}")
@@ -2138,18 +2137,19 @@ class SegLinearPlan:
         """Tasks of one output block (one contribution with k <= 128, or
         none): column chunk-major, so that the workgroups running at one time
         on an XCD share a chunk's weight columns in its L2."""
-        R = self._ks_rows(mine[0][2] if mine else 0)   # the task height for this k
+        k = mine[0][2] if mine else 0
+        R, chunk = self._ks_rows(k), SEG_KS_CHUNK[128 if k <= 128 else 256]
         r0, rows, sp = self._row_tiles(rng, d, R)
-        cb = np.arange(0, n, SEG_KS_CHUNK, dtype=np.int64)
+        cb = np.arange(0, n, chunk, dtype=np.int64)
         t = np.zeros((len(cb), len(r0), 10), dtype=np.int64)
         t[:, :, 0] = Z * s_o + r0 * n
         t[:, :, 1] = rows
         t[:, :, 2] = n
         t[:, :, 3] = cb[:, None]
-        t[:, :, 4] = np.minimum(n, cb + SEG_KS_CHUNK)[:, None]
+        t[:, :, 4] = np.minimum(n, cb + chunk)[:, None]
         t[:, :, 5] = -1 if boff is None else boff + sp * b_stride
         if mine:
-            s_i, k, f_off = mine[0][1], mine[0][2], mine[0][6]
+            s_i, f_off = mine[0][1], mine[0][6]
             t[:, :, 6] = Z * s_i + r0 * k
             t[:, :, 7] = k
             t[:, :, 8] = f_off + sp * f_stride
@@ -2274,9 +2274,9 @@ def seg_linear_presplit(x: torch.Tensor, y: torch.Tensor, planes: Optional[torch
                                                  plan.tiles.data_ptr(), plan.n_tiles, plan.contribs.data_ptr(),
                                                  float(alpha), st), "tace_seg_linear_presplit")
     if plan.n_ks:
-        for R, n_t, tasks in plan.ks_groups:
+        for k_max, n_t, tasks in plan.ks_groups:
             N.check(N.lib().tace_seg_linear_presplit_ks(x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr,
-                                                        tasks.data_ptr(), n_t, R, float(alpha), st),
+                                                        tasks.data_ptr(), n_t, k_max, float(alpha), st),
                     "tace_seg_linear_presplit_ks")
     _t1(tok, (plan.x_numel, plan.y_numel, plan.w_numel, plan.flops))
     return y

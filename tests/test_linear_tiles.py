@@ -122,3 +122,45 @@ def test_stacked_values_of_structures():
                                      ([1.0], np.float64, (3, 3), cell), ([np.ones((3, 1))], np.int32, (3,), flag)):
         with pytest.raises(ValueError):
             ops._stacked(items, dtype, shape, one)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [5, 12, 32, 40, 96, 128, 130, 232, 256])
+def test_short_k_tasks_equal_the_tile_kernel(cuda, k, monkeypatch):
+    """Wide blocks of one contribution: tasks of 1 .. 64 rows (32 and fewer
+    multiply half a tile), k around the 32-k steps and off the 8-k loads,
+    column chunks with a remainder off the 32 columns: the bits of the kernel
+    that keeps whole tiles, with a bias, and with an addend up to rounding.
+    An infinity in one row stays in that row."""
+    from tace_amd import model as pm
+    counts = [1, 31, 32, 33, 0, 64, 65, 97, 150] * 4
+    S, Z = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(k)
+    lin = pm.e3nnElementLinear(f"{k}x0e+{k}x1o", "1093x0e+300x1o", S)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn(lin.weight.shape, generator=g))
+        lin.bias.copy_(torch.randn(lin.bias.shape, generator=g))
+    lin = lin.to(cuda).requires_grad_(False)
+    species = torch.repeat_interleave(torch.arange(S), torch.tensor(counts))
+    sp = pm.SpeciesPlan(torch.nn.functional.one_hot(species, S).float().to(cuda))
+    x = torch.randn(Z, lin.lay.dim_in, generator=g).to(cuda)
+    add = torch.randn(Z, lin.lay.dim_out, generator=g).to(cuda)
+    x.view(-1)[3 * k + 1] = float("inf")   # node 3 of the first block
+    rr, seg = pm._linear_route(x, lin.weight, lin.lay, sp.ranges)
+    assert seg
+    res = []
+    for min_n in (None, 256):
+        monkeypatch.setattr(ops, "SEG_KS_MIN_N", min_n)
+        lin.lay._seg.clear()
+        plan = lin.lay.seg_plan("fwd", rr, Z, x, lin.weight, lin.bias)
+        assert (plan.n_ks > 0) == (min_n is not None)
+        y = pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.5)
+        z = pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.5, out=add.clone(), addend=add)
+        res.append((y, z))
+    (y0, z0), (y1, z1) = res
+    bad = ~torch.isfinite(y0)
+    assert int(bad.sum()) == 1093 and torch.equal(bad, ~torch.isfinite(y1)) and torch.equal(bad, ~torch.isfinite(z1))
+    y0, y1, z0, z1 = (v[~bad] for v in (y0, y1, z0, z1))
+    assert torch.equal(y0, y1)
+    # sums started from the addend or ended with it: a rounding each of sums of k <= 256 products
+    assert ((z1 - z0).abs().max() / z0.abs().max()).item() < 2e-6
