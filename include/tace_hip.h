@@ -240,17 +240,20 @@ int tace_radial_mlp_bwd(int dtype, const void* radial, const void* g_h, int64_t 
  *   tace_radial_mlp_out_bwd_f32: its input gradient (the backward of the
  *   last Linear of mlp.py:136-191), g_h [E, 64] = alpha g_out [E, n_out] @
  *   weight^T, the same way (g_out and weight 16-byte aligned when n_out is a
- *   multiple of 4; weights are constants: no weight gradient). */
+ *   multiple of 4; weights are constants: no weight gradient).  splits > 1
+ *   (none of them empty in whole 32-column slabs) spreads n_out over that many
+ *   workgroups per 128 rows through parts [splits, rows, 64], added in order
+ *   (g_h and parts 16-byte aligned); 1 leaves parts unread. */
 int tace_radial_mlp_out_f32(const float* h, const float* weight, int64_t n_edges, int32_t n_out, float alpha,
                             float* out, void* stream);
 int tace_radial_mlp_out_bwd_f32(const float* g_out, const float* weight, int64_t n_edges, int32_t n_out, float alpha,
-                                float* g_h, void* stream);
+                                float* g_h, int32_t splits, float* parts, void* stream);
 /* the same for weight rows shared by edge pairs: g_h [n_rows, 64] = alpha
  * (g_out[rows_a[r]] + g_out[rows_b[r]]) @ weight^T, the sum in float32
  * (rows_b[r] < 0: g_out[rows_a[r]] alone); g_out [E, n_out] per edge. */
 int tace_radial_mlp_out_bwd_pairs_f32(const float* g_out, const int32_t* rows_a, const int32_t* rows_b,
                                       int64_t n_rows, int32_t n_out, float alpha, const float* weight, float* g_h,
-                                      void* stream);
+                                      int32_t splits, float* parts, void* stream);
 
 /* ---- per-species (element) linears
  * tace_seg_linear replaces the per-element o3.Linear of e3nnElementLinear

@@ -40,7 +40,8 @@ _SIGS = {
     "tace_edge_tp_bwd_rows": (_c_int, [_c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64,
                                        _c_i32, _c_i32, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp]),
     "tace_edge_pairs": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp, _vp, _vp]),
-    "tace_radial_mlp_out_bwd_pairs_f32": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, ctypes.c_float, _vp, _vp, _vp]),
+    "tace_radial_mlp_out_bwd_pairs_f32": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, ctypes.c_float, _vp, _vp, _c_i32,
+                                                   _vp, _vp]),
     "tace_edge_tp_bwd_noalloc": (_c_int, [_c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64,
                                           _c_i32, _c_i32, _vp, _vp, _vp, _vp, _vp, _vp]),
     "tace_edge_rtp_fwd": (_c_int, [_c_int, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _c_i64, _c_i64,
@@ -81,7 +82,7 @@ _SIGS = {
     "tace_radial_mlp_fwd": (_c_int, [_c_int, _vp, _c_i64, _c_i32, _c_i32, _vp, _vp, _vp]),
     "tace_radial_mlp_bwd": (_c_int, [_c_int, _vp, _vp, _c_i64, _c_i32, _c_i32, _vp, _vp, _vp]),
     "tace_radial_mlp_out_f32": (_c_int, [_vp, _vp, _c_i64, _c_i32, ctypes.c_float, _vp, _vp]),
-    "tace_radial_mlp_out_bwd_f32": (_c_int, [_vp, _vp, _c_i64, _c_i32, ctypes.c_float, _vp, _vp]),
+    "tace_radial_mlp_out_bwd_f32": (_c_int, [_vp, _vp, _c_i64, _c_i32, ctypes.c_float, _vp, _c_i32, _vp, _vp]),
     "tace_seg_linear": (_c_int, [_c_int, _c_i32, _c_i32, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_dbl, _vp]),
     "tace_bf16x3_split_blocks": (_c_int, [_vp, _vp, _vp, _c_i64, _vp, _c_i64, _vp]),
     "tace_seg_linear_presplit": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _vp, _c_dbl, _vp]),

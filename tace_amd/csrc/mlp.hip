@@ -430,7 +430,13 @@ __global__ __launch_bounds__(256) void k_mlp_out_f32(const float* __restrict__ h
 // L2) once into three bf16 planes in LDS, from which lane (i, q) reads
 // W[32 cb + i][same k] -- step s item j of both operands is k = k0 + 16 q +
 // 8 s + j.  The next slab's loads are issued before the current slab's
-// MFMAs.  Read-bound on g.
+// MFMAs.  Read-bound on g with enough wavefronts in flight; a launch of few
+// rows has too few, each going through all of N one slab's latency at a time,
+// so there N is spread over gridDim.y workgroups (n_per columns each) that
+// write their sums apart (k_mlp_out_bwd_sum adds them in order).  At N = 2,944
+// with pairs: 500 rows 137 -> 20 us, 12,000 164 -> 64, 23,031 173 -> 129 (543
+// MB), 40,000 252 -> 209; from 130,000 rows on parts only add traffic (577 ->
+// 611).
 __device__ __forceinline__ void mlp_ld16(const float* __restrict__ row, int k, int N, bool ok, bool vec, float* v) {
   if (ok && vec && k + 16 <= N) {
     const f4_t* p = reinterpret_cast<const f4_t*>(row + k);
@@ -466,7 +472,8 @@ __device__ __forceinline__ void mlp_ld8(const float* __restrict__ row, int k, in
 template <bool PAIRS>
 __global__ __launch_bounds__(256) void k_mlp_out_bwd_f32(const float* __restrict__ g, const float* __restrict__ Wm,
                                                          int64_t E, int N, float alpha, float* __restrict__ gh,
-                                                         const int* __restrict__ ra, const int* __restrict__ rb) {
+                                                         const int* __restrict__ ra, const int* __restrict__ rb,
+                                                         int n_per) {
   constexpr int BSTR = 40;                       // bf16 per LDS row: 32 k + 8 pad (80 bytes)
   __shared__ __attribute__((aligned(16))) unsigned short Bp[3 * 64 * BSTR];   // term p, column c, k
   const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -487,10 +494,12 @@ __global__ __launch_bounds__(256) void k_mlp_out_bwd_f32(const float* __restrict
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[cb][r] = 0.0f;
   float a[16], w[8], a2[16];
-  mlp_ld16(grow, 16 * q, N, rok, vec, a);
-  if (PAIRS) mlp_ld16(grow2, 16 * q, N, rbe >= 0, vec, a2);
-  mlp_ld8(wrow, wk, N, vec, w);
-  for (int k0 = 0; k0 < N; k0 += 32) {
+  const int kb = (int)blockIdx.y * n_per, ke = min(N, kb + n_per);
+  gh += (int64_t)blockIdx.y * E * 64;
+  mlp_ld16(grow, kb + 16 * q, N, rok, vec, a);
+  if (PAIRS) mlp_ld16(grow2, kb + 16 * q, N, rbe >= 0, vec, a2);
+  mlp_ld8(wrow, kb + wk, N, vec, w);
+  for (int k0 = kb; k0 < ke; k0 += 32) {
     bx3_bf8 wt[3];
     bx3_split8(w, wt);
 #pragma unroll
@@ -503,7 +512,7 @@ __global__ __launch_bounds__(256) void k_mlp_out_bwd_f32(const float* __restrict
 #pragma unroll
     for (int s = 0; s < 2; ++s) bx3_split8(a + 8 * s, at[s]);
     __syncthreads();
-    if (k0 + 32 < N) {   // next slab in flight during this slab's MFMAs
+    if (k0 + 32 < ke) {   // next slab in flight during this slab's MFMAs
       mlp_ld16(grow, k0 + 32 + 16 * q, N, rok, vec, a);
       if (PAIRS) mlp_ld16(grow2, k0 + 32 + 16 * q, N, rbe >= 0, vec, a2);
       mlp_ld8(wrow, k0 + 32 + wk, N, vec, w);
@@ -529,6 +538,16 @@ __global__ __launch_bounds__(256) void k_mlp_out_bwd_f32(const float* __restrict
       const int64_t row = e0 + 8 * (r >> 2) + 4 * q + (r & 3);
       if (row < E) gh[row * 64 + 32 * cb + i] = alpha * acc[cb][r];
     }
+}
+
+// g_h = the sum of its n_per-wide parts of N, in order (n4 = 16 E float4)
+__global__ __launch_bounds__(256) void k_mlp_out_bwd_sum(const f4_t* __restrict__ parts, int splits, int64_t n4,
+                                                         f4_t* __restrict__ gh) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f4_t s = parts[i];
+  for (int p = 1; p < splits; ++p) s += parts[p * n4 + i];
+  gh[i] = s;
 }
 
 size_t mlp_lds_bytes(int n_in, int n_layers) {
@@ -629,12 +648,21 @@ int tace_radial_mlp_out_f32(const float* h, const float* weight, int64_t n_edges
   if (n_edges == 0) return 0;
   if (!h || !weight || !out) return tace_fail_msg("tace_radial_mlp_out_f32: null pointer");
   if (((uintptr_t)h & 15) != 0) return tace_fail_msg("tace_radial_mlp_out_f32: h must be 16-byte aligned");
-  // 1,024 edges per chunk, fewer (down to 128) when that leaves fewer than
-  // 2,048 workgroups: small systems still fill the GPU
+  // Two workgroups (eight wavefronts of 252 registers) run on a CU, 64 on an
+  // XCD, and each first reads and splits its 64 columns of W per wavefront, as
+  // long as four blocks of edges take.  So a chunk is as long as lets the
+  // workgroups of an XCD (n_col_tiles per chunk) fill its 64 places once, or
+  // the fewest times that keep it at 1,024 edges or fewer: at 2,944 columns
+  // 23,031 edges 96 -> 77 us, 40,000 157 -> 136; at 512 columns 70,000 edges
+  // 50 -> 41; 500 edges 14 -> 9.5 (all against halving 1,024 until 2,048
+  // workgroups, down to 128).
   const int n_col_tiles = (n_out + 255) / 256;
-  int edges_per_chunk = 1024;
-  while (edges_per_chunk > 128 && n_col_tiles * ((n_edges + edges_per_chunk - 1) / edges_per_chunk) < 2048)
-    edges_per_chunk >>= 1;
+  int64_t epc = 2048;
+  for (int64_t rounds = 1; epc > 1024; ++rounds) {
+    const int64_t per_xcd = 64 * rounds / n_col_tiles;   // chunks
+    if (per_xcd > 0) epc = 32 * ((n_edges + 256 * per_xcd - 1) / (256 * per_xcd));
+  }
+  const int edges_per_chunk = (int)epc;
   const int64_t n_chunks = (n_edges + edges_per_chunk - 1) / edges_per_chunk;
   const int64_t n_wg = n_col_tiles * ((n_chunks + 7) / 8) * 8;
   if (n_wg > INT32_MAX) return tace_fail_msg("tace_radial_mlp_out_f32: too many edges");
@@ -643,34 +671,51 @@ int tace_radial_mlp_out_f32(const float* h, const float* weight, int64_t n_edges
   return tace_check_launch("tace_radial_mlp_out_f32");
 }
 
+// the launches of both forms of the last layer's input gradient
+static int mlp_out_bwd(const char* who, const float* g_out, const int32_t* rows_a, const int32_t* rows_b, bool pairs,
+                       const float* weight, int64_t n_rows, int32_t n_out, float alpha, float* g_h, int32_t splits,
+                       float* parts, void* stream) {
+  char msg[128];
+  const char* bad = nullptr;
+  const int64_t n_wg = (n_rows + 127) / 128;
+  const int32_t n_per = splits > 0 ? 32 * ((n_out + 32 * splits - 1) / (32 * splits)) : 0;   // whole 32-wide slabs
+  if (n_rows < 0 || n_out <= 0) bad = "bad sizes";
+  else if (splits < 1 || splits > 64 || (int64_t)(splits - 1) * n_per >= n_out) bad = "bad number of parts";
+  else if (n_rows == 0) return 0;
+  else if (!g_out || !weight || !g_h || (splits > 1 && !parts) || (pairs && (!rows_a || !rows_b))) bad = "null pointer";
+  else if ((n_out & 3) == 0 && ((((uintptr_t)g_out) | ((uintptr_t)weight)) & 15) != 0)
+    bad = "g_out and weight must be 16-byte aligned";
+  else if (splits > 1 && ((((uintptr_t)g_h) | ((uintptr_t)parts)) & 15) != 0) bad = "g_h must be 16-byte aligned";
+  else if (n_wg > INT32_MAX) bad = "too many rows";
+  if (bad) {
+    snprintf(msg, sizeof(msg), "%s: %s", who, bad);
+    return tace_fail_msg(msg);
+  }
+  float* const o = splits > 1 ? parts : g_h;
+  const dim3 g((unsigned)n_wg, (unsigned)splits), b(256);
+  if (pairs)
+    hipLaunchKernelGGL(k_mlp_out_bwd_f32<true>, g, b, 0, (hipStream_t)stream, g_out, weight, n_rows, n_out, alpha, o,
+                       (const int*)rows_a, (const int*)rows_b, n_per);
+  else
+    hipLaunchKernelGGL(k_mlp_out_bwd_f32<false>, g, b, 0, (hipStream_t)stream, g_out, weight, n_rows, n_out, alpha, o,
+                       nullptr, nullptr, n_per);
+  if (splits > 1)
+    hipLaunchKernelGGL(k_mlp_out_bwd_sum, dim3((unsigned)((16 * n_rows + 255) / 256)), b, 0, (hipStream_t)stream,
+                       (const f4_t*)parts, splits, 16 * n_rows, (f4_t*)g_h);
+  return tace_check_launch(who);
+}
+
 int tace_radial_mlp_out_bwd_f32(const float* g_out, const float* weight, int64_t n_edges, int32_t n_out, float alpha,
-                                float* g_h, void* stream) {
-  if (n_edges < 0 || n_out <= 0) return tace_fail_msg("tace_radial_mlp_out_bwd_f32: bad sizes");
-  if (n_edges == 0) return 0;
-  if (!g_out || !weight || !g_h) return tace_fail_msg("tace_radial_mlp_out_bwd_f32: null pointer");
-  if ((n_out & 3) == 0 && ((((uintptr_t)g_out) | ((uintptr_t)weight)) & 15) != 0)
-    return tace_fail_msg("tace_radial_mlp_out_bwd_f32: g_out and weight must be 16-byte aligned");
-  const int64_t n_wg = (n_edges + 127) / 128;
-  if (n_wg > INT32_MAX) return tace_fail_msg("tace_radial_mlp_out_bwd_f32: too many edges");
-  hipLaunchKernelGGL(k_mlp_out_bwd_f32<false>, dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, g_out,
-                     weight, n_edges, n_out, alpha, g_h, nullptr, nullptr);
-  return tace_check_launch("tace_radial_mlp_out_bwd_f32");
+                                float* g_h, int32_t splits, float* parts, void* stream) {
+  return mlp_out_bwd("tace_radial_mlp_out_bwd_f32", g_out, nullptr, nullptr, false, weight, n_edges, n_out, alpha, g_h,
+                     splits, parts, stream);
 }
 
 int tace_radial_mlp_out_bwd_pairs_f32(const float* g_out, const int32_t* rows_a, const int32_t* rows_b,
                                       int64_t n_rows, int32_t n_out, float alpha, const float* weight, float* g_h,
-                                      void* stream) {
-  if (n_rows < 0 || n_out <= 0) return tace_fail_msg("tace_radial_mlp_out_bwd_pairs_f32: bad sizes");
-  if (n_rows == 0) return 0;
-  if (!g_out || !rows_a || !rows_b || !weight || !g_h)
-    return tace_fail_msg("tace_radial_mlp_out_bwd_pairs_f32: null pointer");
-  if ((n_out & 3) == 0 && ((((uintptr_t)g_out) | ((uintptr_t)weight)) & 15) != 0)
-    return tace_fail_msg("tace_radial_mlp_out_bwd_pairs_f32: g_out and weight must be 16-byte aligned");
-  const int64_t n_wg = (n_rows + 127) / 128;
-  if (n_wg > INT32_MAX) return tace_fail_msg("tace_radial_mlp_out_bwd_pairs_f32: too many rows");
-  hipLaunchKernelGGL(k_mlp_out_bwd_f32<true>, dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, g_out,
-                     weight, n_rows, n_out, alpha, g_h, (const int*)rows_a, (const int*)rows_b);
-  return tace_check_launch("tace_radial_mlp_out_bwd_pairs_f32");
+                                      int32_t splits, float* parts, void* stream) {
+  return mlp_out_bwd("tace_radial_mlp_out_bwd_pairs_f32", g_out, rows_a, rows_b, true, weight, n_rows, n_out, alpha,
+                     g_h, splits, parts, stream);
 }
 
 }  // extern "C"

@@ -1813,6 +1813,20 @@ def launch_mlp_out_f32(h, W, alpha: float) -> torch.Tensor:
     return out
 
 
+def _mlp_out_bwd_parts(rows: int, n: int, device):
+    """(parts, their buffer or None): over how many workgroups per 128 rows
+    the last layer's input gradient spreads its n columns.  At most the four
+    workgroups per CU that run together (23,031 rows of 2,944 columns: 76 us in
+    five parts, 88 in six), or two parts that nearly do; of at least eight
+    32-column slabs, or of 24 where there is a workgroup per CU already (70,000
+    rows: 2,944 columns in two parts 400 -> 361 us, 512 columns in two 68 -> 76)."""
+    wgs, slabs = max(1, (rows + 127) // 128), (n + 31) // 32
+    q = 1024 // wgs if wgs <= 512 else 1200 // wgs
+    q = max(1, min(q, slabs // (8 if wgs <= 256 else 24), 64))
+    q = -(-slabs // -(-slabs // q))   # none empty
+    return q, torch.empty(q, rows, 64, dtype=torch.float32, device=device) if q > 1 else None
+
+
 def launch_mlp_out_bwd_f32(g, W, alpha: float) -> torch.Tensor:
     """alpha g @ W^T (g [E, n_out], W [64, n_out]): the last layer's input
     gradient, in float32 on the bf16 MFMA (three-term split)."""
@@ -1821,7 +1835,9 @@ def launch_mlp_out_bwd_f32(g, W, alpha: float) -> torch.Tensor:
     _req(W, "weight", torch.float32, (64, n))
     gh = torch.empty(E, 64, dtype=torch.float32, device=g.device)
     tok = _t0("radial_mlp_out_bwd")
-    N.check(N.lib().tace_radial_mlp_out_bwd_f32(g.data_ptr(), W.data_ptr(), E, n, float(alpha), gh.data_ptr(),
+    q, parts = _mlp_out_bwd_parts(E, n, g.device)
+    N.check(N.lib().tace_radial_mlp_out_bwd_f32(g.data_ptr(), W.data_ptr(), E, n, float(alpha), gh.data_ptr(), q,
+                                                None if parts is None else parts.data_ptr(),
                                                 N.stream_ptr(g.device)), "tace_radial_mlp_out_bwd_f32")
     _t1(tok, (E, n))
     return gh
@@ -1835,10 +1851,12 @@ def launch_mlp_out_bwd_pairs_f32(g, pairs: EdgePairs, W, alpha: float) -> torch.
     _req(W, "weight", torch.float32, (64, n))
     gh = torch.empty(pairs.n_rows, 64, dtype=torch.float32, device=g.device)
     tok = _t0("radial_mlp_out_bwd")
+    q, parts = _mlp_out_bwd_parts(pairs.n_rows, n, g.device)
     N.check(N.lib().tace_radial_mlp_out_bwd_pairs_f32(g.data_ptr(), pairs.row_edges.data_ptr(),
                                                       pairs.row_partner.data_ptr(), pairs.n_rows, n, float(alpha),
-                                                      W.data_ptr(), gh.data_ptr(), N.stream_ptr(g.device)),
-            "tace_radial_mlp_out_bwd_pairs_f32")
+                                                      W.data_ptr(), gh.data_ptr(), q,
+                                                      None if parts is None else parts.data_ptr(),
+                                                      N.stream_ptr(g.device)), "tace_radial_mlp_out_bwd_pairs_f32")
     _t1(tok, (E, n))
     return gh
 

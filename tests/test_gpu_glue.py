@@ -219,3 +219,34 @@ def test_edge_index_of_csr(cuda, n, most):
     want = torch.repeat_interleave(torch.arange(n), counts)
     assert ei.dtype == torch.int64 and dst.dtype == torch.int32
     assert torch.equal(ei.cpu(), torch.stack([src.to(torch.int64), want])) and torch.equal(dst.cpu().to(torch.int64), want)
+
+
+@pytest.mark.parametrize("E,n", [(1, 5), (31, 260), (33, 768), (129, 2944), (1000, 36), (4097, 2944), (33000, 1000),
+                                 (140000, 256)])
+def test_last_radial_layer_parts(cuda, E, n):
+    """Last layer and its input gradient (of edges and of pair rows, some
+    alone): chunks and column parts of every length, remainders of 32 edges,
+    128 rows and 32 columns.  At most six products per 16 terms are added one
+    after another, each sum rounded once, and a part more."""
+    g = torch.Generator().manual_seed(E + n)
+    h, W, go = torch.randn(E, 64, generator=g), torch.randn(64, n, generator=g), torch.randn(E, n, generator=g)
+    hc, Wc, gc = h.to(cuda), W.to(cuda), go.to(cuda)
+    w64, u = W.double(), 2.0 ** -24
+    rows = torch.cat([torch.arange(0, E, max(1, E // 400)), torch.tensor([E - 1])])
+    got = ops.launch_mlp_out_f32(hc, Wc, 0.5).cpu()[rows].double()
+    bound = (6 * 64 / 16 + 8) * u * 0.5 * (h[rows].double().abs() @ w64.abs())
+    assert ((got - 0.5 * h[rows].double() @ w64).abs() <= bound).all()
+    q, parts = ops._mlp_out_bwd_parts(E, n, cuda)
+    assert (q == 1) == (parts is None) and (q - 1) * 32 * -(-((n + 31) // 32) // q) < n
+    tol = (6 * n / 16 + 8 + q) * u * 0.5
+    if n % 4 == 0:
+        got = ops.launch_mlp_out_bwd_f32(gc, Wc, 0.5).cpu()[rows].double()
+        assert ((got - 0.5 * go[rows].double() @ w64.t()).abs() <= tol * (go[rows].double().abs() @ w64.abs().t())).all()
+    ra = torch.randperm(E, generator=g).to(torch.int32)
+    rb = torch.where(torch.arange(E) % 7 == 0, -1, torch.randperm(E, generator=g)).to(torch.int32)
+    pairs = ops.EdgePairs(E, ra.to(cuda), ra.to(cuda), rb.to(cuda))
+    got = ops.launch_mlp_out_bwd_pairs_f32(gc, pairs, Wc, 0.5).cpu()[rows].double()
+    a, b = go[ra[rows].long()], go[rb[rows].clamp_min(0).long()] * (rb[rows] >= 0)[:, None]
+    s = a.double() + b.double()
+    mag = (a.double().abs() + b.double().abs()) @ w64.abs().t()
+    assert ((got - 0.5 * s @ w64.t()).abs() <= (tol + u) * mag).all()
