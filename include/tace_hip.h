@@ -232,6 +232,13 @@ int tace_edge_vec_bwd(int dtype, const void* g_vec, const int32_t* rowptr, const
 #define TACE_MLP_MAX_LAYERS 4
 int tace_radial_mlp_fwd(int dtype, const void* radial, int64_t n_edges, int32_t n_in, int32_t n_layers,
                         const void* weights, void* h, void* stream);
+/* tace_radial_mlp_fwd in float32 with layer l's weights read from weights[l]
+ * (host array of device pointers, [n_in | 64, 64] row-major) and multiplied by
+ * scales[l]; the products, back to back, are also written to flat [n_in + 64
+ * (n_layers - 1), 64]: the weights tace_radial_mlp_bwd takes. */
+int tace_radial_mlp_fwd_scaled(const float* radial, int64_t n_edges, int32_t n_in, int32_t n_layers,
+                               const float* const* weights, const double* scales, float* flat, float* h,
+                               void* stream);
 int tace_radial_mlp_bwd(int dtype, const void* radial, const void* g_h, int64_t n_edges, int32_t n_in,
                         int32_t n_layers, const void* weights, void* g_radial, void* stream);
 /* the last (linear) layer in float32: out [E, n_out] = alpha h [E, 64] @

@@ -105,6 +105,7 @@ _SIGS = {
     "tace_narrow_linear": (_c_int, [_c_int, _vp, _c_i64, _c_i32, _vp, _vp, _c_i32, _vp, _vp]),
     "tace_rows_accumulate_runs": (_c_int, [_c_int, _vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i32, _vp, _c_i64,
                                            _vp]),
+    "tace_radial_mlp_fwd_scaled": (_c_int, [_vp, _c_i64, _c_i32, _c_i32, _vp, _vp, _vp, _vp, _vp]),
     "tace_edge_index": (_c_int, [_vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp]),
     "tace_gemm_bx3": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i32, _c_i32, _vp]),
     "tace_layout_operands": (_c_int, [_vp, _c_i64, _vp, _vp]),

@@ -162,13 +162,53 @@ __host__ __device__ __forceinline__ int mlp_lds_weights(int n_in, int n_layers) 
   return (((n_in + 1) & ~1) + (n_layers - 1) * 64) * WSTR;
 }
 
-__device__ __forceinline__ void mlp_stage_weights(const float* __restrict__ wg, int n_in, int n_layers,
-                                                  float* __restrict__ smem) {
-  const int K0p = (n_in + 1) & ~1, rows = K0p + (n_layers - 1) * 64;
-  for (int t = (int)threadIdx.x; t < rows * 64; t += 256) {
-    const int r = t >> 6, j = t & 63;
-    smem[r * WSTR + j] = r < K0p ? (r < n_in ? wg[r * 64 + j] : 0.0f) : wg[(n_in + r - K0p) * 64 + j];
+// The hidden layers' weights: layer l's matrix w[l] (row-major, 64 columns)
+// and the factor it is multiplied with; vec: every w[l] on 16 bytes.
+struct MlpWeights {
+  const float* w[TACE_MLP_MAX_LAYERS];
+  float scale[TACE_MLP_MAX_LAYERS];
+  int vec;
+};
+
+// scaled weights of all layers -> LDS, layer 0 padded to an even number of
+// rows; flat (null: none) receives them back to back.  Every load goes out
+// before the first LDS write: one after the other, the 34 loads per thread of
+// three layers were most of a small launch (23,031 rows:
+// forward 26 -> 17 us, backward 39 -> 26).
+template <int NL>
+__device__ __forceinline__ void mlp_stage_weights(const MlpWeights& src, int n_in, float* __restrict__ smem,
+                                                  float* __restrict__ flat) {
+  typedef float f4s __attribute__((ext_vector_type(4)));
+  const int K0p = (n_in + 1) & ~1, t = (int)threadIdx.x;
+  if (!src.vec) {
+    for (int u = t; u < (K0p + (NL - 1) * 64) * 64; u += 256) {
+      const int r = u >> 6, j = u & 63, l = r < K0p ? 0 : 1 + ((r - K0p) >> 6), rl = l ? (r - K0p) & 63 : r;
+      const float v = r >= n_in && r < K0p ? 0.0f : src.w[l][rl * 64 + j] * src.scale[l];
+      smem[r * WSTR + j] = v;
+      if (flat && !(r >= n_in && r < K0p)) flat[(l ? n_in + r - K0p : r) * 64 + j] = v;
+    }
+    return;
   }
+  constexpr int N0 = 2, NU = N0 + 4 * (NL - 1);   // 4-column units per thread: layer 0 (n_in <= 32), 4 per later layer
+  f4s v[NU];
+#pragma unroll
+  for (int p = 0; p < NU; ++p) {
+    const int l = p < N0 ? 0 : 1 + (p - N0) / 4;
+    const int u = p < N0 ? min(t + 256 * p, 16 * n_in - 1) : t + 256 * ((p - N0) & 3);
+    v[p] = *(const f4s*)(src.w[l] + 4 * u);
+  }
+#pragma unroll
+  for (int p = 0; p < NU; ++p) {
+    const int l = p < N0 ? 0 : 1 + (p - N0) / 4;
+    const int u = p < N0 ? t + 256 * p : t + 256 * ((p - N0) & 3);
+    if (p < N0 && u >= 16 * n_in) continue;
+    const f4s x = v[p] * src.scale[l];
+    const int r = (u >> 4) + (l ? K0p + 64 * (l - 1) : 0), j = 4 * (u & 15);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) smem[r * WSTR + j + e] = x[e];
+    if (flat) *(f4s*)(flat + (l ? n_in + 64 * (l - 1) : 0) * 64 + 4 * u) = x;
+  }
+  if ((n_in & 1) && t < 64) smem[n_in * WSTR + t] = 0.0f;
 }
 
 // pre-activation z of layer `upto` of the 32-edge block at e0, in the
@@ -242,9 +282,10 @@ __device__ __forceinline__ void mlp_block_forward(const float* __restrict__ radi
 
 template <int NL>
 __global__ __launch_bounds__(256) void k_mlp_fwd_mfma(const float* __restrict__ radial, int64_t E, int n_in,
-                                                      const float* __restrict__ wg, float* __restrict__ h) {
+                                                      MlpWeights wg, float* __restrict__ flat,
+                                                      float* __restrict__ h) {
   extern __shared__ float smem[];
-  mlp_stage_weights(wg, n_in, NL, smem);
+  mlp_stage_weights<NL>(wg, n_in, smem, blockIdx.x == 0 ? flat : nullptr);
   __syncthreads();
   const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, i = lane & 31, q = lane >> 5;
   float* __restrict__ T = smem + mlp_lds_weights(n_in, NL) + wave * 32 * TSTRIDE;
@@ -270,10 +311,10 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_mfma(const float* __restrict__ 
 // is needed (one layer in registers, 2 wavefronts per SIMD) measured 0.90 ms.
 template <int NL>
 __global__ __launch_bounds__(256) void k_mlp_bwd_mfma(const float* __restrict__ radial, const float* __restrict__ gh,
-                                                      int64_t E, int n_in, const float* __restrict__ wg,
+                                                      int64_t E, int n_in, MlpWeights wg,
                                                       float* __restrict__ g_radial) {
   extern __shared__ float smem[];
-  mlp_stage_weights(wg, n_in, NL, smem);
+  mlp_stage_weights<NL>(wg, n_in, smem, nullptr);
   __syncthreads();
   const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, i = lane & 31, q = lane >> 5;
   const int K0p = (n_in + 1) & ~1;
@@ -568,6 +609,17 @@ int mlp_lds_attr(const void* fn, size_t bytes) {
   return 0;
 }
 
+// the layers of one contiguous buffer, scaled already
+MlpWeights mlp_flat(const float* w, int n_in, int n_layers) {
+  MlpWeights m;
+  for (int l = 0; l < TACE_MLP_MAX_LAYERS; ++l) {
+    m.w[l] = w + (l && l < n_layers ? (n_in + 64 * (l - 1)) * 64 : 0);
+    m.scale[l] = 1.0f;
+  }
+  m.vec = (((uintptr_t)w) & 15) == 0;
+  return m;
+}
+
 int mlp_checks(const char* who, int64_t E, int32_t n_in, int32_t n_layers) {
   char msg[160];
   if (E < 0 || n_in < 1 || n_in > TACE_MLP_MAX_IN || n_layers < 1 || n_layers > TACE_MLP_MAX_LAYERS) {
@@ -582,6 +634,21 @@ int mlp_checks(const char* who, int64_t E, int32_t n_in, int32_t n_layers) {
 
 extern "C" {
 
+static int mlp_fwd_f32(const char* who, const float* r, int64_t n_edges, int32_t n_in, int32_t n_layers,
+                       const MlpWeights& w, float* flat, float* o, size_t lds, hipStream_t s) {
+#define MLP_FWD(NL)                                                                                   \
+  if (mlp_lds_attr((const void*)k_mlp_fwd_mfma<NL>, lds)) return -1;                                  \
+  hipLaunchKernelGGL(k_mlp_fwd_mfma<NL>, mlp_mfma_grid(n_edges), dim3(256), lds, s, r, n_edges, n_in, w, flat, o)
+  switch (n_layers) {
+    case 1: MLP_FWD(1); break;
+    case 2: MLP_FWD(2); break;
+    case 3: MLP_FWD(3); break;
+    default: MLP_FWD(4); break;
+  }
+#undef MLP_FWD
+  return tace_check_launch(who);
+}
+
 int tace_radial_mlp_fwd(int dtype, const void* radial, int64_t n_edges, int32_t n_in, int32_t n_layers,
                         const void* weights, void* h, void* stream) {
   if (mlp_checks("tace_radial_mlp_fwd", n_edges, n_in, n_layers)) return -1;
@@ -591,18 +658,8 @@ int tace_radial_mlp_fwd(int dtype, const void* radial, int64_t n_edges, int32_t 
   const dim3 g((unsigned)((n_edges + 255) / 256)), b(256);
   if (dtype == TACE_F32) {
     const size_t lds = mlp_lds_bytes(n_in, n_layers);
-    const float *r = (const float*)radial, *w = (const float*)weights;
-    float* o = (float*)h;
-#define MLP_FWD(NL)                                                                                   \
-  if (mlp_lds_attr((const void*)k_mlp_fwd_mfma<NL>, lds)) return -1;                                  \
-  hipLaunchKernelGGL(k_mlp_fwd_mfma<NL>, mlp_mfma_grid(n_edges), b, lds, s, r, n_edges, n_in, w, o)
-    switch (n_layers) {
-      case 1: MLP_FWD(1); break;
-      case 2: MLP_FWD(2); break;
-      case 3: MLP_FWD(3); break;
-      default: MLP_FWD(4); break;
-    }
-#undef MLP_FWD
+    return mlp_fwd_f32("tace_radial_mlp_fwd", (const float*)radial, n_edges, n_in, n_layers,
+                       mlp_flat((const float*)weights, n_in, n_layers), nullptr, (float*)h, lds, s);
   } else if (dtype == TACE_F64) {
     hipLaunchKernelGGL(k_mlp_fwd<double>, g, b, 0, s, (const double*)radial, n_edges, n_in, n_layers,
                        (const double*)weights, (double*)h);
@@ -610,6 +667,25 @@ int tace_radial_mlp_fwd(int dtype, const void* radial, int64_t n_edges, int32_t 
     return tace_fail_msg("tace_radial_mlp_fwd: dtype must be TACE_F32 or TACE_F64");
   }
   return tace_check_launch("tace_radial_mlp_fwd");
+}
+
+int tace_radial_mlp_fwd_scaled(const float* radial, int64_t n_edges, int32_t n_in, int32_t n_layers,
+                               const float* const* weights, const double* scales, float* flat, float* h,
+                               void* stream) {
+  if (mlp_checks("tace_radial_mlp_fwd_scaled", n_edges, n_in, n_layers)) return -1;
+  if (n_edges == 0) return 0;
+  if (!radial || !weights || !scales || !flat || !h)
+    return tace_fail_msg("tace_radial_mlp_fwd_scaled: null pointer");
+  MlpWeights w;
+  w.vec = (((uintptr_t)flat) & 15) == 0;
+  for (int l = 0; l < TACE_MLP_MAX_LAYERS; ++l) {
+    w.w[l] = weights[l < n_layers ? l : 0];
+    w.scale[l] = (float)scales[l < n_layers ? l : 0];
+    if (!w.w[l]) return tace_fail_msg("tace_radial_mlp_fwd_scaled: null pointer");
+    if (((uintptr_t)w.w[l]) & 15) w.vec = 0;
+  }
+  return mlp_fwd_f32("tace_radial_mlp_fwd_scaled", radial, n_edges, n_in, n_layers, w, flat, h,
+                     mlp_lds_bytes(n_in, n_layers), (hipStream_t)stream);
 }
 
 int tace_radial_mlp_bwd(int dtype, const void* radial, const void* g_h, int64_t n_edges, int32_t n_in,
@@ -621,7 +697,8 @@ int tace_radial_mlp_bwd(int dtype, const void* radial, const void* g_h, int64_t 
   const dim3 g((unsigned)((n_edges + 255) / 256)), b(256);
   if (dtype == TACE_F32) {
     const size_t lds = mlp_lds_bytes(n_in, n_layers);
-    const float *r = (const float*)radial, *gg = (const float*)g_h, *w = (const float*)weights;
+    const float *r = (const float*)radial, *gg = (const float*)g_h;
+    const MlpWeights w = mlp_flat((const float*)weights, n_in, n_layers);
     float* o = (float*)g_radial;
 #define MLP_BWD(NL)                                                                                   \
   if (mlp_lds_attr((const void*)k_mlp_bwd_mfma<NL>, lds)) return -1;                                  \

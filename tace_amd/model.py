@@ -589,7 +589,7 @@ class MLP(torch.nn.Module):
     def hidden(self, x):
         """The last hidden activations [E, 64] (fused MLPs only)."""
         lins = [m for m in self.mlp if isinstance(m, mlpLinear)]
-        return ops.radial_mlp_hidden(x, [m.weight * m.alpha for m in lins[:-1]])
+        return ops.radial_mlp_hidden(x, [m.weight for m in lins[:-1]], [m.alpha for m in lins[:-1]])
 
     def last_layer(self):
         """(weight [64, n_out], alpha) of the last linear layer: the MLP's

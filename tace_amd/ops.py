@@ -1772,6 +1772,25 @@ def launch_mlp_hidden_fwd(radial, weights, n_layers: int) -> torch.Tensor:
     return h
 
 
+def launch_mlp_hidden_fwd_scaled(radial, mats, scales):
+    """``launch_mlp_hidden_fwd`` (float32) from the layers' own matrices, each
+    times its scale: (h, the scaled weights back to back, made on the way)."""
+    E, n_in = radial.shape
+    n = len(mats)
+    _req(radial, "radial", torch.float32, (E, n_in))
+    for layer, m in enumerate(mats):
+        _req(m, "weights", torch.float32, (64 if layer else n_in, 64))
+    h = torch.empty(E, 64, dtype=torch.float32, device=radial.device)
+    flat = torch.empty((n_in + 64 * (n - 1)) * 64, dtype=torch.float32, device=radial.device)
+    tok = _t0("radial_mlp_fwd")
+    N.check(N.lib().tace_radial_mlp_fwd_scaled(radial.data_ptr(), E, n_in, n,
+                                               (ctypes.c_void_p * n)(*[m.data_ptr() for m in mats]),
+                                               (ctypes.c_double * n)(*scales), flat.data_ptr(), h.data_ptr(),
+                                               N.stream_ptr(radial.device)), "tace_radial_mlp_fwd_scaled")
+    _t1(tok, (E, n_in, n))
+    return h, flat
+
+
 def launch_mlp_hidden_bwd(radial, gh, weights, n_layers: int) -> torch.Tensor:
     """grad of ``radial`` from the grad of the last hidden activations."""
     E, n_in = radial.shape
@@ -1797,6 +1816,21 @@ class _RadialMlp(torch.autograd.Function):
     def backward(ctx, gh):
         radial, weights = ctx.saved_tensors
         return launch_mlp_hidden_bwd(radial, gh.contiguous(), weights, ctx.n_layers), None, None
+
+
+class _RadialMlpScaled(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, radial, scales, *mats):
+        h, flat = launch_mlp_hidden_fwd_scaled(radial, mats, scales)
+        ctx.save_for_backward(radial, flat)
+        ctx.n_layers = len(mats)
+        return h
+
+    @staticmethod
+    def backward(ctx, gh):
+        radial, flat = ctx.saved_tensors
+        g = launch_mlp_hidden_bwd(radial, gh.contiguous(), flat, ctx.n_layers)
+        return (g, None) + (None,) * ctx.n_layers
 
 
 def launch_mlp_out_f32(h, W, alpha: float) -> torch.Tensor:
@@ -1884,10 +1918,18 @@ def radial_mlp_out(h: torch.Tensor, W: torch.Tensor, alpha: float) -> torch.Tens
     return h.new_empty(h.shape[0], W.shape[1]).addmm_(h, W, beta=0.0, alpha=alpha)
 
 
-def radial_mlp_hidden(radial: torch.Tensor, mats: Sequence[torch.Tensor]) -> torch.Tensor:
+def radial_mlp_hidden(radial: torch.Tensor, mats: Sequence[torch.Tensor],
+                      scales: Optional[Sequence[float]] = None) -> torch.Tensor:
     """silu(... silu(radial @ mats[0]) ... @ mats[-1]) for width-64 hidden
-    layers (scales folded into ``mats``): the last hidden activations [E, 64].
-    The matrices are constants here: gradients flow to ``radial`` only."""
+    layers (each times its entry of ``scales``, if given): the last hidden
+    activations [E, 64].  The matrices are constants here: gradients flow to
+    ``radial`` only."""
+    if scales is not None:
+        if (1 <= len(mats) <= 4 and radial.shape[1] <= 32
+                and all(m.dtype == radial.dtype == torch.float32 and m.device == radial.device and m.is_contiguous()
+                        for m in mats)):
+            return _RadialMlpScaled.apply(radial.contiguous(), tuple(map(float, scales)), *[m.detach() for m in mats])
+        mats = [m * s for m, s in zip(mats, scales)]
     flat = torch.cat([m.detach().reshape(-1) for m in mats]).to(radial.dtype).contiguous()
     return _RadialMlp.apply(radial.contiguous(), flat, len(mats))
 

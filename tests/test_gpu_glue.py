@@ -250,3 +250,27 @@ def test_last_radial_layer_parts(cuda, E, n):
     s = a.double() + b.double()
     mag = (a.double().abs() + b.double().abs()) @ w64.abs().t()
     assert ((got - 0.5 * s @ w64.t()).abs() <= (tol + u) * mag).all()
+
+
+@pytest.mark.parametrize("E,n_in,n,off", [(1, 8, 3, 0), (33, 7, 3, 0), (300, 32, 4, 0), (129, 1, 1, 0), (64, 10, 2, 1),
+                                          (0, 8, 3, 0)])
+def test_hidden_layers_scale_their_weights(cuda, E, n_in, n, off):
+    """Weights scaled in the kernel and before it: the same bits, forward and
+    input gradient (odd first layers, 1 .. 4 layers, matrices off 16 bytes)."""
+    g = torch.Generator().manual_seed(E + n_in)
+    mats = []
+    for layer in range(n):
+        buf = torch.empty((64 if layer else n_in) * 64 + off, device=cuda)
+        mats.append(buf[off:].view(-1, 64).copy_(torch.randn(64 if layer else n_in, 64, generator=g)))
+    scales = [(1.0 if layer == 0 else 2 ** 0.5) / m.shape[0] ** 0.5 for layer, m in enumerate(mats)]
+    x = torch.randn(E, n_in, generator=g).to(cuda).requires_grad_(True)
+    gh = torch.randn(E, 64, generator=g).to(cuda)
+    a = ops.radial_mlp_hidden(x, mats, scales)
+    b = ops.radial_mlp_hidden(x, [m * s for m, s in zip(mats, scales)])
+    (ga,), (gb,) = torch.autograd.grad(a, x, gh), torch.autograd.grad(b, x, gh)
+    assert torch.equal(a, b) and torch.equal(ga, gb)
+    w = [m.double().cpu() * s for m, s in zip(mats, scales)]
+    h = x.detach().double().cpu()
+    for m in w:
+        h = torch.nn.functional.silu(h @ m)
+    assert E == 0 or (a.double().cpu() - h).abs().max() < 1e-5 * h.abs().max().clamp_min(1)
