@@ -1937,8 +1937,12 @@ def radial_mlp_hidden(radial: torch.Tensor, mats: Sequence[torch.Tensor],
 # ------------------------------------------------------ per-species linears ----
 # output blocks of at least this many columns whose tiles have one
 # contribution with k <= 256 (or none) go to tace_seg_linear_presplit_ks
-# (pre-split plans only; None: every tile to the tile kernel)
-SEG_KS_MIN_N = 256
+# (pre-split plans only; None: every tile to the tile kernel).  Its operands
+# come in once instead of a 32-k step at a time: 128 -> 128 channels of 16
+# components, 12,288 nodes 55 -> 47 us, 3,000 nodes of 89 species 26 -> 19, 64
+# channels of 12,288 nodes 32 -> 27; narrower blocks leave its wavefronts
+# without columns
+SEG_KS_MIN_N = 64
 # columns per tace_seg_linear_presplit_ks task of k <= 128 (one group of
 # wavefronts: 512 fill the GPU sooner, 200 rows 44 -> 34 us, and cost nothing
 # at 5,184) and of k <= 256 (two groups: 512 cost 8% at 3,000 rows of 89 species)

@@ -37,6 +37,7 @@ def test_seg_linear_row_halves_equal_in_kernel_split(cuda, irr_in, irr_out, monk
     from tace_amd import model as pm
     monkeypatch.setattr(pm, "SEG_LINEAR_TILE_F32", 128)
     monkeypatch.setattr(ops, "SEG_SPLIT_SLOTS", None)   # split k sums in another order
+    monkeypatch.setattr(ops, "SEG_KS_MIN_N", 256)       # the tile kernel for narrow blocks
     counts = [1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 191, 192, 193, 257, 0] * 3
     S, Z = len(counts), sum(counts)
     species = torch.repeat_interleave(torch.arange(S), torch.tensor(counts))
