@@ -501,12 +501,19 @@ int tace_tece_rotate_out_bwd(int dtype, const void* const* m, const void* alpha,
  *   1. tace_nl_workspace_bytes -> allocate workspace
  *   2. tace_nl_count  -> counts[n] (edges per receiver)
  *   3. tace_scan_i32(counts) -> rowptr[n+1]; E = rowptr[n]
- *   4. tace_nl_fill   -> src[E] (int32), shifts[E,3] (int32) in rowptr order. */
+ *   4. tace_nl_fill   -> src[E] (int32), shifts[E,3] (int32) in rowptr order.
+ * kept (null, or [n_atoms, TACE_NL_KEEP, 4] int32, 16-byte aligned, the same
+ * buffer in both calls): the count leaves each receiver's first TACE_NL_KEEP
+ * hits there, and the fill copies the receivers that have no more instead of
+ * searching again.  Used by the wavefront-per-receiver form only (fewer than
+ * 32,768 atoms, or mode 2 of a batch). */
+#define TACE_NL_KEEP 128
 int64_t tace_nl_workspace_bytes(int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff);
 int tace_nl_count(const double* pos, int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff,
-                  void* workspace, int64_t workspace_bytes, int32_t* counts, void* stream);
+                  void* workspace, int64_t workspace_bytes, int32_t* counts, int32_t* kept, void* stream);
 int tace_nl_fill(const double* pos, int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff,
-                 const void* workspace, const int32_t* rowptr, int32_t* src, int32_t* shifts, void* stream);
+                 const void* workspace, const int32_t* rowptr, const int32_t* kept, int32_t* src, int32_t* shifts,
+                 void* stream);
 /* The same search for a batch of structures (a collated batch of the
  * reference's per-structure get_neighborhood calls,
  * dataset/neighbour_list.py:195-298, one per structure from
@@ -529,10 +536,11 @@ int64_t tace_nl_batch_plan(int32_t n_structs, const int64_t* sizes, const double
                            double cutoff, void* plan, int64_t plan_bytes, int64_t* n_atoms, int64_t* n_bins);
 int64_t tace_nl_batch_workspace_bytes(int64_t n_atoms, int64_t n_bins);
 int tace_nl_batch_count(const double* pos, int64_t n_atoms, int32_t n_structs, const void* plan, int64_t n_bins,
-                        void* workspace, int64_t workspace_bytes, int32_t mode, int32_t* counts, void* stream);
+                        void* workspace, int64_t workspace_bytes, int32_t mode, int32_t* counts, int32_t* kept,
+                        void* stream);
 int tace_nl_batch_fill(const double* pos, int64_t n_atoms, int32_t n_structs, const void* plan, int64_t n_bins,
                        const void* workspace, int64_t workspace_bytes, int32_t mode, const int32_t* rowptr,
-                       int32_t* src, int32_t* shifts, void* stream);
+                       const int32_t* kept, int32_t* src, int32_t* shifts, void* stream);
 /* Segmented row sum added into out: for each segment s < n_segments,
  * out[target[s], :] += sum over k in [rowptr[s], rowptr[s+1]) of
  * rows[slot[k], :] (slot NULL: rows[k]; target NULL: target[s] = s), rows of

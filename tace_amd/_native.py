@@ -94,12 +94,13 @@ _SIGS = {
     "tace_seg_linear_presplit_frag_split": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i32, _c_i32, _vp,
                                                      _c_i64, _c_dbl, _vp]),
     "tace_nl_workspace_bytes": (_c_i64, [_c_i64, _vp, _vp, _c_dbl]),
-    "tace_nl_count": (_c_int, [_vp, _c_i64, _vp, _vp, _c_dbl, _vp, _c_i64, _vp, _vp]),
-    "tace_nl_fill": (_c_int, [_vp, _c_i64, _vp, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp]),
+    "tace_nl_count": (_c_int, [_vp, _c_i64, _vp, _vp, _c_dbl, _vp, _c_i64, _vp, _vp, _vp]),
+    "tace_nl_fill": (_c_int, [_vp, _c_i64, _vp, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp, _vp]),
     "tace_nl_batch_plan": (_c_i64, [_c_i32, _vp, _vp, _vp, _c_dbl, _vp, _c_i64, _vp, _vp]),
     "tace_nl_batch_workspace_bytes": (_c_i64, [_c_i64, _c_i64]),
-    "tace_nl_batch_count": (_c_int, [_vp, _c_i64, _c_i32, _vp, _c_i64, _vp, _c_i64, _c_i32, _vp, _vp]),
-    "tace_nl_batch_fill": (_c_int, [_vp, _c_i64, _c_i32, _vp, _c_i64, _vp, _c_i64, _c_i32, _vp, _vp, _vp, _vp]),
+    "tace_nl_batch_count": (_c_int, [_vp, _c_i64, _c_i32, _vp, _c_i64, _vp, _c_i64, _c_i32, _vp, _vp, _vp]),
+    "tace_nl_batch_fill": (_c_int, [_vp, _c_i64, _c_i32, _vp, _c_i64, _vp, _c_i64, _c_i32, _vp, _vp, _vp, _vp,
+                                    _vp]),
     "tace_rows_accumulate": (_c_int, [_c_int, _vp, _c_i64, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _vp]),
     "tace_graph_sum": (_c_int, [_c_int, _vp, _c_i64, _c_i64, _vp, _c_i64, _vp, _vp]),
     "tace_narrow_linear": (_c_int, [_c_int, _vp, _c_i64, _c_i32, _vp, _vp, _c_i32, _vp, _vp]),

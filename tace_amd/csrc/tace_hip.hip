@@ -700,12 +700,15 @@ static __device__ __forceinline__ bool nl_pair(const double* __restrict__ pos, c
 // atoms, 13k receivers, 27 to some hundred bins each: 175 us a pass, now 77;
 // 12,288 atoms of water 84 -> 37; 1,024 of fcc 24 -> 12.)  Hits are counted by ballot
 // and take their slots by rank, so the edge order is the serial one.  Returns
-// the number of edges.
+// the number of edges.  Counting (FILL false) keeps the first NL_KEEP hits in
+// kept (null: none), so that filling copies them instead of searching again.
+constexpr int NL_KEEP = TACE_NL_KEEP;
+
 template <bool FILL>
 static __device__ __forceinline__ int nl_wave(const double* __restrict__ pos, const NlGeom& g, int b0, int lin, int a,
                                               const int* __restrict__ aimg, const int* __restrict__ bstart,
                                               const int* __restrict__ batoms, int base, int* __restrict__ src,
-                                              int* __restrict__ shift) {
+                                              int* __restrict__ shift, int4* __restrict__ kept) {
   const int lane = (int)(threadIdx.x & 63);
   const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
   const int ba[3] = {lin / (g.nb[1] * g.nb[2]), (lin / g.nb[2]) % g.nb[1], lin % g.nb[2]};
@@ -761,8 +764,10 @@ static __device__ __forceinline__ int nl_wave(const double* __restrict__ pos, co
         hit = nl_pair(pos, aimg, g, a, ax, ay, az, oa, tx, ty, tz, b, S);
       }
       const unsigned long long mask = __ballot(hit);
+      const int rank = cnt + __popcll(mask & ((1ull << lane) - 1ull));
+      if (!FILL && kept && hit && rank < NL_KEEP) kept[rank] = make_int4(b, S[0], S[1], S[2]);
       if (FILL && hit) {
-        const int slot = base + cnt + __popcll(mask & ((1ull << lane) - 1ull));
+        const int slot = base + rank;
         src[slot] = b;
         shift[3 * slot] = S[0];
         shift[3 * slot + 1] = S[1];
@@ -772,6 +777,37 @@ static __device__ __forceinline__ int nl_wave(const double* __restrict__ pos, co
     }
   }
   return cnt;
+}
+
+// One wavefront's receiver a: counts its edges (keeping the hits), or fills
+// them: from the kept hits when they all are there, else by a second search.
+// (128 crystals of 8-200 atoms, 361k edges: fill 76 -> 12 us, count 76 -> 81.)
+template <bool FILL>
+static __device__ __forceinline__ void nl_wave_edges(const double* __restrict__ pos, const NlGeom& g, int b0, int lin,
+                                                     int a, const int* __restrict__ aimg,
+                                                     const int* __restrict__ bstart, const int* __restrict__ batoms,
+                                                     int* __restrict__ counts, const int* __restrict__ rowptr,
+                                                     int* __restrict__ src, int* __restrict__ shift,
+                                                     int4* __restrict__ kept) {
+  const int lane = (int)(threadIdx.x & 63);
+  if (kept) kept += (int64_t)a * NL_KEEP;
+  if constexpr (FILL) {
+    const int base = rowptr[a], c = rowptr[a + 1] - base;
+    if (kept && c <= NL_KEEP) {
+      for (int k = lane; k < c; k += 64) {
+        const int4 h = kept[k];
+        src[base + k] = h.x;
+        shift[3 * (base + k)] = h.y;
+        shift[3 * (base + k) + 1] = h.z;
+        shift[3 * (base + k) + 2] = h.w;
+      }
+    } else {
+      nl_wave<true>(pos, g, b0, lin, a, aimg, bstart, batoms, base, src, shift, nullptr);
+    }
+  } else {
+    const int c = nl_wave<false>(pos, g, b0, lin, a, aimg, bstart, batoms, 0, nullptr, nullptr, kept);
+    if (lane == 0) counts[a] = c;
+  }
 }
 
 // For receiver a: every source b and shift S with |r_a - r_b + S.cell|^2 < rc^2,
@@ -787,13 +823,12 @@ __global__ __launch_bounds__(256) void k_nl_edges(const double* __restrict__ pos
                                                   const int* __restrict__ abin, const int* __restrict__ aimg,
                                                   const int* __restrict__ bstart, const int* __restrict__ batoms,
                                                   int* __restrict__ counts, const int* __restrict__ rowptr,
-                                                  int* __restrict__ src, int* __restrict__ shift) {
-  const int lane = WAVE ? (int)(threadIdx.x & 63) : 0;
+                                                  int* __restrict__ src, int* __restrict__ shift,
+                                                  int4* __restrict__ kept) {
   const int a = WAVE ? (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) : (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (a >= n) return;
   if constexpr (WAVE) {
-    const int c = nl_wave<FILL>(pos, g, 0, abin[a], a, aimg, bstart, batoms, FILL ? rowptr[a] : 0, src, shift);
-    if (!FILL && lane == 0) counts[a] = c;
+    nl_wave_edges<FILL>(pos, g, 0, abin[a], a, aimg, bstart, batoms, counts, rowptr, src, shift, kept);
     return;
   }
   const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
@@ -850,16 +885,15 @@ __global__ __launch_bounds__(256) void k_nlb_edges(const double* __restrict__ po
                                                    const int* __restrict__ abin, const int* __restrict__ aimg,
                                                    const int* __restrict__ bstart, const int* __restrict__ batoms,
                                                    int* __restrict__ counts, const int* __restrict__ rowptr,
-                                                   int* __restrict__ src, int* __restrict__ shift) {
-  const int lane = WAVE ? (int)(threadIdx.x & 63) : 0;
+                                                   int* __restrict__ src, int* __restrict__ shift,
+                                                  int4* __restrict__ kept) {
   const int a = WAVE ? (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) : (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (a >= n) return;
   const int s = nlb_struct_of(B, a);
   const NlGeom& g = B.geo[s];
   const int b0 = B.boff[s];
   if constexpr (WAVE) {
-    const int c = nl_wave<FILL>(pos, g, b0, abin[a] - b0, a, aimg, bstart, batoms, FILL ? rowptr[a] : 0, src, shift);
-    if (!FILL && lane == 0) counts[a] = c;
+    nl_wave_edges<FILL>(pos, g, b0, abin[a] - b0, a, aimg, bstart, batoms, counts, rowptr, src, shift, kept);
     return;
   }
   const double ax = pos[3 * a], ay = pos[3 * a + 1], az = pos[3 * a + 2];
@@ -1469,7 +1503,7 @@ int64_t tace_nl_workspace_bytes(int64_t n_atoms, const double* cell, const int32
 }
 
 int tace_nl_count(const double* pos, int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff,
-                  void* workspace, int64_t workspace_bytes, int32_t* counts, void* stream) {
+                  void* workspace, int64_t workspace_bytes, int32_t* counts, int32_t* kept, void* stream) {
   NlGeom g;
   if (!cell || !pbc) return fail("tace_nl_count: null pointer");
   if (nl_geometry(cell, pbc, cutoff, &g)) return -1;
@@ -1479,6 +1513,7 @@ int tace_nl_count(const double* pos, int64_t n_atoms, const double* cell, const 
   const int64_t nbins = (int64_t)g.nb[0] * g.nb[1] * g.nb[2];
   if (workspace_bytes < (int64_t)sizeof(int32_t) * (n_atoms * 6 + nbins * 3 + 1))
     return fail("tace_nl_count: workspace too small");
+  if (((uintptr_t)kept) & 15) return fail("tace_nl_count: kept must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int n = (int)n_atoms;
   int* abin = (int*)workspace;
@@ -1496,21 +1531,23 @@ int tace_nl_count(const double* pos, int64_t n_atoms, const double* cell, const 
   hipLaunchKernelGGL(k_nlb_rank, ga, ba, 0, s, abin, n, bstart, unsorted, batoms);
   if (n < NL_WAVE_MAX)
     hipLaunchKernelGGL((k_nl_edges<false, true>), dim3((n + 3) / 4), dim3(256), 0, s, pos, n, g, abin, aimg, bstart,
-                       batoms, counts, nullptr, nullptr, nullptr);
+                       batoms, counts, nullptr, nullptr, nullptr, (int4*)kept);
   else
     hipLaunchKernelGGL((k_nl_edges<false, false>), dim3((n + 255) / 256), dim3(256), 0, s, pos, n, g, abin, aimg,
-                       bstart, batoms, counts, nullptr, nullptr, nullptr);
+                       bstart, batoms, counts, nullptr, nullptr, nullptr, (int4*)kept);
   return check_launch("tace_nl_count");
 }
 
 int tace_nl_fill(const double* pos, int64_t n_atoms, const double* cell, const int32_t* pbc, double cutoff,
-                 const void* workspace, const int32_t* rowptr, int32_t* src, int32_t* shifts, void* stream) {
+                 const void* workspace, const int32_t* rowptr, const int32_t* kept, int32_t* src, int32_t* shifts,
+                 void* stream) {
   NlGeom g;
   if (!cell || !pbc) return fail("tace_nl_fill: null pointer");
   if (nl_geometry(cell, pbc, cutoff, &g)) return -1;
   if (n_atoms <= 0) return 0;
   if (!pos || !workspace || !rowptr || !src || !shifts) return fail("tace_nl_fill: null pointer");
   const int64_t nbins = (int64_t)g.nb[0] * g.nb[1] * g.nb[2];
+  if (((uintptr_t)kept) & 15) return fail("tace_nl_fill: kept must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int n = (int)n_atoms;
   const int* abin = (const int*)workspace;
@@ -1521,10 +1558,10 @@ int tace_nl_fill(const double* pos, int64_t n_atoms, const double* cell, const i
   const int* batoms = bfill + nbins;
   if (n < NL_WAVE_MAX)
     hipLaunchKernelGGL((k_nl_edges<true, true>), dim3((n + 3) / 4), dim3(256), 0, s, pos, n, g, abin, aimg, bstart,
-                       batoms, nullptr, rowptr, src, shifts);
+                       batoms, nullptr, rowptr, src, shifts, (int4*)kept);
   else
     hipLaunchKernelGGL((k_nl_edges<true, false>), dim3((n + 255) / 256), dim3(256), 0, s, pos, n, g, abin, aimg,
-                       bstart, batoms, nullptr, rowptr, src, shifts);
+                       bstart, batoms, nullptr, rowptr, src, shifts, (int4*)kept);
   return check_launch("tace_nl_fill");
 }
 
@@ -1595,12 +1632,14 @@ static bool nlb_wave_mode(int64_t n_atoms, int32_t mode) {
 }
 
 int tace_nl_batch_count(const double* pos, int64_t n_atoms, int32_t n_structs, const void* plan, int64_t n_bins,
-                        void* workspace, int64_t workspace_bytes, int32_t mode, int32_t* counts, void* stream) {
+                        void* workspace, int64_t workspace_bytes, int32_t mode, int32_t* counts, int32_t* kept,
+                        void* stream) {
   NlBatch B;
   if (nlb_setup("tace_nl_batch_count", plan, n_structs, n_atoms, n_bins, workspace, workspace_bytes, &B)) return -1;
   if (mode < 0 || mode > 2) return fail("tace_nl_batch_count: mode must be 0 (auto), 1 (thread) or 2 (wave)");
   if (n_atoms == 0) return 0;
   if (!pos || !counts) return fail("tace_nl_batch_count: null pointer");
+  if (((uintptr_t)kept) & 15) return fail("tace_nl_batch_count: kept must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int n = (int)n_atoms, nb = (int)n_bins;
   int* abin = (int*)workspace;
@@ -1618,21 +1657,22 @@ int tace_nl_batch_count(const double* pos, int64_t n_atoms, int32_t n_structs, c
   hipLaunchKernelGGL(k_nlb_rank, ga, ba, 0, s, abin, n, bstart, unsorted, batoms);
   if (nlb_wave_mode(n_atoms, mode))
     hipLaunchKernelGGL((k_nlb_edges<false, true>), dim3((n + 3) / 4), dim3(256), 0, s, pos, n, B, abin, aimg,
-                       bstart, batoms, counts, nullptr, nullptr, nullptr);
+                       bstart, batoms, counts, nullptr, nullptr, nullptr, (int4*)kept);
   else
     hipLaunchKernelGGL((k_nlb_edges<false, false>), dim3((n + 255) / 256), dim3(256), 0, s, pos, n, B, abin, aimg,
-                       bstart, batoms, counts, nullptr, nullptr, nullptr);
+                       bstart, batoms, counts, nullptr, nullptr, nullptr, (int4*)kept);
   return check_launch("tace_nl_batch_count");
 }
 
 int tace_nl_batch_fill(const double* pos, int64_t n_atoms, int32_t n_structs, const void* plan, int64_t n_bins,
                        const void* workspace, int64_t workspace_bytes, int32_t mode, const int32_t* rowptr,
-                       int32_t* src, int32_t* shifts, void* stream) {
+                       const int32_t* kept, int32_t* src, int32_t* shifts, void* stream) {
   NlBatch B;
   if (nlb_setup("tace_nl_batch_fill", plan, n_structs, n_atoms, n_bins, workspace, workspace_bytes, &B)) return -1;
   if (mode < 0 || mode > 2) return fail("tace_nl_batch_fill: mode must be 0 (auto), 1 (thread) or 2 (wave)");
   if (n_atoms == 0) return 0;
   if (!pos || !rowptr || !src || !shifts) return fail("tace_nl_batch_fill: null pointer");
+  if (((uintptr_t)kept) & 15) return fail("tace_nl_batch_fill: kept must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
   const int n = (int)n_atoms, nb = (int)n_bins;
   const int* abin = (const int*)workspace;
@@ -1643,10 +1683,10 @@ int tace_nl_batch_fill(const double* pos, int64_t n_atoms, int32_t n_structs, co
   const int* batoms = bfill + nb;
   if (nlb_wave_mode(n_atoms, mode))
     hipLaunchKernelGGL((k_nlb_edges<true, true>), dim3((n + 3) / 4), dim3(256), 0, s, pos, n, B, abin, aimg,
-                       bstart, batoms, nullptr, rowptr, src, shifts);
+                       bstart, batoms, nullptr, rowptr, src, shifts, (int4*)kept);
   else
     hipLaunchKernelGGL((k_nlb_edges<true, false>), dim3((n + 255) / 256), dim3(256), 0, s, pos, n, B, abin, aimg,
-                       bstart, batoms, nullptr, rowptr, src, shifts);
+                       bstart, batoms, nullptr, rowptr, src, shifts, (int4*)kept);
   return check_launch("tace_nl_batch_fill");
 }
 

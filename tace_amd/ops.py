@@ -2423,6 +2423,17 @@ def _runs(ls: Sequence[int]):
 
 
 # ------------------------------------------------------------ neighbours ----
+NL_KEEP, NL_KEEP_ATOMS = 128, 32768   # TACE_NL_KEEP; the wavefront-per-receiver form's sizes
+
+
+def _nl_kept(n: int, mode: int, device) -> Optional[torch.Tensor]:
+    """The neighbour search's buffer of hits (2 KB an atom, at most 64 MB), or
+    None: larger systems count with a thread per receiver, or search twice."""
+    if mode == 1 or not 0 < n < NL_KEEP_ATOMS:
+        return None
+    return torch.empty(n, NL_KEEP, 4, dtype=torch.int32, device=device)
+
+
 def neighbour_list(positions: torch.Tensor, cell, pbc, cutoff: float):
     """GPU cell-list neighbour search (float64).
 
@@ -2441,8 +2452,10 @@ def neighbour_list(positions: torch.Tensor, cell, pbc, cutoff: float):
     ws = torch.empty(max(int(nbytes), 4), dtype=torch.uint8, device=dev)
     counts = torch.empty(n, dtype=torch.int32, device=dev)
     s = N.stream_ptr(dev)
+    kept = _nl_kept(n, 0, dev)
+    k_ptr = None if kept is None else kept.data_ptr()
     N.check(L.tace_nl_count(positions.data_ptr(), n, cell_np.ctypes.data, pbc_np.ctypes.data, float(cutoff),
-                            ws.data_ptr(), int(nbytes), counts.data_ptr(), s), "tace_nl_count")
+                            ws.data_ptr(), int(nbytes), counts.data_ptr(), k_ptr, s), "tace_nl_count")
     rowptr = torch.empty(n + 1, dtype=torch.int32, device=dev)
     N.check(L.tace_scan_i32(counts.data_ptr(), n, rowptr.data_ptr(), s), "tace_scan_i32")
     E = int(rowptr[-1].item())
@@ -2450,7 +2463,7 @@ def neighbour_list(positions: torch.Tensor, cell, pbc, cutoff: float):
     shifts = torch.empty(E, 3, dtype=torch.int32, device=dev)
     if E > 0:
         N.check(L.tace_nl_fill(positions.data_ptr(), n, cell_np.ctypes.data, pbc_np.ctypes.data, float(cutoff),
-                               ws.data_ptr(), rowptr.data_ptr(), src.data_ptr(), shifts.data_ptr(), s),
+                               ws.data_ptr(), rowptr.data_ptr(), k_ptr, src.data_ptr(), shifts.data_ptr(), s),
                 "tace_nl_fill")
     return rowptr, src, shifts
 
@@ -2519,8 +2532,10 @@ def neighbour_list_batch(positions: torch.Tensor, sizes: Sequence[int], cells, p
     ws = torch.empty(max(wsb, 4), dtype=torch.uint8, device=dev)
     counts = torch.empty(max(n_tot, 1), dtype=torch.int32, device=dev)
     st = N.stream_ptr(dev)
+    kept = _nl_kept(n_tot, mode, dev)
+    k_ptr = None if kept is None else kept.data_ptr()
     N.check(L.tace_nl_batch_count(positions.data_ptr(), n_tot, ns, plan.data_ptr(), nb.value, ws.data_ptr(), wsb,
-                                  mode, counts.data_ptr(), st), "tace_nl_batch_count")
+                                  mode, counts.data_ptr(), k_ptr, st), "tace_nl_batch_count")
     rowptr = torch.empty(n_tot + 1, dtype=torch.int32, device=dev)
     N.check(L.tace_scan_i32(counts.data_ptr(), n_tot, rowptr.data_ptr(), st), "tace_scan_i32")
     E = int(rowptr[-1].item())
@@ -2528,7 +2543,7 @@ def neighbour_list_batch(positions: torch.Tensor, sizes: Sequence[int], cells, p
     shifts = torch.empty(E, 3, dtype=torch.int32, device=dev)
     if E > 0:
         N.check(L.tace_nl_batch_fill(positions.data_ptr(), n_tot, ns, plan.data_ptr(), nb.value, ws.data_ptr(), wsb,
-                                     mode, rowptr.data_ptr(), src.data_ptr(), shifts.data_ptr(), st),
+                                     mode, rowptr.data_ptr(), k_ptr, src.data_ptr(), shifts.data_ptr(), st),
                 "tace_nl_batch_fill")
     return rowptr, src, shifts
 

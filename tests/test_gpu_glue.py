@@ -274,3 +274,24 @@ def test_hidden_layers_scale_their_weights(cuda, E, n_in, n, off):
     for m in w:
         h = torch.nn.functional.silu(h @ m)
     assert E == 0 or (a.double().cpu() - h).abs().max() < 1e-5 * h.abs().max().clamp_min(1)
+
+
+@pytest.mark.parametrize("n,box,rc", [(1, 3.0, 0.5), (1, 3.0, 6.0), (40, 6.0, 4.2), (260, 7.5, 4.0), (260, 7.5, 5.6)])
+def test_neighbours_kept_or_searched_again(cuda, n, box, rc, monkeypatch):
+    """Receivers with no neighbour, with fewer than the kept hits, around them
+    and with more: copied, searched again and by a thread per receiver, the
+    same edges in the same order."""
+    g = torch.Generator().manual_seed(n)
+    pos = (torch.rand(n, 3, generator=g, dtype=torch.float64) * box).to(cuda)
+    cell = (box * torch.eye(3, dtype=torch.float64)).numpy()
+    args = (pos, [n], [cell], [(True, True, False)], rc)
+    kept, single = ops.neighbour_list_batch(*args), ops.neighbour_list(pos, cell, (True, True, False), rc)
+    thread = ops.neighbour_list_batch(*args, mode=1)
+    monkeypatch.setattr(ops, "NL_KEEP_ATOMS", 0)
+    again = ops.neighbour_list_batch(*args)
+    for other in (single, thread, again):
+        assert all(torch.equal(a, b) for a, b in zip(kept, other))
+    counts = kept[0].diff()
+    if n == 260:
+        over = counts > ops.NL_KEEP
+        assert over.any() and bool((~over).any()) == (rc < 5)
