@@ -1,16 +1,22 @@
 // Stable grouping of integer keys (the receiver and sender CSRs of an edge
 // list): positions 0 .. n-1 ordered by key, in position order within a key,
-// and each key's range.  A counting sort: count (each position's place among
-// its key's, in arrival order), scan, scatter, then every position is moved
-// to its rank by id inside its key's range.  The degrees of a neighbour list
-// are tens to hundreds, so the ranking reads each range a few dozen times
-// from L1 and L2, where a radix or merge sort and a binary search take 10 to
-// 30 launches.  Measured against those (us): the sender CSR of 46k edges of
-// 1,024 nodes 58 -> 25, of 1.06 M edges of 12,288 nodes 124 -> 71; the
-// receiver and sender CSR of shuffled edges 291 -> 81 and 607 -> 221 (with
-// the checks; one wait for the host instead of three); 5.6 M edges of 101k
-// nodes 261 (random keys of that size, which no neighbour list has, 282 ->
-// 552: the counting atomics then miss L2).
+// and each key's range.  A radix sort from the low digit that moves (key,
+// position) pairs only: per digit a workgroup counts its 2,048 positions in
+// LDS, one scan per digit value turns the counts into places, and a position's
+// rank among the equal digits of its wavefront comes from ballots.  No atomic
+// reaches memory and no step depends on how the keys are distributed.  (A
+// counting sort by atomics, ranking every range by its length squared, was
+// faster at best and did not have that: atomics on neighbouring keys meet in
+// one slice of the memory, a hub or a handful of keys makes the ranges long.)
+//
+// us, library sort and binary search | that counting sort | this: senders of
+// fcc lists of 78 edges a node, 13,500 nodes 124 | 81 | 57, with node ids
+// shuffled 124 | 163 | 67; 97,556 nodes shuffled 362 | 751 | 395; 8,192 equal
+// keys 41 | 3,129 | 15; 361,000 sorted under 16 keys 120 | 4,296 | 23; 30 M
+// random under 1 M keys 1,431 | 3,473 | 2,062 (runs of a digit are a few
+// words long: stores; the caller sorts lists that long).  The receiver CSR of
+// 1.05 M edges with the checks and the host's wait, sorted 228 | 253 | 85,
+// shuffled 459 | 133 | 98 (bincount, two minima, argsort before).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -21,11 +27,6 @@ int tace_fail_msg(const char* msg);   // tace_hip.hip
 int tace_check_launch(const char* what);
 
 namespace {
-
-// ranges longer than this are ordered by a workgroup that walks all keys
-// (k_group_long) instead of a rank per entry, whose cost grows with the
-// square of the range
-constexpr int LONG_RANGE = 4096;
 
 // the keys, and (other != null) a second array of the same range that is only
 // checked and converted (an edge list's senders beside its receivers)
@@ -55,112 +56,195 @@ struct Keys {
   }
 };
 
+// keys outside the range come after all others
+__device__ __forceinline__ int sort_key(int k32, int n_keys) { return k32 < 0 ? n_keys : k32; }
+
+// the lanes that hold this lane's digit (of `bits` bits), of those with in
+__device__ __forceinline__ unsigned long long same_digit(int d, int bits, bool in) {
+  unsigned long long m = __ballot(in);
+  for (int b = 0; b < bits; ++b) {
+    const bool one = (d >> b) & 1;
+    const unsigned long long v = __ballot(one);
+    m &= one ? v : ~v;
+  }
+  return m;
+}
+
+// this lane's place among its wavefront's equal digits so far: cnt[d] holds
+// them and grows by this step's
+__device__ __forceinline__ int digit_rank(int* cnt, int d, int bits, bool in, int lane) {
+  const unsigned long long m = same_digit(d, bits, in);
+  const int r = __popcll(m & ((1ull << lane) - 1));
+  int before = 0;
+  if (in && r == 0) before = atomicAdd(cnt + d, __popcll(m));
+  return r + __shfl(before, in ? __ffsll((long long)m) - 1 : lane, 64);
+}
+
+constexpr int MAX_BITS = 9, MAX_BINS = 1 << MAX_BITS;   // a digit's
+// positions a workgroup: a run of 64 STEPS per wavefront (1.05 M edges, 2
+// digits: 57 us; 16 steps 71, 32 steps 101, a workgroup's steps being serial)
+constexpr int STEPS = 8, CHUNK = 256 * STEPS;
+
+// Counts of the lowest digit per workgroup, hist [bins + 2][nwg]; the last two
+// rows hold the flags.  Reads, checks and converts the keys.
 template <typename K>
-__global__ __launch_bounds__(256) void k_group_count(Keys<K> in, int n, int n_keys, int* __restrict__ k32,
-                                                     int* __restrict__ cnt, int* __restrict__ place,
-                                                     int* __restrict__ flags) {
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (i >= n) return;
-  const int key = in.get(i, n_keys, flags);
-  k32[i] = key;
-  if (key >= 0) place[i] = atomicAdd(cnt + key, 1);
-}
-
-__global__ __launch_bounds__(1024) void k_group_scan(const int* __restrict__ cnt, int m, int* __restrict__ out) {
-  scan_1024(cnt, m, out);
-}
-
-__global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ k32, const int* __restrict__ place,
-                                                       int n, const int* __restrict__ rowptr, int* __restrict__ tmp) {
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (i >= n || k32[i] < 0) return;
-  tmp[rowptr[k32[i]] + place[i]] = i;
-}
-
-__global__ __launch_bounds__(256) void k_group_rank(const int* __restrict__ k32, int n, const int* __restrict__ rowptr,
-                                                    const int* __restrict__ tmp, int* __restrict__ order) {
-  const int q = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (q >= n) return;
-  const int i = tmp[q];
-  if (i < 0) return;   // a position whose key was out of range left its slot empty
-  const int key = k32[i], b = rowptr[key], e = rowptr[key + 1];
-  if (e - b > LONG_RANGE) return;
-  int r = b;
+__global__ __launch_bounds__(256) void k_group_first(Keys<K> in, int n, int n_keys, int bins, int* __restrict__ k32,
+                                                     int* __restrict__ hist) {
+  __shared__ int cnt[MAX_BINS + 2];
+  const int t = (int)threadIdx.x;
+  for (int b = t; b < bins + 2; b += 256) cnt[b] = 0;
+  __syncthreads();
+  const int64_t i0 = (int64_t)blockIdx.x * CHUNK + t;
 #pragma unroll 4
-  for (int p = b; p < e; ++p) r += tmp[p] < i;
-  order[r] = i;
+  for (int u = 0; u < STEPS; ++u) {
+    if (i0 + 256 * u >= n) break;
+    const int i = (int)i0 + 256 * u, key = in.get(i, n_keys, cnt + bins);
+    k32[i] = key;
+    atomicAdd(cnt + (sort_key(key, n_keys) & (bins - 1)), 1);
+  }
+  __syncthreads();
+  for (int b = t; b < bins + 2; b += 256) hist[(int64_t)b * gridDim.x + blockIdx.x] = cnt[b];
 }
 
-// the ranges longer than LONG_RANGE: each holds a multiple of LONG_RANGE; the
-// workgroup of the first one walks all keys and keeps the range's in order
-__global__ __launch_bounds__(1024) void k_group_long(const int* __restrict__ k32, int n, const int* __restrict__ rowptr,
-                                                     const int* __restrict__ tmp, int* __restrict__ order) {
-  __shared__ int wcnt[16];
-  const int q = (int)blockIdx.x * LONG_RANGE;
-  if (q >= n) return;
-  const int i0 = tmp[q];
-  if (i0 < 0) return;
-  const int key = k32[i0], b = rowptr[key], e = rowptr[key + 1];
-  if (e - b <= LONG_RANGE || q - LONG_RANGE >= b) return;   // short, or another workgroup's
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
-  int at = b;
-  for (int p = 0; p < n; p += 1024) {
-    const bool hit = p + t < n && k32[p + t] == key;
-    const unsigned long long mask = __ballot(hit);
-    if (lane == 0) wcnt[w] = __popcll(mask);
-    __syncthreads();
-    int before = 0, total = 0;
+// the same of a later digit (no flags)
+__global__ __launch_bounds__(256) void k_group_count(const int* __restrict__ keys, int n, int shift, int bins,
+                                                     int* __restrict__ hist) {
+  __shared__ int cnt[MAX_BINS];
+  const int t = (int)threadIdx.x;
+  for (int b = t; b < bins; b += 256) cnt[b] = 0;
+  __syncthreads();
+  const int64_t i0 = (int64_t)blockIdx.x * CHUNK + t;
+#pragma unroll 4
+  for (int u = 0; u < STEPS; ++u) {
+    if (i0 + 256 * u >= n) break;
+    atomicAdd(cnt + ((keys[i0 + 256 * u] >> shift) & (bins - 1)), 1);
+  }
+  __syncthreads();
+  for (int b = t; b < bins; b += 256) hist[(int64_t)b * gridDim.x + blockIdx.x] = cnt[b];
+}
+
+// a workgroup per digit value: its counts before each workgroup, offs [bins +
+// 2][nwg + 1], the last column their total; flags from the two rows after them
+__global__ __launch_bounds__(1024) void k_group_scan(const int* __restrict__ hist, int nwg, int bins,
+                                                     int* __restrict__ offs, int* __restrict__ flags) {
+  int* o = offs + (int64_t)blockIdx.x * (nwg + 1);
+  scan_1024(hist + (int64_t)blockIdx.x * nwg, nwg, o);
+  if (flags && (int)blockIdx.x >= bins && threadIdx.x == 0) flags[blockIdx.x - bins] = o[nwg] != 0;
+}
+
+// Every (key, position) to its place by one digit.  pos null: position i is i.
+__global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ keys, const int* __restrict__ pos, int n,
+                                                       int n_keys, int shift, int bits, const int* __restrict__ offs,
+                                                       int* __restrict__ keys_out, int* __restrict__ pos_out) {
+  __shared__ int cnt[4][MAX_BINS], wsum[4];
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, bins = 1 << bits, nwg = (int)gridDim.x;
+  for (int b = t; b < 4 * MAX_BINS; b += 256) cnt[b / MAX_BINS][b % MAX_BINS] = 0;
+  __syncthreads();
+  const int64_t i0 = (int64_t)blockIdx.x * CHUNK + 64 * STEPS * w + lane;
+  int key[STEPS], rank[STEPS];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      if (k < w) before += wcnt[k];
-      total += wcnt[k];
+  for (int u = 0; u < STEPS; ++u) {
+    key[u] = i0 + 64 * u < n ? sort_key(keys[i0 + 64 * u], n_keys) : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u)
+    rank[u] = digit_rank(cnt[w], (key[u] >> shift) & (bins - 1), bits, key[u] >= 0, lane);
+  __syncthreads();
+  // where each digit's positions of each wavefront go: all smaller digits,
+  // the digit's in the workgroups before, in the wavefronts before.  Thread t
+  // has digits 2 t and 2 t + 1.
+  int total[2], s = 0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    total[q] = 2 * t + q < bins ? offs[(int64_t)(2 * t + q) * (nwg + 1) + nwg] : 0;
+    s += total[q];
+  }
+  int inc = s;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += x;
+  }
+  if (lane == 63) wsum[w] = inc;
+  __syncthreads();
+  int run = inc - s;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k < w) run += wsum[k];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    if (2 * t + q < bins) {
+      int at = run + offs[(int64_t)(2 * t + q) * (nwg + 1) + blockIdx.x];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int c = cnt[k][2 * t + q];
+        cnt[k][2 * t + q] = at;
+        at += c;
+      }
     }
-    if (hit) order[at + before + __popcll(mask & ((1ull << lane) - 1))] = p + t;
-    at += total;
-    __syncthreads();
+    run += total[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) {
+    if (key[u] < 0) continue;
+    const int at = cnt[w][(key[u] >> shift) & (bins - 1)] + rank[u];
+    keys_out[at] = key[u];
+    pos_out[at] = pos ? pos[i0 + 64 * u] : (int)(i0 + 64 * u);
   }
 }
 
-__global__ __launch_bounds__(256) void k_group_fill(int* __restrict__ a, int64_t na, int va, int* __restrict__ b,
-                                                    int64_t nb, int vb) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < na) a[i] = va;
-  if (i < nb) b[i] = vb;
+// rowptr[k] = the number of sorted keys below k
+__global__ __launch_bounds__(256) void k_group_rows(const int* __restrict__ sorted, int n, int n_keys,
+                                                    int* __restrict__ rowptr) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k > n_keys) return;
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int mid = lo + (hi - lo) / 2;
+    if (sorted[mid] < k) lo = mid + 1;
+    else hi = mid;
+  }
+  rowptr[k] = lo;
 }
 
-// All of it in one workgroup for few positions (counts, places and ranges in
-// LDS): below SMALL_N the launches, not the work, take the time.
-constexpr int SMALL_N = 8192, SMALL_KEYS = 4096;
+// All of it in one workgroup for few positions, (key, position) packed in one
+// word and kept in LDS: below SMALL_N the launches, not the work, take the time.
+constexpr int SMALL_N = 8192, SMALL_KEYS = 4096, POS_BITS = 13, SMALL_BITS = 7, SMALL_BINS = 1 << SMALL_BITS;
 
 template <typename K>
-__global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_keys, int* __restrict__ k32,
-                                                      int* __restrict__ rowptr, int* __restrict__ order,
-                                                      int* __restrict__ flags) {
-  __shared__ int cnt[SMALL_KEYS], start[SMALL_KEYS + 1], tmp[SMALL_N], wsum[16], fl[2];
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
-  for (int i = t; i < n_keys; i += 1024) cnt[i] = 0;
+__global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_keys, int bits, int passes,
+                                                      int* __restrict__ k32, int* __restrict__ rowptr,
+                                                      int* __restrict__ order, int* __restrict__ flags) {
+  __shared__ int data[SMALL_N], cnt[16][SMALL_BINS], wsum[16], fl[2];
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, bins = 1 << bits;
+  constexpr int PER = SMALL_N / 1024;   // a run of 64 PER positions per wavefront
   if (t < 2) fl[t] = 0;
   __syncthreads();
-  constexpr int PER = SMALL_N / 1024;
-  int key[PER], place[PER];
+  const int i0 = 64 * PER * w + lane;
+  int v[PER], rank[PER];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int i = t + 1024 * u;
-    key[u] = -1;
+    const int i = i0 + 64 * u;
+    v[u] = -1;
     if (i < n) {
-      k32[i] = key[u] = in.get(i, n_keys, fl);
-      if (key[u] >= 0) place[u] = atomicAdd(&cnt[key[u]], 1);
+      const int key = in.get(i, n_keys, fl);
+      k32[i] = key;
+      v[u] = (sort_key(key, n_keys) << POS_BITS) | i;
     }
   }
-  __syncthreads();
-  // exclusive scan of cnt: four counts per thread
-  {
-    int v[4], s = 0;
+  for (int p = 0; p < passes; ++p) {
+    const int shift = POS_BITS + p * bits;
+    for (int b = t; b < 16 * SMALL_BINS; b += 1024) cnt[b / SMALL_BINS][b % SMALL_BINS] = 0;
+    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      v[q] = 4 * t + q < n_keys ? cnt[4 * t + q] : 0;
-      s += v[q];
-    }
+    for (int u = 0; u < PER; ++u)
+      rank[u] = digit_rank(cnt[w], (v[u] >> shift) & (bins - 1), bits, v[u] >= 0, lane);
+    __syncthreads();
+    // exclusive scan over (digit, wavefront): thread t has two wavefronts'
+    // counts of digit t / 8
+    int* c = &cnt[2 * (t & 7)][t >> 3];
+    const int a0 = c[0], a1 = c[SMALL_BINS], s = a0 + a1;
     int inc = s;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -169,68 +253,94 @@ __global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_k
     }
     if (lane == 63) wsum[w] = inc;
     __syncthreads();
-    int run = inc - s, total = 0;
+    int run = inc - s;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
+    for (int k = 0; k < 16; ++k)
       if (k < w) run += wsum[k];
-      total += wsum[k];
-    }
+    c[0] = run;
+    c[SMALL_BINS] = run + a0;
+    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (4 * t + q < n_keys) start[4 * t + q] = rowptr[4 * t + q] = run;
-      run += v[q];
-    }
-    if (t == 0) start[n_keys] = rowptr[n_keys] = total;
+    for (int u = 0; u < PER; ++u)
+      if (v[u] >= 0) data[cnt[w][(v[u] >> shift) & (bins - 1)] + rank[u]] = v[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) v[u] = i0 + 64 * u < n ? data[i0 + 64 * u] : -1;
+    // (the next pass's barriers keep its writes of data behind these reads)
   }
-  __syncthreads();
 #pragma unroll
   for (int u = 0; u < PER; ++u)
-    if (key[u] >= 0) tmp[start[key[u]] + place[u]] = t + 1024 * u;
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    if (key[u] < 0) continue;
-    const int i = t + 1024 * u, e = start[key[u] + 1];
-    int r = start[key[u]];
-    for (int p = start[key[u]]; p < e; ++p) r += tmp[p] < i;
-    order[r] = i;
+    if (v[u] >= 0) order[i0 + 64 * u] = v[u] & (SMALL_N - 1);
+  for (int k = t; k <= n_keys; k += 1024) {
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if ((data[mid] >> POS_BITS) < k) lo = mid + 1;
+      else hi = mid;
+    }
+    rowptr[k] = lo;
   }
   if (t < 2 && flags) flags[t] = fl[t];
+}
+
+// digits of at most `most` bits for sort keys 0 .. n_keys
+void digits(int n_keys, int most, int* bits, int* passes) {
+  int nb = 1;
+  while (nb < 31 && (n_keys >> nb) != 0) ++nb;
+  *passes = (nb + most - 1) / most;
+  *bits = (nb + *passes - 1) / *passes;
 }
 
 template <typename K>
 int group_keys(const Keys<K>& in, int n, int n_keys, int32_t* k32, int32_t* rowptr, int32_t* order, int32_t* work,
                int32_t* flags, hipStream_t s) {
+  int bits, passes;
   if (n <= SMALL_N && n_keys <= SMALL_KEYS) {
-    hipLaunchKernelGGL(k_group_small<K>, dim3(1), dim3(1024), 0, s, in, n, n_keys, k32, rowptr, order, flags);
+    digits(n_keys, SMALL_BITS, &bits, &passes);
+    hipLaunchKernelGGL(k_group_small<K>, dim3(1), dim3(1024), 0, s, in, n, n_keys, bits, passes, k32, rowptr, order,
+                       flags);
     return tace_check_launch("tace_group_keys");
   }
-  int* cnt = work;            // n_keys, then two flags when the caller wants none
-  int* fl = cnt + n_keys;
-  int* place = fl + 2;        // n
-  int* tmp = place + n;       // n
-  int* f = flags ? flags : fl;
-  const unsigned nb = (unsigned)((n + 255) / 256);
-  const int64_t most = n_keys + 2 > n ? (int64_t)n_keys + 2 : n;
-  hipLaunchKernelGGL(k_group_fill, dim3((unsigned)((most + 255) / 256)), dim3(256), 0, s, cnt, (int64_t)n_keys + 2, 0,
-                     tmp, (int64_t)n, -1);
-  if (flags) hipLaunchKernelGGL(k_group_fill, dim3(1), dim3(256), 0, s, flags, (int64_t)2, 0, flags, (int64_t)0, 0);
-  if (n > 0)
-    hipLaunchKernelGGL(k_group_count<K>, dim3(nb), dim3(256), 0, s, in, n, n_keys, k32, cnt, place, f);
-  hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(1024), 0, s, cnt, n_keys, rowptr);
-  if (n > 0) {
-    hipLaunchKernelGGL(k_group_scatter, dim3(nb), dim3(256), 0, s, k32, place, n, rowptr, tmp);
-    hipLaunchKernelGGL(k_group_rank, dim3(nb), dim3(256), 0, s, k32, n, rowptr, tmp, order);
-    if (n > LONG_RANGE)
-      hipLaunchKernelGGL(k_group_long, dim3((unsigned)((n + LONG_RANGE - 1) / LONG_RANGE)), dim3(1024), 0, s, k32, n,
-                         rowptr, tmp, order);
+  digits(n_keys, MAX_BITS, &bits, &passes);
+  const int bins = 1 << bits, nwg = n / CHUNK + (n % CHUNK != 0);
+  // the last pass writes (sorted, order), the ones before it alternate between
+  // that and (keys_b, pos_b); none reads what it writes
+  int* sorted = work;
+  int* keys_b = sorted + n;
+  int* pos_b = keys_b + n;
+  int* hist = pos_b + n;                              // (bins + 2) nwg
+  int* offs = hist + (int64_t)(bins + 2) * nwg;       // (bins + 2) (nwg + 1)
+  const int *keys = k32, *pos = nullptr;
+  if (n == 0 && flags) {   // (the flags of no keys)
+    hipLaunchKernelGGL(k_group_scan, dim3(2), dim3(1024), 0, s, hist, 0, 0, offs, flags);
   }
+  for (int p = 0; p < passes && n > 0; ++p) {
+    const bool last = ((passes - 1 - p) & 1) == 0;
+    int *ko = last ? sorted : keys_b, *po = last ? order : pos_b;
+    if (p == 0)
+      hipLaunchKernelGGL(k_group_first<K>, dim3((unsigned)nwg), dim3(256), 0, s, in, n, n_keys, bins, k32, hist);
+    else
+      hipLaunchKernelGGL(k_group_count, dim3((unsigned)nwg), dim3(256), 0, s, keys, n, p * bits, bins, hist);
+    hipLaunchKernelGGL(k_group_scan, dim3((unsigned)(p == 0 ? bins + 2 : bins)), dim3(1024), 0, s, hist, nwg, bins,
+                       offs, flags);
+    hipLaunchKernelGGL(k_group_scatter, dim3((unsigned)nwg), dim3(256), 0, s, keys, pos, n, n_keys, p * bits, bits,
+                       offs, ko, po);
+    keys = ko;
+    pos = po;
+  }
+  hipLaunchKernelGGL(k_group_rows, dim3((unsigned)(n_keys / 256 + 1)), dim3(256), 0, s, sorted, n, n_keys, rowptr);
   return tace_check_launch("tace_group_keys");
 }
 
 }  // namespace
 
-extern "C" int64_t tace_group_keys_work(int64_t n, int64_t n_keys) { return 2 * n + n_keys + 4; }
+extern "C" int64_t tace_group_keys_work(int64_t n, int64_t n_keys) {
+  // three arrays of n and the counts of MAX_BINS digit values and two flags
+  // per workgroup before and after their scan
+  (void)n_keys;
+  const int64_t nwg = (n + CHUNK - 1) / CHUNK;
+  return 3 * n + (MAX_BINS + 2) * (2 * nwg + 1);
+}
 
 extern "C" int tace_group_keys(int key_bytes, const void* keys, int64_t stride, const int32_t* through, int64_t n,
                                int64_t n_keys, int32_t* keys32, int32_t* rowptr, int32_t* order, const void* other,

@@ -1,0 +1,90 @@
+"""The stable key grouping (``tace_group_keys``): any distribution of the keys gives the stable sort, at the same cost."""
+
+import pytest
+import torch
+
+from tace_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _keys(kind, n, n_keys, seed):
+    g = torch.Generator().manual_seed(seed)
+    k = torch.randint(0, max(n_keys, 1), (n,), generator=g)
+    if kind == "equal":
+        k[:] = n_keys - 1
+    elif kind == "sorted":
+        k = k.sort()[0]
+    elif kind == "hub":
+        k[torch.rand(n, generator=g) < 0.9] = n_keys // 2
+    elif kind == "outside":   # below, just above and far above the range
+        k[torch.rand(n, generator=g) < 0.2] = -1
+        k[torch.rand(n, generator=g) < 0.2] = n_keys
+        k[::7] = 2 ** 31 - 1
+    return k
+
+
+# one workgroup with one and two digits; several with 1 .. 4 digits; keys around
+# a power of two (the value of keys outside the range is n_keys); a workgroup's
+# 2,048 positions, a wavefront's 64 and their remainders
+SHAPES = [(1, 1), (63, 127), (64, 128), (65, 4096), (8192, 4096), (8191, 4095), (8192, 4097), (8193, 1), (2049, 5000), (10240, 4097),
+          (12288, 511), (12289, 512), (20000, 262143), (20001, 262144), (30000, 2 ** 27 + 5), (0, 5000)]
+
+
+@pytest.mark.parametrize("kind", ["even", "equal", "sorted", "hub", "outside"])
+@pytest.mark.parametrize("n,n_keys", SHAPES)
+def test_grouping_equals_stable_sort(cuda, kind, n, n_keys):
+    keys = _keys(kind, n, n_keys, n + n_keys)
+    ok = (keys >= 0) & (keys < n_keys)
+    dev = keys.to(cuda)
+    flags = torch.full((2,), -1, dtype=torch.int32, device=cuda)
+    k32, rp, order, other = ops._group_keys(dev, n_keys, other=dev, flags=flags)
+    assert torch.equal(k32.cpu().long(), torch.where(ok, keys, torch.full_like(keys, -1)))
+    assert torch.equal(other.cpu().long(), keys)
+    last = int(ok.sum())
+    assert int(rp[-1]) == last
+    assert torch.equal(order.cpu().long(), torch.argsort(torch.where(ok, keys, torch.full_like(keys, n_keys)), stable=True))
+    counts = torch.bincount(keys[ok], minlength=min(n_keys, 1 << 20))
+    assert torch.equal(rp[:counts.numel() + 1].cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]))
+    assert flags.tolist() == [int(last < n), int(bool((keys[1:] < keys[:-1]).any()))]
+
+
+def _time(f):
+    """Least of ten passes, in ms."""
+    best = 1e9
+    for _ in range(10):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("n,n_keys", [(8192, 4096), (361000, 13000), (1000000, 16)])
+def test_grouping_costs_the_same_for_any_keys(cuda, n, n_keys):
+    """A counting sort with ranges ranked by comparison took 60 to 150 times as
+    long for equal keys as for even ones, and 30 for sorted few."""
+    t = {kind: _time(lambda k=_keys(kind, n, n_keys, 1).to(cuda): ops.group_by_key(k, n_keys))
+         for kind in ("even", "even", "equal", "sorted", "hub")}
+    even = _time(lambda k=_keys("even", n, 13000, 1).to(cuda): ops.group_by_key(k, 13000))
+    assert max(t.values()) < 5 * even + 0.1, t
+
+
+@pytest.mark.parametrize("E", [ops.GROUP_MAX, ops.GROUP_MAX + 1])
+def test_long_lists_by_the_library_sort(cuda, E):
+    """Both sides of the limit, sender ranges of sorted and of shuffled edges: the same order."""
+    n = 100000
+    dst = torch.arange(E, device=cuda) * n // E
+    src = (dst * 7919 + torch.arange(E, device=cuda) * 104729) % n
+    perm = (torch.arange(E, device=cuda) * 99991) % E
+    perm = perm if perm.unique().numel() == E else torch.arange(E - 1, -1, -1, device=cuda)
+    for e in (torch.stack([src, dst]), torch.stack([src[perm], dst[perm]])):
+        plan = ops.EdgePlan.from_edge_index(e, n)
+        by_slot = plan.src if plan.eid is None else plan.src[plan.eid.long()]
+        rp, slot = plan.sender_csr()
+        assert torch.equal(slot.long(), torch.argsort(by_slot, stable=True))
+        assert torch.equal(rp[1:].long(), torch.bincount(by_slot, minlength=n).cumsum(0))
+        rp2, order = ops.group_by_key(by_slot, n)
+        assert torch.equal(rp, rp2) and torch.equal(slot, order)
