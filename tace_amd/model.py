@@ -1351,8 +1351,9 @@ class TACE(torch.nn.Module):
             w2 = l2.weight.detach() * (l2.lay.ins[0][5] * SILU_CST)
             tab = [t[0].to(x.dtype).contiguous() for t in (self.atomic_energy_layer.atomic_energy, self.scale_shift.scale,
                                                             self.scale_shift.shift)]
-            return ops.EnergyHead.apply(x.contiguous(), sp.inv, w1, w2, attrs.contiguous(), *tab, batch.contiguous(),
-                                        ptr.contiguous(), plan.rowptr)
+            return ops.EnergyHead.apply(x.contiguous(), sp.inv, w1, w2, attrs.contiguous(), *tab,
+                                        batch.to(torch.int64).contiguous(), ptr.to(torch.int64).contiguous(),
+                                        plan.rowptr)
         # E0(Z_n) (OneHotToAtomicEnergy, blocks.py:250-286) as a masked row sum (a
         # [N, S] x [S, 1] product would be a library GEMM launch)
         e_base = (attrs * self.atomic_energy_layer.atomic_energy[0]).sum(-1)
