@@ -926,6 +926,13 @@ def _frozen(*mods: torch.nn.Module) -> bool:
     return not any(p.requires_grad for m in mods for p in m.parameters())
 
 
+def _hooked(m: torch.nn.Module) -> bool:
+    """A hook that a call of the module would run."""
+    glob = torch.nn.modules.module
+    return any(getattr(o, pre + h) for o, pre in ((m, "_"), (glob, "_global_"))
+               for h in ("forward_hooks", "forward_pre_hooks", "backward_hooks", "backward_pre_hooks"))
+
+
 class _SharedInputLinearsFn(torch.autograd.Function):
     """Two linears of one input as one autograd node (the interaction's
     linear_up and its resnet linear, ``inter.py:212-227``): the second's input
@@ -1324,12 +1331,21 @@ class TACE(torch.nn.Module):
 
     def _head_fits(self, x, attrs, plan, sp) -> bool:
         """Whether the readout, the element tables and the per-graph sums run
-        on ``ops.EnergyHead``: frozen parameters, one hidden layer of 16, and a
-        receiver CSR over exactly these nodes."""
-        lin = self.energy_readouts[0].linear2
-        return (x.is_cuda and not (ops.MODE.double or ops.MODE.export) and x.dtype in (torch.float32, torch.float64)
-                and attrs.dtype == x.dtype and not attrs.requires_grad and _frozen(self.energy_readouts[0])
-                and len(lin) == 2 and lin[0].weight.numel() == 16 * x.shape[1] and lin[1].weight.numel() == 16
+        on ``ops.EnergyHead``: the readout built here, one hidden layer of 16,
+        and nothing that would notice that its modules are not called or that
+        only x gets a gradient; a receiver CSR over exactly these nodes."""
+        readout = self.energy_readouts[0]
+        if type(readout) is not ScalarReadOut or ops.MODE.double or ops.MODE.export or not x.is_cuda:
+            return False
+        lin = readout.linear2
+        mods = [readout, *lin]
+        consts = [attrs, self.atomic_energy_layer.atomic_energy, self.scale_shift.scale, self.scale_shift.shift]
+        return (len(lin) == 2 and all(type(m) is e3nnLinear and m.bias is None for m in lin)
+                and not any("forward" in vars(m) or _hooked(m) for m in mods) and _frozen(readout)
+                and lin[0].weight.numel() == 16 * x.shape[1] and lin[1].weight.numel() == 16
+                and x.dtype in (torch.float32, torch.float64)
+                and all(t.dtype == x.dtype and t.device == x.device and not t.requires_grad
+                        for t in consts + [m.weight for m in lin])
                 and x.shape[1] <= 512 and 0 < x.shape[0] == attrs.shape[0] and sp.inv is not None
                 and isinstance(plan, ops.EdgePlan) and plan.n_nodes == x.shape[0])
 
@@ -1349,8 +1365,8 @@ class TACE(torch.nn.Module):
             l1, l2 = self.energy_readouts[0].linear2
             w1 = l1.weight.detach().view(x.shape[1], 16) * l1.lay.ins[0][5]
             w2 = l2.weight.detach() * (l2.lay.ins[0][5] * SILU_CST)
-            tab = [t[0].to(x.dtype).contiguous() for t in (self.atomic_energy_layer.atomic_energy, self.scale_shift.scale,
-                                                            self.scale_shift.shift)]
+            tab = [t[0].contiguous() for t in (self.atomic_energy_layer.atomic_energy, self.scale_shift.scale,
+                                               self.scale_shift.shift)]
             return ops.EnergyHead.apply(x.contiguous(), sp.inv, w1, w2, attrs.contiguous(), *tab,
                                         batch.to(torch.int64).contiguous(), ptr.to(torch.int64).contiguous(),
                                         plan.rowptr)

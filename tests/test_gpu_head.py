@@ -44,3 +44,104 @@ def test_int32_batch_and_ptr(cuda, keys, monkeypatch):
         assert torch.equal(got[k], want[k]), k
     # (a ptr of 32 bits has the lattice gradient summed edge by edge)
     assert (got["stress"] - want["stress"]).abs().max() <= 1e-5 * want["stress"].abs().max()
+
+
+def _energy(model, g):
+    """(energy, node energies) of the readout function alone, and the edge vectors."""
+    vec = pm.ops.edge_vectors(g["positions"], g["lattice"], g["edge_shifts"].to(g["positions"].dtype), g["_edge_plan"],
+                              g["_dst32"], g["batch"][g["edge_index"][0]]).requires_grad_(True)
+    return *model.readout_fn.energy(g, g["_edge_plan"], vec), vec
+
+
+def _same(a, b):
+    """Two float32 routes: sums of at most 32 products and 17 nodes in another order."""
+    return all((u.double() - v.double()).abs().max() <= 1e-5 * v.abs().max() for u, v in zip(a, b))
+
+
+@pytest.mark.parametrize("where", ["readout", "hidden", "last", "global"])
+@pytest.mark.parametrize("kind", ["pre", "post", "back"])
+def test_hooks_on_the_readout_run(cuda, where, kind, monkeypatch):
+    model, g = _batch(cuda)
+    want = model(g)
+    readout = model.readout_fn.energy_readouts[0]
+    seen = []
+    hook = lambda m, *a: seen.append(m) if m in (readout, *readout.linear2) else None
+    if where == "global":
+        reg = {"pre": torch.nn.modules.module.register_module_forward_pre_hook,
+               "post": torch.nn.modules.module.register_module_forward_hook,
+               "back": torch.nn.modules.module.register_module_full_backward_hook}[kind]
+    else:
+        m = {"readout": readout, "hidden": readout.linear2[0], "last": readout.linear2[1]}[where]
+        reg = {"pre": m.register_forward_pre_hook, "post": m.register_forward_hook,
+               "back": m.register_full_backward_hook}[kind]
+    handle = reg(hook)
+    try:
+        got = model(g)
+    finally:
+        handle.remove()
+    assert seen
+    assert _same([got["energy"], got["forces"]], [want["energy"], want["forces"]])
+    calls = _head_calls(monkeypatch)   # the kernel again without the hook
+    assert torch.equal(model(g)["energy"], want["energy"]) and calls
+
+
+@pytest.mark.parametrize("name", ["scale_shift.scale", "scale_shift.shift", "atomic_energy_layer.atomic_energy"])
+def test_element_tables_get_their_gradient(cuda, name):
+    """A table that takes a gradient: against the sums over each species' nodes."""
+    model, g = _batch(cuda, torch.float64)
+    fn = model.readout_fn
+    mod, buf = fn.get_submodule(name.split(".")[0]), name.split(".")[1]
+    t = getattr(mod, buf).clone().requires_grad_(True)
+    E0, en0, _ = _energy(model, g)
+    setattr(mod, buf, t)
+    E, en, _ = _energy(model, g)
+    (gt,) = torch.autograd.grad(E.sum(), t)
+    assert (E - E0).abs().max() < 1e-12 * E0.abs().max() and (en - en0).abs().max() < 1e-12 * en0.abs().max()
+    alone = torch.arange(len(en), device=cuda) == 26   # the atom alone in its cell
+    attrs = g["node_attrs"]
+    base = (attrs * fn.atomic_energy_layer.atomic_energy[0]).sum(-1)
+    if buf == "shift":
+        want = attrs[~alone].sum(0)
+    elif buf == "atomic_energy":
+        want = attrs.sum(0)
+    else:
+        sc, sh = ((attrs * v[0]).sum(-1) for v in (fn.scale_shift.scale, fn.scale_shift.shift))
+        want = (attrs * ((en - base - sh) / sc).unsqueeze(1))[~alone].sum(0)
+    assert (gt[0] - want).abs().max() < 1e-10 * want.abs().max().clamp_min(1.0)
+
+
+def test_readout_of_another_make_is_called(cuda):
+    """A module put in the readout's place, a readout whose forward was set, a
+    linear of a subclass: all are called; a table of another type keeps its
+    precision."""
+    model, g = _batch(cuda)
+    fn = model.readout_fn
+    E0, en0, _ = _energy(model, g)
+    own = fn.energy_readouts[0]
+
+    class Twice(torch.nn.Module):
+        def forward(self, x):
+            return 2 * own(x)
+
+    scale, shift = ((g["node_attrs"] * v[0]).sum(-1) for v in (fn.scale_shift.scale, fn.scale_shift.shift))
+    base = (g["node_attrs"] * fn.atomic_energy_layer.atomic_energy[0]).sum(-1)
+    alone = torch.arange(len(en0), device=cuda) == 26
+    twice = torch.where(alone, en0, 2 * (en0 - base) - shift + base)
+    fn.energy_readouts[0] = Twice()
+    assert _same([_energy(model, g)[1]], [twice])
+    fn.energy_readouts[0] = own
+    own.forward = lambda x: 2 * type(own).forward(own, x)
+    assert _same([_energy(model, g)[1]], [twice])
+    del own.forward
+
+    class Other(pm.e3nnLinear):
+        def forward(self, x, alpha=1.0):
+            return 2 * super().forward(x, alpha)
+
+    own.linear2[1].__class__ = Other
+    assert _same([_energy(model, g)[1]], [twice])
+    own.linear2[1].__class__ = pm.e3nnLinear
+    fn.atomic_energy_layer.double()
+    E, en, _ = _energy(model, g)
+    assert E.dtype == en.dtype == torch.float64 and _same([E, en], [E0, en0])
+
