@@ -837,6 +837,14 @@ def uuu_tp(x1, x2, var: TpVariant, C: int, layout: int = 0, w: Optional[torch.Te
 
 
 # ------------------------------------------------------------ gate, readout ----
+def first_order_only(what: str) -> None:
+    """Called in a backward whose kernel leaves no graph behind it: raises
+    where a graph of the gradients is asked for (``create_graph``)."""
+    if torch.is_grad_enabled():
+        raise RuntimeError(f"{what}: no second derivative in the inference form of the operators; evaluate inside "
+                           "ops.differentiable_twice()")
+
+
 def launch_gate_fwd(x: torch.Tensor, C: int, n_blocks: int, cst: float) -> torch.Tensor:
     """``tace_gate_fwd`` on group-major x [n, C (n_blocks + n_blocks^2)]."""
     n = x.shape[0]
@@ -889,6 +897,7 @@ class EnergyHead(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gE, gn):
+        first_order_only("the energy readout")
         if gE is None and gn is None:
             return (None,) * 11
         hid, fac, row_of, batch, w1 = ctx.saved_tensors
