@@ -1988,6 +1988,12 @@ SEG_SPLIT_MAX_WORK = 384
 # 1565
 SEG_STREAM_BYTES = 256 << 20
 SEG_STREAM_STEPS = 84
+# a split launch holds one 64 KB partial tile per split of each of its tiles;
+# plans with more than about this many bytes of them run as several launches,
+# one after another through the same partial tiles.  89 species, 256 channels:
+# 0.45 GB at 5,003 nodes and 6.9 GB at 100,000 in one launch.  The product layer
+# at 5,003 nodes, us: 64 MB 8,712, 128 MB 8,668, 256 MB 8,645, one launch 8,652
+SEG_PARTIAL_BYTES = 256 << 20
 
 
 def seg_split_count(n_work: int, nks_min: int, nks_max: int) -> int:
@@ -2150,13 +2156,21 @@ class SegLinearPlan:
         if len(t) and len(c):
             ksum = np.concatenate([[0], np.cumsum(c[:, 1])])
             self.flops = int(2 * (t[:, 1] * np.minimum(TN, t[:, 2] - t[:, 3]) * (ksum[t[:, 6]] - ksum[t[:, 5]])).sum())
-        if self.tile_frag and 8 % self.splits == 0 and len(t) >= SEG_BALANCE_MIN:
+        # equal runs of the tiles, one launch each (one launch unless split)
+        most = max(1, SEG_PARTIAL_BYTES // (65536 * self.splits)) if self.splits > 1 else max(1, len(t))
+        parts = np.array_split(t, max(1, -(-len(t) // most)))
+        if self.tile_frag and 8 % self.splits == 0:
             # a tile costs its 32-k steps (and about four for its start and
             # stores) per 64 rows
             steps = np.concatenate([[0], np.cumsum((c[:, 1] + 31) // 32)])
-            steps = steps[t[:, 6]] - steps[t[:, 5]] + 4
-            t = _xcd_balanced(t, steps * ((t[:, 1] + 63) // 64), steps, 8 // self.splits)
-            self.n_tiles = len(t)
+            for i, u in enumerate(parts):
+                if len(u) >= SEG_BALANCE_MIN:
+                    length = steps[u[:, 6]] - steps[u[:, 5]] + 4
+                    parts[i] = _xcd_balanced(u, length * ((u[:, 1] + 63) // 64), length, 8 // self.splits)
+        first = np.cumsum([0] + [len(u) for u in parts])
+        self.launches = [(int(a), int(b - a)) for a, b in zip(first, first[1:])]   # (first tile, tiles)
+        t = np.concatenate(parts)
+        self.n_tiles = len(t)
         self.tiles = torch.from_numpy(np.ascontiguousarray(t)).to(device)
         self.contribs = torch.from_numpy(np.ascontiguousarray(c) if len(c) else np.zeros((1, 4), np.int64)).to(device)
         self.scales = torch.from_numpy(s if len(s) else np.zeros(1)).to(device)
@@ -2336,12 +2350,12 @@ def seg_linear_presplit(x: torch.Tensor, y: torch.Tensor, planes: Optional[torch
     b_ptr = None if bias is None else bias.data_ptr()
     a_ptr = _addend_ptr(addend, y)
     if plan.tile_frag and plan.splits > 1:
-        pe = plan.n_tiles * plan.splits * 16384
+        pe = max(n for _, n in plan.launches) * plan.splits * 16384
         partials = torch.empty(pe, dtype=torch.float32, device=x.device)
-        N.check(N.lib().tace_seg_linear_presplit_frag_split(x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr,
-                                                            plan.tiles.data_ptr(), plan.n_tiles,
-                                                            plan.contribs.data_ptr(), int(plan.tile_aligned),
-                                                            plan.splits, partials.data_ptr(), pe, float(alpha), st),
+        for t0, n_t in plan.launches:
+            N.check(N.lib().tace_seg_linear_presplit_frag_split(
+                x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr, plan.tiles[t0:t0 + n_t].data_ptr(), n_t,
+                plan.contribs.data_ptr(), int(plan.tile_aligned), plan.splits, partials.data_ptr(), pe, float(alpha), st),
                 "tace_seg_linear_presplit_frag_split")
     elif plan.tile_frag:
         N.check(N.lib().tace_seg_linear_presplit_frag(x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr,
