@@ -2041,6 +2041,12 @@ def _xcd_balanced(table: np.ndarray, cost: np.ndarray, length: np.ndarray, runs:
     return out
 
 
+def seg_settings() -> tuple:
+    """Every setting that decides a ``SegLinearPlan`` (part of a plan cache's key)."""
+    return (SEG_KS_MIN_N, tuple(sorted(SEG_KS_CHUNK.items())), SEG_TILE_FRAG, SEG_SPLIT_SLOTS, SEG_SPLIT_MIN_STEPS,
+            SEG_SPLIT_MAX_WORK, SEG_STREAM_BYTES, SEG_STREAM_STEPS, SEG_PARTIAL_BYTES, SEG_BALANCE_MIN)
+
+
 class SegLinearPlan:
     """Device tables of ``tace_seg_linear`` for one direction of one
     per-species linear over one set of species row ranges.

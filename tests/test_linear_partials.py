@@ -30,6 +30,27 @@ def test_partial_tiles_are_bounded(n):
     assert covered == n * 256 * 16 and len(np.unique(rows[:, [0, 3]], axis=0)) == len(rows)
 
 
+@pytest.mark.parametrize("name,value", [
+    ("SEG_KS_MIN_N", None), ("SEG_KS_CHUNK", {128: 256, 256: 1024}), ("SEG_TILE_FRAG", False), ("SEG_SPLIT_SLOTS", None),
+    ("SEG_SPLIT_MIN_STEPS", 2), ("SEG_SPLIT_MAX_WORK", 0), ("SEG_STREAM_BYTES", 1 << 10), ("SEG_STREAM_STEPS", 4),
+    ("SEG_PARTIAL_BYTES", 1 << 16), ("SEG_BALANCE_MIN", 1)])
+def test_a_changed_setting_makes_another_plan(name, value, monkeypatch):
+    lay = pm._LinearLayout(pm.Irreps("600x0e+90x1o"), pm.Irreps("160x0e+300x1o"))
+    w, x = torch.empty(2, lay.weight_numel, device="meta"), torch.empty(0)
+    rr = [(0, 0, 70), (1, 70, 200)]
+    make = lambda: lay.seg_plan("fwd", rr, 200, x, w, None)
+    first = make()
+    assert make() is first
+    with monkeypatch.context() as m:
+        m.setattr(ops, name, value)
+        assert make() is not first
+    assert make() is first
+    # the settings the plan reads, and no others
+    assert {n for n in vars(ops) if n.startswith("SEG_")} == {"SEG_KS_MIN_N", "SEG_KS_CHUNK", "SEG_TILE_FRAG", "SEG_SPLIT_SLOTS",
+            "SEG_SPLIT_MIN_STEPS", "SEG_SPLIT_MAX_WORK", "SEG_STREAM_BYTES", "SEG_STREAM_STEPS", "SEG_PARTIAL_BYTES",
+            "SEG_BALANCE_MIN"}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tiles", [1, 7, 64, 100])
 def test_several_launches_give_the_bits_of_one(cuda, tiles, monkeypatch):
@@ -50,7 +71,6 @@ def test_several_launches_give_the_bits_of_one(cuda, tiles, monkeypatch):
     res = []
     for limit in (1 << 40, tiles * 4 * 65536):
         monkeypatch.setattr(ops, "SEG_PARTIAL_BYTES", limit)
-        lin.lay._seg.clear()
         y = pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.9, out=None, addend=add)
         z = add.clone()
         pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.9, out=z, addend=z)
