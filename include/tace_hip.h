@@ -40,7 +40,8 @@
 extern "C" {
 #endif
 
-#define TACE_HIP_ABI_VERSION 32
+/* raised with every change of a prototype or of what an argument means */
+#define TACE_HIP_ABI_VERSION 33
 #define TACE_MAX_CHANNELS 512
 #define TACE_F32 0
 #define TACE_F64 1
@@ -635,10 +636,10 @@ int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, vo
  * receivers, and bincount + cumsum): key i is keys[(through ? through[i] : i)
  * * stride], of key_bytes 4 or 8.  keys32 [n]: the keys (-1 outside [0,
  * n_keys)); rowptr [n_keys + 1] and order [n]: the positions in key order,
- * ascending within a key (positions with a key outside the range take no
- * part).  other (may be NULL): n more keys, other[i * other_stride], checked
- * against the same range and converted into other32 [n] (an edge list's
- * senders).  flags (int32 [2], may be NULL): [0] nonzero if some key or other
+ * ascending within a key (positions with a key outside the range come after
+ * all others, outside every range of rowptr).  other (may be NULL): n more
+ * keys, other[i * other_stride], checked against the same range and converted
+ * into other32 [n] (an edge list's senders).  flags (int32 [2], may be NULL): [0] nonzero if some key or other
  * key is outside the range, [1] if the keys are not ascending.  work:
  * tace_group_keys_work int32. */
 int64_t tace_group_keys_work(int64_t n, int64_t n_keys);

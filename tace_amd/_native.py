@@ -15,6 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libtace_hip.so")
 
 F32, F64 = 0, 1
+ABI_VERSION = 33   # TACE_HIP_ABI_VERSION of the signatures below
 
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
@@ -140,6 +141,10 @@ def lib() -> ctypes.CDLL:
                         f"libtace_hip.so not found at {LIB_PATH}; build it with "
                         "`python -m tace_amd.build` (hipcc, gfx950)")
                 L = ctypes.CDLL(LIB_PATH)
+                got = L.tace_abi_version()
+                if got != ABI_VERSION:
+                    raise NativeError(f"{LIB_PATH} has ABI version {got}, these bindings are for {ABI_VERSION}; "
+                                      "build it again with `python -m tace_amd.build`")
                 for name, (res, args) in _SIGS.items():
                     f = getattr(L, name)
                     f.restype = res
