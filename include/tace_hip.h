@@ -331,8 +331,8 @@ int tace_seg_linear_presplit(const float* x, float* y, const float* addend, cons
  * (tace_seg_linear_ks_rows(k): the height for k, 0 when not supported),
  * each over a column range, with the weights split in MFMA fragment order
  * (tace_bf16x3_split_blocks layout 1).  k_max is 128 or 256: every task's k is
- * at most that, and a task whose k exceeds it gets NaN in every output of its
- * tile:
+ * at most that, and a task whose k exceeds it, or of more than 64 rows, gets
+ * NaN in every output of its tile:
  *   tasks int64 [n_tasks, 10]: out_base (offset of the tile's row 0, column 0
  *         in y), rows (1..64), n (block width = row stride of y), cb, ce (its
  *         columns [cb, ce), ce <= n), bias_off (-1 none), x_base (offset of
