@@ -396,7 +396,7 @@ def sub_plan(plan: ops.EdgePlan, n0: int, n1: int, e0: int, e1: int) -> ops.Edge
 # ----------------------------------------------------------- fused operator --
 # bf16 channel mixing: SO(2) GEMMs on tace_so2_gemm_bf16 / _kt (bias in the
 # epilogue) where they measured faster than the library GEMM on fe101k
-# (_so2_route); False: torch.mm / addmm (addmm copies the bias into the output
+# (``_so2_route``); False: torch.mm / addmm (addmm copies the bias into the output
 # and accumulates onto it); SO2_GEMM_ALL: every shape on the hand-written ones
 SO2_GEMM = True
 SO2_GEMM_ALL = False
@@ -404,8 +404,7 @@ SO2_GEMM_ALL = False
 
 # kernel per SO(2) GEMM shape (k, n, biased) under bf16 mixing: "kt" =
 # tace_so2_gemm_bf16_kt (A through LDS in 64-k stages, 128 x 256 tiles), "lds"
-# = tace_so2_gemm_bf16 (a row tile's whole k in LDS), None = the library
-# (torch.mm / addmm).  Measured per call on the fe101k chunk shapes (2^20
+# = tace_so2_gemm_bf16 (a row tile's whole k in LDS).  Measured per call on the fe101k chunk shapes (2^20
 # edges: block 0 has 1 M rows, blocks m > 0 2 M), library / lds / kt in ms:
 #   biased:   384->384 1.22 / 0.77 / 0.72, 768->1152 3.90 / 3.06 / 2.52,
 #             96->384 0.90 / 0.37 / 0.74
@@ -430,8 +429,7 @@ _SO2_TABLE = {
 
 
 def _so2_route(k: int, n: int, bias: bool):
-    """Kernel for the SO(2) GEMM [rows, k] x [k, n] (+ bias): "kt", "lds" or
-    None (the library); see _SO2_TABLE."""
+    """Kernel for the SO(2) GEMM [rows, k] x [k, n] (+ bias): "kt" or "lds"; see _SO2_TABLE."""
     if SO2_GEMM_ALL:
         return "kt" if k >= 256 else "lds"
     key = (k, n, bool(bias))
@@ -448,18 +446,14 @@ F32_GEMM = True
 
 
 class _Operand:
-    """One right GEMM operand [k, n] of the fused operator: ``frag``, its copy
-    in MFMA fragment order (bf16 or three bf16 terms, None in float64), and
-    ``plain()``, the matrix itself for the library."""
+    """One right GEMM operand [k, n] of the fused operator, as one of ``frag``,
+    its copy in MFMA fragment order (bf16 or three bf16 terms), and ``plain``,
+    the matrix itself for the library.  Both are copies made in the forward:
+    the backward's products are with the weights of its forward."""
 
-    def __init__(self, k: int, n: int, plain):
-        self.k, self.n, self.frag = k, n, None
-        self._plain, self._made = plain, None
-
-    def plain(self) -> torch.Tensor:
-        if self._made is None:
-            self._made = self._plain()
-        return self._made
+    def __init__(self, k: int, n: int, make):
+        self.k, self.n, self.make = k, n, make
+        self.frag = self.plain = None
 
 
 class _FusedParams:
@@ -515,6 +509,8 @@ class _FusedParams:
         self.mlp_layers = len(lins) - 1
         self.mlp_W = lins[-1].weight.detach().to(dtype).contiguous()
         self.mlp_alpha = float(lins[-1].alpha)
+        if dtype != torch.float32 or self.mlp_W.shape[1] % 4:   # (else the backward's kernel takes mlp_W)
+            self.mlp_WT = (lins[-1].weight.detach() * lins[-1].alpha).to(dtype).t().contiguous()
         biases = [lin.m0_rlinear.bias for lin in shared]
         nr, no = rp.weight.shape[1], rp.weight.shape[0]
         floats = [("s_b", [(v, v.numel(), 1.0) for v in biases], 1, sum(v.numel() for v in biases), False, 1, 1),
@@ -523,9 +519,17 @@ class _FusedParams:
                   ("rp_T", [(rp.weight, no, rp.alpha)], nr, no, False, 1, nr),
                   ("rp_N", [(rp.weight, no, rp.alpha)], no, nr, True, 0, nr)]
         params = [w for _, segs, _ in gemms[::2] for w, _, _ in segs] + [w for f in floats for w, _, _ in f[1]]
-        if dtype == torch.float32 and all(p.is_cuda and p.dtype == dtype and p.is_contiguous() for p in params):
+        kernels = SO2_GEMM if self.bf16 else F32_GEMM
+        if (kernels and dtype == torch.float32
+                and all(p.is_cuda and p.dtype == dtype and p.is_contiguous() for p in params)):
             self._layout(conv, gemms, floats, params)
             return
+        for o, _, _ in gemms:
+            m = o.make()
+            if kernels and self.bf16:
+                o.frag = ops.bf16_fragment_order(m)
+            else:
+                o.plain = m
         self.s_b = torch.cat([v.detach() for v in biases]).to(dtype).contiguous()
         Wrp = (rp.weight * rp.alpha).detach().to(dtype)
         self.rp_T, self.rp_N = Wrp.t().contiguous(), Wrp.contiguous()
@@ -566,17 +570,12 @@ class _FusedParams:
     def mm(self, x, B: _Operand, b=None):
         """x @ B (+ b): bf16 operands with float32 accumulation and output
         under bf16 mixing, else in the features' precision."""
-        if self.bf16:
-            r = _so2_route(B.k, B.n, b is not None) if SO2_GEMM else None
-            if r is not None and x.dtype == torch.bfloat16:
-                frag = B.frag if B.frag is not None else ops.bf16_fragment_order(B.plain())
-                return ops.so2_gemm_bf16(x, frag, B.n, B.k, b, ktiled=r == "kt")
-            if b is None:
-                return torch.mm(x, B.plain(), out_dtype=torch.float32)
-            return torch.addmm(b, x, B.plain(), out_dtype=torch.float32)
-        if F32_GEMM and B.frag is not None:
+        if B.frag is not None:
+            if self.bf16:
+                return ops.so2_gemm_bf16(x, B.frag, B.n, B.k, b, ktiled=_so2_route(B.k, B.n, b is not None) == "kt")
             return ops.gemm_bx3(x, B.frag, B.n, B.k, b)
-        return torch.mm(x, B.plain()) if b is None else torch.addmm(b, x, B.plain())
+        out = dict(out_dtype=torch.float32) if self.bf16 else {}
+        return torch.mm(x, B.plain, **out) if b is None else torch.addmm(b, x, B.plain, **out)
 
     mm_grad = mm
 
@@ -650,7 +649,7 @@ def _fused_chunk_bwd(P: _FusedParams, x_lc, R, W, rs, rd, plan: ops.EdgePlan, ou
     if gw.dtype == torch.float32 and gw.shape[1] % 4 == 0:
         gh = ops.launch_mlp_out_bwd_f32(gw, P.mlp_W, P.mlp_alpha)
     else:
-        gh = torch.mm(gw, P.mlp_W.t()).mul_(P.mlp_alpha)
+        gh = torch.mm(gw, P.mlp_WT)
     gR = torch.add(gR, ops.launch_mlp_hidden_bwd(R, gh, P.mlp_flat, P.mlp_layers), out=gR_out)
     return gR, gW
 
