@@ -41,7 +41,7 @@ extern "C" {
 #endif
 
 /* raised with every change of a prototype or of what an argument means */
-#define TACE_HIP_ABI_VERSION 33
+#define TACE_HIP_ABI_VERSION 34
 #define TACE_MAX_CHANNELS 512
 #define TACE_F32 0
 #define TACE_F64 1
@@ -622,15 +622,17 @@ int tace_edge_index(const int32_t* rowptr, const int32_t* src, int64_t n_nodes, 
  * tace_bf16x3_split_blocks layout 1), 16-byte aligned; x and y row-major. */
 int tace_gemm_bx3(const float* x, const uint16_t* w_frag, const float* bias, float* y, int64_t m, int32_t n, int32_t k,
                   void* stream);
-/* Several GEMM operands B [k, n] laid out from float32 weights in one launch.
- * table: 20 x int64 per operand on the device: kind (0 bf16 in MFMA fragment
+/* Several GEMM operands B [k, n] laid out from float32 weights, up to 24 in one
+ * launch.  table: 20 x int64 per operand in host memory, read before the call
+ * returns: kind (0 bf16 in MFMA fragment
  * order, 1024 ceil(k/32) ceil(n/16) bytes; 1 its three terms, three times
  * that; 2 float32 row-major), k, n, byte offset in out (a multiple of 16),
  * number of segments (1..4), axis (0: segments stacked along n, 1: along k),
  * trans (B[kk][c] = W[c][kk], else W[kk][c]), row stride of every W, then per
  * segment the device address of W, its length along the axis and its scale as
- * a double's bits.  Values are scaled in float32, then rounded or split. */
-int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, void* stream);
+ * a double's bits.  Values are scaled in float32, then rounded or split.  An
+ * operand that would end past out_bytes is refused. */
+int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, int64_t out_bytes, void* stream);
 
 /* Positions 0 .. n-1 grouped by key (torch.argsort(stable=True) of the
  * receivers, and bincount + cumsum): key i is keys[(through ? through[i] : i)

@@ -15,7 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "libtace_hip.so")
 
 F32, F64 = 0, 1
-ABI_VERSION = 33   # TACE_HIP_ABI_VERSION of the signatures below
+ABI_VERSION = 34   # TACE_HIP_ABI_VERSION of the signatures below
 
 _lib: Optional[ctypes.CDLL] = None
 _lock = threading.Lock()
@@ -110,7 +110,7 @@ _SIGS = {
     "tace_radial_mlp_fwd_scaled": (_c_int, [_vp, _c_i64, _c_i32, _c_i32, _vp, _vp, _vp, _vp, _vp]),
     "tace_edge_index": (_c_int, [_vp, _vp, _c_i64, _c_i64, _vp, _vp, _vp]),
     "tace_gemm_bx3": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _c_i32, _c_i32, _vp]),
-    "tace_layout_operands": (_c_int, [_vp, _c_i64, _vp, _vp]),
+    "tace_layout_operands": (_c_int, [_vp, _c_i64, _vp, _c_i64, _vp]),
     "tace_group_keys_work": (_c_i64, [_c_i64, _c_i64]),
     "tace_group_keys": (_c_int, [_c_int, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp,
                                  _vp]),

@@ -24,6 +24,7 @@
 // written, by the lane that writes it.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #include "../../include/tace_hip.h"
 #include "bf16x3.h"
@@ -1200,7 +1201,9 @@ __global__ __launch_bounds__(256) void k_split_blocks(const float* __restrict__ 
 // W[c][kk], else W[kk][c]), row stride of every W, then per segment its
 // address, its length along the axis and its scale (a double's bits).  A
 // thread makes the eight values of one lane's fragment (or one float), so its
-// stores are 16 bytes; blockIdx.y picks the operand.
+// stores are 16 bytes; blockIdx.y picks the operand.  The operands come as a
+// kernel argument, 24 a launch: a launch, recorded or not, holds its own, and
+// no address is kept in memory between calls.
 struct OpDesc {
   int64_t d[20];
 
@@ -1224,11 +1227,13 @@ struct OpDesc {
   }
 };
 
-__global__ __launch_bounds__(256) void k_layout_operands(const int64_t* __restrict__ table,
-                                                         unsigned char* __restrict__ out) {
-  OpDesc o;   // uniform: in scalar registers
-#pragma unroll
-  for (int i = 0; i < 20; ++i) o.d[i] = table[20 * (int64_t)blockIdx.y + i];
+constexpr int OPS_LAUNCH = 24;
+struct OpTable {   // 3,840 bytes
+  OpDesc op[OPS_LAUNCH];
+};
+
+__global__ __launch_bounds__(256) void k_layout_operands(const OpTable table, unsigned char* __restrict__ out) {
+  const OpDesc& o = table.op[blockIdx.y];   // uniform: in scalar registers
   const int kind = (int)o.d[0], k = (int)o.d[1], n = (int)o.d[2];
   unsigned char* dst = out + o.d[3];
   if (kind == 2) {
@@ -1258,14 +1263,38 @@ __global__ __launch_bounds__(256) void k_layout_operands(const int64_t* __restri
 
 }  // namespace
 
-extern "C" int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, void* stream) {
+extern "C" int tace_layout_operands(const int64_t* table, int64_t n_operands, void* out, int64_t out_bytes,
+                                    void* stream) {
   if (n_operands < 0 || n_operands > 65535) return tace_fail_msg("tace_layout_operands: 0..65535 operands");
   if (n_operands == 0) return 0;
   if (!table || !out || (((uintptr_t)out) & 15) != 0)
     return tace_fail_msg("tace_layout_operands: null or misaligned pointer");
-  hipLaunchKernelGGL(k_layout_operands, dim3(64, (unsigned)n_operands), dim3(256), 0, (hipStream_t)stream, table,
-                     (unsigned char*)out);
-  return tace_check_launch("tace_layout_operands");
+  for (int64_t i = 0; i < n_operands; ++i) {
+    const int64_t* d = table + 20 * i;
+    if (d[0] < 0 || d[0] > 2 || d[1] <= 0 || d[2] <= 0 || d[1] > 0xffffff || d[2] > 0xffffff || d[4] < 1 || d[4] > 4 ||
+        d[5] < 0 || d[5] > 1 || d[3] < 0 || (d[3] & 15) != 0)
+      return tace_fail_msg("tace_layout_operands: bad operand");
+    const int64_t frag = 1024 * ((d[1] + 31) / 32) * ((d[2] + 15) / 16);
+    if (d[3] + (d[0] == 0 ? frag : d[0] == 1 ? 3 * frag : 4 * d[1] * d[2]) > out_bytes)
+      return tace_fail_msg("tace_layout_operands: an operand ends past out");
+    int64_t along = 0;
+    for (int64_t s = 0; s < d[4]; ++s) {
+      if (!d[8 + 3 * s] || d[9 + 3 * s] <= 0) return tace_fail_msg("tace_layout_operands: bad segment");
+      along += d[9 + 3 * s];
+    }
+    if (along != (d[5] == 0 ? d[2] : d[1]))
+      return tace_fail_msg("tace_layout_operands: the segments are not the operand's length");
+  }
+  for (int64_t i = 0; i < n_operands; i += OPS_LAUNCH) {
+    OpTable t;
+    const int m = (int)(n_operands - i < OPS_LAUNCH ? n_operands - i : OPS_LAUNCH);
+    memset(&t, 0, sizeof(t));
+    memcpy(&t, table + 20 * i, sizeof(OpDesc) * m);
+    hipLaunchKernelGGL(k_layout_operands, dim3(64, (unsigned)m), dim3(256), 0, (hipStream_t)stream, t,
+                       (unsigned char*)out);
+    if (int rc = tace_check_launch("tace_layout_operands")) return rc;
+  }
+  return 0;
 }
 
 extern "C" int tace_bf16x3_split_blocks(const float* w, const int64_t* blocks, const double* scales,

@@ -1283,12 +1283,16 @@ def so2_gemm_bf16(a: torch.Tensor, b_frag: torch.Tensor, n: int, k: int,
     return out
 
 
-def layout_operands(table: torch.Tensor, nbytes: int) -> torch.Tensor:
-    """The operands of ``tace_layout_operands``' table [n, 20] (int64, on the
-    GPU, whose addresses the caller keeps alive) in one new buffer of bytes."""
-    _req(table, "table", torch.int64, (table.shape[0], 20))
-    out = torch.empty(nbytes, dtype=torch.uint8, device=table.device)
-    N.check(N.lib().tace_layout_operands(table.data_ptr(), table.shape[0], out.data_ptr(), N.stream_ptr(table.device)),
+def layout_operands(table: torch.Tensor, nbytes: int, device=None) -> torch.Tensor:
+    """The operands of ``tace_layout_operands``' table [n, 20] (int64; on the
+    host, or copied there from the GPU whose addresses it holds) in one new
+    buffer of bytes on ``device`` (the table's, if it is on a GPU)."""
+    dev = table.device if device is None else torch.device(device)
+    t = table.cpu()
+    if t.dtype != torch.int64 or t.dim() != 2 or t.shape[1] != 20 or not t.is_contiguous():
+        raise ValueError("layout operands: the table must be a contiguous int64 [n, 20] tensor")
+    out = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    N.check(N.lib().tace_layout_operands(t.data_ptr(), t.shape[0], out.data_ptr(), nbytes, N.stream_ptr(dev)),
             "tace_layout_operands")
     return out
 

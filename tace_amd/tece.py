@@ -17,6 +17,7 @@ features come and go in the model's group-major, species-sorted layout.
 
 from __future__ import annotations
 
+import array
 import math
 import struct
 from typing import List, Optional
@@ -462,12 +463,10 @@ class _FusedParams:
     W (input-gradient operand), the biases, the radial projection, the
     attention scale and the radial MLP.
 
-    In float32 one launch (``tace_layout_operands``) reads every weight and
-    writes all operands, in the fragment order of the mixing precision's GEMM
+    In float32 two launches (``tace_layout_operands``) read every weight and
+    write all operands, in the fragment order of the mixing precision's GEMM
     kernel; made by torch operations they took about 130 launches a forward.
-    Only the table of addresses and sizes is kept between calls (on the
-    convolution, for the addresses it was made from); the weights are read
-    every time."""
+    Nothing is kept between calls."""
 
     def __init__(self, conv: "TeceConvolution", mlp, dtype):
         self.lmax, self.H, self.A, self.C = conv.lmax, conv.H, conv.A, conv.C
@@ -522,7 +521,7 @@ class _FusedParams:
         kernels = SO2_GEMM if self.bf16 else F32_GEMM
         if (kernels and dtype == torch.float32
                 and all(p.is_cuda and p.dtype == dtype and p.is_contiguous() for p in params)):
-            self._layout(conv, gemms, floats, params)
+            self._layout(gemms, floats, params[0].device)
             return
         for o, _, _ in gemms:
             m = o.make()
@@ -535,32 +534,25 @@ class _FusedParams:
         self.rp_T, self.rp_N = Wrp.t().contiguous(), Wrp.contiguous()
         self.mlp_flat = torch.cat([(m.weight * m.alpha).detach().reshape(-1) for m in lins[:-1]]).to(dtype).contiguous()
 
-    def _layout(self, conv, gemms, floats, params):
-        """All operands in one launch; see the class."""
-        dev = params[0].device
-        key = (self.bf16, str(dev)) + tuple(p.data_ptr() for p in params)
-        kept = conv.__dict__.get("_operand_table")
-        if kept is None or kept[0] != key:
-            rows, places, at = [], [], 0
+    def _layout(self, gemms, floats, dev):
+        """All operands in one buffer; see the class."""
+        table, places, at = array.array("q"), [], 0
 
-            def add(kind, k, n, segs, along_k, trans, ld, nbytes):
-                nonlocal at
-                row = [kind, k, n, at, len(segs), int(along_k), trans, ld]
-                for w, length, alpha in segs:
-                    row += [w.data_ptr(), length, struct.unpack("q", struct.pack("d", alpha))[0]]
-                rows.append(row + [0] * (20 - len(row)))
-                places.append((at, nbytes))
-                at += (nbytes + 15) // 16 * 16
-            for o, segs, along_k in gemms:
-                size = 1024 * ((o.k + 31) // 32) * ((o.n + 15) // 16)
-                cin = o.n if along_k else o.k
-                add(0 if self.bf16 else 1, o.k, o.n, segs, along_k, int(not along_k), cin, size * (1 if self.bf16 else 3))
-            for _nm, segs, k, n, along_k, trans, ld in floats:
-                add(2, k, n, segs, along_k, trans, ld, 4 * k * n)
-            kept = (key, torch.tensor(rows, dtype=torch.int64, device=dev), places, at)
-            conv.__dict__["_operand_table"] = kept
-        _, table, places, nbytes = kept
-        buf = ops.layout_operands(table, nbytes)
+        def add(kind, k, n, segs, along_k, trans, ld, nbytes):
+            nonlocal at
+            table.extend((kind, k, n, at, len(segs), along_k, trans, ld))
+            for w, length, alpha in segs:
+                table.extend((w.data_ptr(), length, struct.unpack("q", struct.pack("d", alpha))[0]))
+            table.extend((0,) * (12 - 3 * len(segs)))
+            places.append((at, nbytes))
+            at += (nbytes + 15) // 16 * 16
+        for o, segs, along_k in gemms:
+            size = 1024 * ((o.k + 31) // 32) * ((o.n + 15) // 16)
+            cin = o.n if along_k else o.k
+            add(0 if self.bf16 else 1, o.k, o.n, segs, int(along_k), int(not along_k), cin, size * (1 if self.bf16 else 3))
+        for _nm, segs, k, n, along_k, trans, ld in floats:
+            add(2, k, n, segs, int(along_k), trans, ld, 4 * k * n)
+        buf = ops.layout_operands(torch.frombuffer(table, dtype=torch.int64).view(-1, 20), at, dev)
         for (o, _, _), (at, size) in zip(gemms, places):
             o.frag = buf[at:at + size].view(torch.bfloat16 if self.bf16 else torch.int16)
         for (nm, _, k, n, *_), (at, size) in zip(floats, places[len(gemms):]):

@@ -59,3 +59,54 @@ def test_backward_is_of_the_forwards_weights(cuda, dtype, mixing, kernels, strid
     assert torch.equal(out, again)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     assert not torch.equal(f(), out)
+
+
+def _params(conv, mlp):
+    P = tece._FusedParams(conv, mlp, torch.float32)
+    return P, [o.frag for T in (P.k_T, P.k_N, P.q_T, P.q_N, P.d_T, P.d_N, P.s_T, P.s_N) for o in T] + [
+        P.s_b, P.mlp_flat, P.rp_T, P.rp_N]
+
+
+def test_nothing_is_kept_and_scales_are_read(cuda):
+    """Another scale of a linear makes other operands; a call leaves nothing on the module."""
+    f, conv, mlp, _ = _layer(cuda, torch.float32)
+    before = set(vars(conv))
+    out = f()
+    conv.linear_down.m0_rlinear.alpha *= 2
+    twice = f()
+    conv.linear_down.m0_rlinear.alpha /= 2
+    assert set(vars(conv)) == before
+    assert not torch.equal(twice, out) and torch.equal(f(), out)
+
+
+@pytest.mark.parametrize("mixing", [None, torch.bfloat16])
+def test_operands_in_a_recorded_graph(cuda, mixing):
+    """The layout recorded at its first call; replays read the weights as they
+    are then, also after the module has moved to other weights and been used."""
+    f, conv, mlp, _ = _layer(cuda, torch.float32, mixing)
+    held = [p.data for m in (conv, mlp) for p in m.parameters()]   # the recorded weights stay
+    graph = torch.cuda.CUDAGraph()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        conv.temperature_logit.sigmoid()
+    torch.cuda.current_stream().wait_stream(s)
+    with torch.cuda.graph(graph):
+        P, got = _params(conv, mlp)
+    eager = lambda: [t.clone() for t in _params(conv, mlp)[1]]
+    for step in range(3):
+        with torch.no_grad():
+            for p in held:
+                p.mul_(1.25)
+        want = eager()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, want)), step
+    for m in (conv, mlp):   # other storages; the graph keeps to the recorded ones
+        for p in m.parameters():
+            p.data = p.data.clone().mul_(3.0)
+    f()
+    torch.cuda.synchronize()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, want))
