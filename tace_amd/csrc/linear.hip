@@ -747,6 +747,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
   }
 
+  // which of this lane's outputs are not finite (bit 8 i + 4 j + q)
+  unsigned odd = 0;
+  if constexpr (!SPLIT) {
+    if (!tiles) {
+#pragma unroll
+      for (int e = 0; e < 8 * WM; ++e) odd |= (unsigned)!__builtin_isfinite(acc[e >> 3][(e >> 2) & 1][e & 3]) << e;
+    }
+  }
   // the bias of this lane's 8 columns (no loads are outstanding here)
   f4 bv[2];
 #pragma unroll
@@ -785,6 +793,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           if (col + q < n) dst[q] = v[q];
+      }
+    }
+  }
+  if constexpr (!SPLIT) {
+    // The dense product has the infinities of a float32 one: an infinity, or an
+    // x past bf16's largest, splits into terms of both signs, so its outputs
+    // came out NaN.  They are summed once more in order (rare; a sum that is
+    // NaN ends there).
+    if (odd) {
+      __threadfence_block();   // behind the other lanes' stores of the same outputs
+      const int nks = (dense.k + 31) >> 5;
+      for (; odd; odd &= odd - 1) {
+        const int e = __ffs(odd) - 1, r = 16 * (e >> 3) + fr, cl = c0 + wc + 16 * ((e >> 2) & 1) + 4 * fg + (e & 3);
+        if (r >= rows || cl >= n) continue;
+        const float* xr = x + (int64_t)(r0 + r) * dense.k;
+        const unsigned short* wc0 = wfrag + (int64_t)(cl >> 4) * nks * 1536 + 8 * (cl & 15);
+        float s = 0.f;
+        for (int kk = 0; kk < dense.k && s == s; ++kk) {
+          const unsigned short* w = wc0 + (int64_t)(kk >> 5) * 1536 + 128 * ((kk & 31) >> 3) + (kk & 7);
+          const float w0 = __uint_as_float((unsigned)w[0] << 16);
+          const float wv = __builtin_isinf(w0)
+              ? w0 : w0 + (__uint_as_float((unsigned)w[512] << 16) + __uint_as_float((unsigned)w[1024] << 16));
+          s = fmaf(xr[kk], wv, s);
+        }
+        y[out_base + (int64_t)r * n + cl] = bias ? s + bias[cl] : s;
       }
     }
   }
@@ -1228,6 +1261,7 @@ struct OpDesc {
 };
 
 constexpr int OPS_LAUNCH = 24;
+constexpr float BF16_MAX = 0x1.fep127f;
 struct OpTable {   // 3,840 bytes
   OpDesc op[OPS_LAUNCH];
 };
@@ -1255,6 +1289,16 @@ __global__ __launch_bounds__(256) void k_layout_operands(const OpTable table, un
     if (kind == 0) {
       *(bx3_bf8*)(dst + 1024 * run + 16 * lane) = h[0];
     } else {
+      // a weight that rounds past bf16's largest has that as its first term
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (__builtin_isinf((float)h[0][j]) && __builtin_isfinite(v[j])) {
+          h[0][j] = (__bf16)(v[j] < 0.f ? -BF16_MAX : BF16_MAX);
+          const float r = v[j] - (float)h[0][j];
+          h[1][j] = (__bf16)r;
+          h[2][j] = (__bf16)(r - (float)h[1][j]);
+        }
+      }
 #pragma unroll
       for (int p = 0; p < 3; ++p) *(bx3_bf8*)(dst + 1024 * (3 * run + p) + 16 * lane) = h[p];
     }
