@@ -10,13 +10,14 @@
 // one slice of the memory, a hub or a handful of keys makes the ranges long.)
 //
 // us, library sort and binary search | that counting sort | this: senders of
-// fcc lists of 78 edges a node, 13,500 nodes 124 | 81 | 57, with node ids
-// shuffled 124 | 163 | 67; 97,556 nodes shuffled 362 | 751 | 395; 8,192 equal
-// keys 41 | 3,129 | 15; 361,000 sorted under 16 keys 120 | 4,296 | 23; 30 M
-// random under 1 M keys 1,431 | 3,473 | 2,062 (runs of a digit are a few
-// words long: stores; the caller sorts lists that long).  The receiver CSR of
-// 1.05 M edges with the checks and the host's wait, sorted 228 | 253 | 85,
-// shuffled 459 | 133 | 98 (bincount, two minima, argsort before).
+// fcc lists of 78 edges a node, 13,500 nodes 124 | 81 | 51, with node ids
+// shuffled 124 | 163 | 58; 97,556 nodes shuffled 362 | 751 | 289; 8,192 equal
+// keys 41 | 3,129 | 15; 361,000 sorted under 16 keys 120 | 4,296 | 22; 30 M
+// random under 1 M keys 1,431 | 3,473 | 1,002.  The receiver CSR of 1.05 M
+// edges with the checks and the host's wait, sorted 228 | 253 | 78, shuffled
+// 459 | 133 | 87 (bincount, two minima, argsort before).  A few microseconds
+// per launch at 300,000 edges, latency; what the loads of a thread wait for
+// together decides the large sizes (97,556 nodes shuffled: 395 one by one).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -39,20 +40,23 @@ struct Keys {
   int64_t ostride;
   int* other32;
 
+  struct Loaded {
+    K key, before, other;   // key i, key i - 1, other key i
+  };
+
+  __device__ __forceinline__ Loaded load(int i) const {
+    const int64_t p = through ? through[i] : i, q = i == 0 ? p : through ? (int64_t)through[i - 1] : p - 1;
+    return {keys[p * stride], keys[q * stride], other ? other[i * ostride] : (K)0};
+  }
+
   // key i as an int, -1 outside [0, n_keys); flags[0]: some key (or other
   // key) outside, flags[1]: keys not ascending
-  __device__ __forceinline__ int get(int i, int n_keys, int* flags) const {
-    const int64_t p = through ? through[i] : i;
-    const K k = keys[p * stride];
-    bool ok = k >= 0 && k < (K)n_keys;
-    if (!ok) flags[0] = 1;
-    if (i > 0 && keys[(through ? (int64_t)through[i - 1] : p - 1) * stride] > k) flags[1] = 1;
-    if (other) {
-      const K o = other[i * ostride];
-      other32[i] = (int)o;
-      if (o < 0 || o >= (K)n_keys) flags[0] = 1;
-    }
-    return ok ? (int)k : -1;
+  __device__ __forceinline__ int take(const Loaded& v, int i, int n_keys, int* flags) const {
+    bool ok = v.key >= 0 && v.key < (K)n_keys;
+    if (v.before > v.key) flags[1] = 1;
+    if (other) other32[i] = (int)v.other;
+    if (!ok || (other && (v.other < 0 || v.other >= (K)n_keys))) flags[0] = 1;
+    return ok ? (int)v.key : -1;
   }
 };
 
@@ -81,8 +85,9 @@ __device__ __forceinline__ int digit_rank(int* cnt, int d, int bits, bool in, in
 }
 
 constexpr int MAX_BITS = 9, MAX_BINS = 1 << MAX_BITS;   // a digit's
-// positions a workgroup: a run of 64 STEPS per wavefront (1.05 M edges, 2
-// digits: 57 us; 16 steps 71, 32 steps 101, a workgroup's steps being serial)
+// positions a workgroup: a run of 64 STEPS per wavefront, whose ranks are a
+// serial chain (1.05 M edges, 2 digits, loads one by one: 57 us; 16 steps 71,
+// 32 steps 101)
 constexpr int STEPS = 8, CHUNK = 256 * STEPS;
 
 // Counts of the lowest digit per workgroup, hist [bins + 2][nwg]; the last two
@@ -94,11 +99,15 @@ __global__ __launch_bounds__(256) void k_group_first(Keys<K> in, int n, int n_ke
   const int t = (int)threadIdx.x;
   for (int b = t; b < bins + 2; b += 256) cnt[b] = 0;
   __syncthreads();
+  // every load goes out before the first is waited for (past the end: the last key)
   const int64_t i0 = (int64_t)blockIdx.x * CHUNK + t;
-#pragma unroll 4
+  typename Keys<K>::Loaded v[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) v[u] = in.load((int)min(i0 + 256 * u, (int64_t)n - 1));
+#pragma unroll
   for (int u = 0; u < STEPS; ++u) {
     if (i0 + 256 * u >= n) break;
-    const int i = (int)i0 + 256 * u, key = in.get(i, n_keys, cnt + bins);
+    const int i = (int)i0 + 256 * u, key = in.take(v[u], i, n_keys, cnt + bins);
     k32[i] = key;
     atomicAdd(cnt + (sort_key(key, n_keys) & (bins - 1)), 1);
   }
@@ -114,11 +123,12 @@ __global__ __launch_bounds__(256) void k_group_count(const int* __restrict__ key
   for (int b = t; b < bins; b += 256) cnt[b] = 0;
   __syncthreads();
   const int64_t i0 = (int64_t)blockIdx.x * CHUNK + t;
-#pragma unroll 4
-  for (int u = 0; u < STEPS; ++u) {
-    if (i0 + 256 * u >= n) break;
-    atomicAdd(cnt + ((keys[i0 + 256 * u] >> shift) & (bins - 1)), 1);
-  }
+  int v[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) v[u] = keys[min(i0 + 256 * u, (int64_t)n - 1)];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u)
+    if (i0 + 256 * u < n) atomicAdd(cnt + ((v[u] >> shift) & (bins - 1)), 1);
   __syncthreads();
   for (int b = t; b < bins; b += 256) hist[(int64_t)b * gridDim.x + blockIdx.x] = cnt[b];
 }
@@ -136,29 +146,31 @@ __global__ __launch_bounds__(1024) void k_group_scan(const int* __restrict__ his
 __global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ keys, const int* __restrict__ pos, int n,
                                                        int n_keys, int shift, int bits, const int* __restrict__ offs,
                                                        int* __restrict__ keys_out, int* __restrict__ pos_out) {
-  __shared__ int cnt[4][MAX_BINS], wsum[4];
+  __shared__ int cnt[4][MAX_BINS], total[MAX_BINS], before[MAX_BINS], wsum[4];
   const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, bins = 1 << bits, nwg = (int)gridDim.x;
-  for (int b = t; b < 4 * MAX_BINS; b += 256) cnt[b / MAX_BINS][b % MAX_BINS] = 0;
-  __syncthreads();
+  for (int b = t; b < bins; b += 256) cnt[0][b] = cnt[1][b] = cnt[2][b] = cnt[3][b] = 0;
   const int64_t i0 = (int64_t)blockIdx.x * CHUNK + 64 * STEPS * w + lane;
-  int key[STEPS], rank[STEPS];
+  int key[STEPS], rank[STEPS], at0[STEPS];
 #pragma unroll
   for (int u = 0; u < STEPS; ++u) {
-    key[u] = i0 + 64 * u < n ? sort_key(keys[i0 + 64 * u], n_keys) : -1;
+    const int64_t i = min(i0 + 64 * u, (int64_t)n - 1);
+    key[u] = keys[i];
+    at0[u] = pos ? pos[i] : (int)i;
   }
-#pragma unroll
-  for (int u = 0; u < STEPS; ++u)
-    rank[u] = digit_rank(cnt[w], (key[u] >> shift) & (bins - 1), bits, key[u] >= 0, lane);
+  for (int b = t; b < bins; b += 256) {
+    total[b] = offs[(int64_t)b * (nwg + 1) + nwg];
+    before[b] = offs[(int64_t)b * (nwg + 1) + blockIdx.x];
+  }
   __syncthreads();
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) {
+    key[u] = i0 + 64 * u < n ? sort_key(key[u], n_keys) : -1;
+    rank[u] = digit_rank(cnt[w], (key[u] >> shift) & (bins - 1), bits, key[u] >= 0, lane);
+  }
   // where each digit's positions of each wavefront go: all smaller digits,
   // the digit's in the workgroups before, in the wavefronts before.  Thread t
   // has digits 2 t and 2 t + 1.
-  int total[2], s = 0;
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    total[q] = 2 * t + q < bins ? offs[(int64_t)(2 * t + q) * (nwg + 1) + nwg] : 0;
-    s += total[q];
-  }
+  const int s = (2 * t < bins ? total[2 * t] : 0) + (2 * t + 1 < bins ? total[2 * t + 1] : 0);
   int inc = s;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -173,16 +185,17 @@ __global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ k
     if (k < w) run += wsum[k];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    if (2 * t + q < bins) {
-      int at = run + offs[(int64_t)(2 * t + q) * (nwg + 1) + blockIdx.x];
+    const int b = 2 * t + q;
+    if (b < bins) {
+      int at = run + before[b];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int c = cnt[k][2 * t + q];
-        cnt[k][2 * t + q] = at;
+        const int c = cnt[k][b];
+        cnt[k][b] = at;
         at += c;
       }
+      run += total[b];
     }
-    run += total[q];
   }
   __syncthreads();
 #pragma unroll
@@ -190,7 +203,7 @@ __global__ __launch_bounds__(256) void k_group_scatter(const int* __restrict__ k
     if (key[u] < 0) continue;
     const int at = cnt[w][(key[u] >> shift) & (bins - 1)] + rank[u];
     keys_out[at] = key[u];
-    pos_out[at] = pos ? pos[i0 + 64 * u] : (int)(i0 + 64 * u);
+    pos_out[at] = at0[u];
   }
 }
 
@@ -228,7 +241,7 @@ __global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_k
     const int i = i0 + 64 * u;
     v[u] = -1;
     if (i < n) {
-      const int key = in.get(i, n_keys, fl);
+      const int key = in.take(in.load(i), i, n_keys, fl);
       k32[i] = key;
       v[u] = (sort_key(key, n_keys) << POS_BITS) | i;
     }

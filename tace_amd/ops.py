@@ -199,7 +199,7 @@ class EdgePlan:
         """(s_rowptr int32 [N+1], s_slot int32 [E]): receiver-sorted slots grouped
         by sender, stable -- the fixed order of the grad_x segmented sum."""
         if self._sender is None:
-            if self.src.is_cuda and self.n_edges <= GROUP_MAX:
+            if self.src.is_cuda:
                 self._sender = _group_keys(self.src, self.n_nodes, through=self.eid)[1:3]
             else:
                 slot_src = self.src if self.eid is None else self.src[self.eid.long()]
@@ -1451,12 +1451,6 @@ def scatter_add_rows(out: torch.Tensor, index: torch.Tensor, src: torch.Tensor) 
     return rows_accumulate(out.view(n, -1), src.reshape(E, -1).contiguous(), rp, slot).view(out.shape)
 
 
-# positions up to which tace_group_keys groups them without a check; beyond, the
-# library's sort: 7.6 M edges of 97,556 nodes 318 against 352 us (shuffled node
-# ids 395, 362), 11.2 M random keys 629, 525, 30 M 2,062, 1,431
-GROUP_MAX = 8 << 20
-
-
 def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor] = None,
                 other: Optional[torch.Tensor] = None, flags: Optional[torch.Tensor] = None):
     """``tace_group_keys`` on 1-D GPU keys (any stride; ``through``: int32
@@ -1483,13 +1477,12 @@ def _group_keys(keys: torch.Tensor, n_keys: int, through: Optional[torch.Tensor]
 def group_by_key(keys: torch.Tensor, n_keys: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """(rowptr int32 [n_keys+1], order int32 [E]) of keys in [0, n_keys): the
     positions grouped by key, in position order within a key, and each key's
-    range (no host synchronisation): ``tace_group_keys`` on the GPU up to
-    ``GROUP_MAX`` positions, a stable sort and a binary search of the sorted
-    keys elsewhere."""
+    range (no host synchronisation): ``tace_group_keys`` on the GPU, a stable
+    sort and a binary search of the sorted keys elsewhere."""
     if n_keys >= 2 ** 31:
         raise ValueError("group_by_key: more than 2^31 keys")
     if (keys.is_cuda and keys.dim() == 1 and keys.dtype in (torch.int64, torch.int32)
-            and keys.shape[0] <= GROUP_MAX and n_keys < 2 ** 31 - 8192):
+            and max(n_keys, keys.shape[0]) < 2 ** 31 - 8192):
         return _group_keys(keys, n_keys)[1:3]
     k32 = keys.to(torch.int32)
     srt, order = torch.sort(k32, stable=True)

@@ -72,19 +72,14 @@ def test_grouping_costs_the_same_for_any_keys(cuda, n, n_keys):
     assert max(t.values()) < 5 * even + 0.1, t
 
 
-@pytest.mark.parametrize("E", [ops.GROUP_MAX, ops.GROUP_MAX + 1])
-def test_long_lists_by_the_library_sort(cuda, E):
-    """Both sides of the limit, sender ranges of sorted and of shuffled edges: the same order."""
-    n = 100000
-    dst = torch.arange(E, device=cuda) * n // E
-    src = (dst * 7919 + torch.arange(E, device=cuda) * 104729) % n
-    perm = (torch.arange(E, device=cuda) * 99991) % E
-    perm = perm if perm.unique().numel() == E else torch.arange(E - 1, -1, -1, device=cuda)
-    for e in (torch.stack([src, dst]), torch.stack([src[perm], dst[perm]])):
-        plan = ops.EdgePlan.from_edge_index(e, n)
-        by_slot = plan.src if plan.eid is None else plan.src[plan.eid.long()]
-        rp, slot = plan.sender_csr()
-        assert torch.equal(slot.long(), torch.argsort(by_slot, stable=True))
-        assert torch.equal(rp[1:].long(), torch.bincount(by_slot, minlength=n).cumsum(0))
-        rp2, order = ops.group_by_key(by_slot, n)
-        assert torch.equal(rp, rp2) and torch.equal(slot, order)
+def test_long_list(cuda):
+    """9 M shuffled edges of 300,000 nodes: three digits, more workgroups than a scan takes at once."""
+    E, n = 9000001, 300000
+    i = torch.arange(E, device=cuda)
+    dst, src = (i * 99991) % E * n // E, (i * 104729 + 17) % n
+    plan = ops.EdgePlan.from_edge_index(torch.stack([src, dst]), n)
+    assert torch.equal(plan.eid.long(), torch.argsort(dst, stable=True))
+    by_slot = plan.src[plan.eid.long()]
+    rp, slot = plan.sender_csr()
+    assert torch.equal(slot.long(), torch.argsort(by_slot, stable=True))
+    assert torch.equal(rp[1:].long(), torch.bincount(by_slot, minlength=n).cumsum(0))
