@@ -231,19 +231,28 @@ __global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_k
                                                       int* __restrict__ order, int* __restrict__ flags) {
   __shared__ int data[SMALL_N], cnt[16][SMALL_BINS], wsum[16], fl[2];
   const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, bins = 1 << bits;
-  constexpr int PER = SMALL_N / 1024;   // a run of 64 PER positions per wavefront
+  // each wavefront a run of 64 `steps` positions: all of them take part however
+  // few there are, as the steps are serial (1,792 edges: 12 us with 8 steps)
+  constexpr int PER = SMALL_N / 1024;
+  const int steps = (n + 1023) >> 10;
   if (t < 2) fl[t] = 0;
   __syncthreads();
-  const int i0 = 64 * PER * w + lane;
+  const int i0 = 64 * steps * w + lane;
   int v[PER], rank[PER];
+  {
+    typename Keys<K>::Loaded l[PER];
 #pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int i = i0 + 64 * u;
-    v[u] = -1;
-    if (i < n) {
-      const int key = in.take(in.load(i), i, n_keys, fl);
-      k32[i] = key;
-      v[u] = (sort_key(key, n_keys) << POS_BITS) | i;
+    for (int u = 0; u < PER; ++u)
+      if (u < steps) l[u] = in.load(min(i0 + 64 * u, n - 1));   // (no steps without positions)
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = i0 + 64 * u;
+      v[u] = -1;
+      if (u < steps && i < n) {
+        const int key = in.take(l[u], i, n_keys, fl);
+        k32[i] = key;
+        v[u] = (sort_key(key, n_keys) << POS_BITS) | i;
+      }
     }
   }
   for (int p = 0; p < passes; ++p) {
@@ -252,7 +261,7 @@ __global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_k
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < PER; ++u)
-      rank[u] = digit_rank(cnt[w], (v[u] >> shift) & (bins - 1), bits, v[u] >= 0, lane);
+      if (u < steps) rank[u] = digit_rank(cnt[w], (v[u] >> shift) & (bins - 1), bits, v[u] >= 0, lane);
     __syncthreads();
     // exclusive scan over (digit, wavefront): thread t has two wavefronts'
     // counts of digit t / 8
@@ -278,7 +287,7 @@ __global__ __launch_bounds__(1024) void k_group_small(Keys<K> in, int n, int n_k
       if (v[u] >= 0) data[cnt[w][(v[u] >> shift) & (bins - 1)] + rank[u]] = v[u];
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < PER; ++u) v[u] = i0 + 64 * u < n ? data[i0 + 64 * u] : -1;
+    for (int u = 0; u < PER; ++u) v[u] = u < steps && i0 + 64 * u < n ? data[i0 + 64 * u] : -1;
     // (the next pass's barriers keep its writes of data behind these reads)
   }
 #pragma unroll
