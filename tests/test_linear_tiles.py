@@ -83,7 +83,6 @@ def test_seg_linear_streamed_weights_split(cuda, steps, want, monkeypatch):
     run = lambda: pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.9, out=None, addend=add)
     monkeypatch.setattr(ops, "SEG_SPLIT_MAX_WORK", 0)
     ref = run()
-    lin.lay._seg.clear()
     monkeypatch.setattr(ops, "SEG_STREAM_BYTES", 1 << 20)
     monkeypatch.setattr(ops, "SEG_STREAM_STEPS", steps)
     monkeypatch.setattr(ops, "SEG_SPLIT_MIN_STEPS", 1)
@@ -152,7 +151,6 @@ def test_short_k_tasks_equal_the_tile_kernel(cuda, k, monkeypatch):
     res = []
     for min_n in (None, 256):
         monkeypatch.setattr(ops, "SEG_KS_MIN_N", min_n)
-        lin.lay._seg.clear()
         plan = lin.lay.seg_plan("fwd", rr, Z, x, lin.weight, lin.bias)
         assert (plan.n_ks > 0) == (min_n is not None)
         y = pm._linear_apply(x, lin.weight, lin.bias, lin.lay, rr, seg, 0.5)
