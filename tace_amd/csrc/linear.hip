@@ -504,17 +504,16 @@ __global__ __launch_bounds__(256) void k_seg_linear_bx3s(const float* __restrict
 //    for 32 columns: 142 registers, so three workgroups run per CU and one's
 //    MFMAs cover another's loads and splits (a whole tile per workgroup, 2 x 2
 //    wavefronts of 64 x 64, ran two at 232 registers), and row blocks past
-//    the tile's rows are left out 32 at a time.  What bounds it then is the
-//    power the matrix cores draw: with both at full load the 64-row form
-//    needs 17% fewer cycles but runs at 1.54 instead of 1.85 GHz, and a
-//    library bf16 product loses the same share from all-zero to random
-//    operands (2247 -> 1602 TFLOP/s).  Taller or wider wavefront tiles (128 x
-//    32 with two workgroups per CU) measured slower.  The tables' XCD runs
-//    matter as much (_xcd_balanced in ops.py).  Both together, whole tiles in
-//    runs of equal length -> halves in runs of equal cost: 12,288 rows x (1 +
-//    3 + 5 + 7), k 2,944-5,376 into 128 columns, 1666 -> 1309 us (142 -> 181
-//    TFLOP/s); the same at 1,024 rows and 4 species 247 -> 153 us; 128 -> 128
-//    shared linears 52 -> 51 us.
+//    the tile's rows are left out 32 at a time.  Taller or wider wavefront
+//    tiles (128 x 32 with two workgroups per CU) measured slower.  The tables'
+//    XCD runs matter as much (_xcd_balanced in ops.py).  Both together, whole
+//    tiles in runs of equal length -> halves in runs of equal cost: 12,288
+//    rows x (1 + 3 + 5 + 7), k 2,944-5,376 into 128 columns, 1660 -> 1325 us
+//    (143 -> 179 TFLOP/s, 3.50 -> 2.46 M cycles, MFMA pipe 39 -> 56% busy); the
+//    same at 1,024 rows and 4 species 167 -> 145 us; 128 -> 128 shared linears
+//    52 -> 51 us.  Part of what is left is power: 1,164 us with all operands
+//    zero, and a library bf16 product goes from 1,337 TFLOP/s on random
+//    operands to 1,707 on zeros.
 // Tiles, contributions and the XCD-grouped tile order are those of
 // k_seg_linear_bx3s (entries of 0 rows are skipped); contribution column 2 is
 // the block's offset in the fragment-order weights.  Per output element the products and their order
@@ -600,8 +599,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // of each other, so what one of them loads the others find in L2.  (With
   // the splits of a tile side by side, or unsplit, the row tiles of a long-k
   // block drift apart by more steps than L2 holds: 5,003 rows of 89 species,
-  // k 5,888-10,752 into 256 columns, 4.8 GB of weights: 19.6 GB fetched and
-  // 3,451 us unsplit, 3,281 us in 4 neighbouring splits, 2,710 us this way.)
+  // k 5,888-10,752 into 256 columns, 4.8 GB of weights: 20.7 GB read and 3,451
+  // us unsplit, 3,281 us in 4 neighbouring splits, 16.3 GB and 2,710 us this way.)
   const int half = (int)(blockIdx.x >> 3) & 1;
   const int wi = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 4);
   const int sp = SPLIT ? wi / n_tiles : 0, tile = SPLIT ? wi - sp * n_tiles : wi;
@@ -902,10 +901,10 @@ __global__ __launch_bounds__(256) void k_seg_split_sum(float* y, const float* ad
 // Two shapes, both of 64 rows: k <= 128 in one group (52 KB of LDS, three
 // workgroups per CU), k <= 256 in two groups (101 KB, one).  Large launches
 // are bound by power and by the writes: 5,184 rows of the 593 x 128 columns of
-// a product basis run the MFMAs at 1.36 PFLOP/s without the stores (442 us)
-// and take 671 us with them (1.6 GB: the two add up, the card is at its power
-// limit), 709 us with 128 rows per workgroup and one workgroup per CU, whose
-// operands came in and went out behind nothing.  Small ones gain from the
+// a product basis take 671 us, 442 in a copy without the stores (1.6 GB; the
+// two add up) and 10% less with all operands zero; 709 us with 128 rows per
+// workgroup and one workgroup per CU, whose operands came in and went out
+// behind nothing.  Small ones gain from the
 // smaller workgroups: 64 rows 41 -> 18 us, 400 rows 88 -> 55, 1,024 rows
 // 170 -> 164, 3,000 rows of 89 species 584 -> 538.  For k <= 256, 32 rows in
 // three workgroups per CU read B twice as often: 3,180 us became 3,431 (6,656

@@ -474,8 +474,8 @@ __global__ __launch_bounds__(256) void k_mlp_out_f32(const float* __restrict__ h
 // MFMAs.  Read-bound on g with enough wavefronts in flight; a launch of few
 // rows has too few, each going through all of N one slab's latency at a time,
 // so there N is spread over gridDim.y workgroups (n_per columns each) that
-// write their sums apart (k_mlp_out_bwd_sum adds them in order).  At N = 2,944
-// with pairs: 500 rows 137 -> 20 us, 12,000 164 -> 64, 23,031 173 -> 129 (543
+// write their sums apart (k_mlp_out_bwd_sum adds them in order).  At N = 2,944,
+// every row the sum of two edges' (one edge's takes 76 us at 23,031): 500 rows 137 -> 20 us, 12,000 164 -> 64, 23,031 173 -> 129 (543
 // MB), 40,000 252 -> 209; from 130,000 rows on parts only add traffic (577 ->
 // 611).
 __device__ __forceinline__ void mlp_ld16(const float* __restrict__ row, int k, int N, bool ok, bool vec, float* v) {

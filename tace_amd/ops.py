@@ -1863,8 +1863,8 @@ def launch_mlp_out_f32(h, W, alpha: float) -> torch.Tensor:
 def _mlp_out_bwd_parts(rows: int, n: int, device):
     """(parts, their buffer or None): over how many workgroups per 128 rows
     the last layer's input gradient spreads its n columns.  At most the four
-    workgroups per CU that run together (23,031 rows of 2,944 columns: 76 us in
-    five parts, 88 in six), or two parts that nearly do; of at least eight
+    workgroups per CU that run together (23,031 rows of 2,944 columns, one edge
+    each: 76 us in five parts, 88 in six), or two parts that nearly do; of at least eight
     32-column slabs, or of 24 where there is a workgroup per CU already (70,000
     rows: 2,944 columns in two parts 400 -> 361 us, 512 columns in two 68 -> 76)."""
     wgs, slabs = max(1, (rows + 127) // 128), (n + 31) // 32
@@ -2231,7 +2231,7 @@ class SegLinearPlan:
         return r0, np.minimum(hi[own] - r0, R), np.maximum(rng[own, 0], 0)
 
     def _ks_tasks(self, Z, s_o, n, d, boff, mine, rng, f_stride, b_stride) -> np.ndarray:
-        """Tasks of one output block (one contribution with k <= 128, or
+        """Tasks of one output block (one contribution with k <= 256, or
         none): column chunk-major, so that the workgroups running at one time
         on an XCD share a chunk's weight columns in its L2."""
         k = mine[0][2] if mine else 0
