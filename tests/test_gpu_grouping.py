@@ -83,3 +83,21 @@ def test_long_list(cuda):
     rp, slot = plan.sender_csr()
     assert torch.equal(slot.long(), torch.argsort(by_slot, stable=True))
     assert torch.equal(rp[1:].long(), torch.bincount(by_slot, minlength=n).cumsum(0))
+
+
+@pytest.mark.parametrize("n,n_keys", [(5000, 300), (70000, 5000)])
+def test_grouping_in_a_recorded_graph(cuda, n, n_keys):
+    """Recorded once, replayed on other keys, with eager groupings between the replays."""
+    keys = _keys("even", n, n_keys, 0).to(cuda)
+    ops.group_by_key(keys, n_keys)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rp, order = ops.group_by_key(keys, n_keys)
+    for seed, kind in enumerate(("hub", "even", "sorted", "equal"), 1):
+        keys.copy_(_keys(kind, n, n_keys, seed))
+        graph.replay()
+        want = ops.group_by_key(keys, n_keys)
+        torch.cuda.synchronize()
+        assert torch.equal(order, want[1]) and torch.equal(rp, want[0])
+        assert torch.equal(order.long(), torch.argsort(keys, stable=True))
