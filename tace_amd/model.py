@@ -926,11 +926,13 @@ def _frozen(*mods: torch.nn.Module) -> bool:
     return not any(p.requires_grad for m in mods for p in m.parameters())
 
 
-def _hooked(m: torch.nn.Module) -> bool:
-    """A hook that a call of the module would run."""
-    glob = torch.nn.modules.module
-    return any(getattr(o, pre + h) for o, pre in ((m, "_"), (glob, "_global_"))
-               for h in ("forward_hooks", "forward_pre_hooks", "backward_hooks", "backward_pre_hooks"))
+def _hooked(*mods: torch.nn.Module) -> bool:
+    """A hook that a call of one of the modules would run."""
+    g = torch.nn.modules.module
+    return bool(g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks
+                or any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                       for m in mods))
 
 
 class _SharedInputLinearsFn(torch.autograd.Function):
@@ -1335,19 +1337,22 @@ class TACE(torch.nn.Module):
         and nothing that would notice that its modules are not called or that
         only x gets a gradient; a receiver CSR over exactly these nodes."""
         readout = self.energy_readouts[0]
-        if type(readout) is not ScalarReadOut or ops.MODE.double or ops.MODE.export or not x.is_cuda:
+        if ops.MODE.double or ops.MODE.export or not x.is_cuda or type(readout) is not ScalarReadOut:
             return False
         lin = readout.linear2
-        mods = [readout, *lin]
-        consts = [attrs, self.atomic_energy_layer.atomic_energy, self.scale_shift.scale, self.scale_shift.shift]
-        return (len(lin) == 2 and all(type(m) is e3nnLinear and m.bias is None for m in lin)
-                and not any("forward" in vars(m) or _hooked(m) for m in mods) and _frozen(readout)
-                and lin[0].weight.numel() == 16 * x.shape[1] and lin[1].weight.numel() == 16
-                and x.dtype in (torch.float32, torch.float64)
-                and all(t.dtype == x.dtype and t.device == x.device and not t.requires_grad
-                        for t in consts + [m.weight for m in lin])
-                and x.shape[1] <= 512 and 0 < x.shape[0] == attrs.shape[0] and sp.inv is not None
-                and isinstance(plan, ops.EdgePlan) and plan.n_nodes == x.shape[0])
+        if len(lin) != 2 or "forward" in vars(readout) or _hooked(readout, *lin):
+            return False
+        dt, n, C = x.dtype, x.shape[0], x.shape[1]
+        for m, numel in zip(lin, (16 * C, 16)):
+            w = m.weight
+            if type(m) is not e3nnLinear or "forward" in vars(m) or m.bias is not None or w.requires_grad \
+                    or w.dtype != dt or w.numel() != numel:
+                return False
+        for t in (attrs, self.atomic_energy_layer.atomic_energy, self.scale_shift.scale, self.scale_shift.shift):
+            if t.dtype != dt or t.requires_grad or not t.is_cuda:
+                return False
+        return (dt in (torch.float32, torch.float64) and C <= 512 and 0 < n == attrs.shape[0] and sp.inv is not None
+                and isinstance(plan, ops.EdgePlan) and plan.n_nodes == n)
 
     def energy(self, data, plan: ops.EdgePlan, edge_vector, exchange=None, pairs: Optional[ops.EdgePairs] = None):
         """Energy branch of ``readout_fn`` (``tace.py:356-418``) + ``ScaleShift``

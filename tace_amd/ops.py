@@ -2040,7 +2040,7 @@ def _xcd_balanced(table: np.ndarray, cost: np.ndarray, length: np.ndarray, runs:
 
 def seg_settings() -> tuple:
     """Every setting that decides a ``SegLinearPlan`` (part of a plan cache's key)."""
-    return (SEG_KS_MIN_N, tuple(sorted(SEG_KS_CHUNK.items())), SEG_TILE_FRAG, SEG_SPLIT_SLOTS, SEG_SPLIT_MIN_STEPS,
+    return (SEG_KS_MIN_N, SEG_KS_CHUNK[128], SEG_KS_CHUNK[256], SEG_TILE_FRAG, SEG_SPLIT_SLOTS, SEG_SPLIT_MIN_STEPS,
             SEG_SPLIT_MAX_WORK, SEG_STREAM_BYTES, SEG_STREAM_STEPS, SEG_PARTIAL_BYTES, SEG_BALANCE_MIN)
 
 
@@ -2172,6 +2172,7 @@ class SegLinearPlan:
                     parts[i] = _xcd_balanced(u, length * ((u[:, 1] + 63) // 64), length, 8 // self.splits)
         first = np.cumsum([0] + [len(u) for u in parts])
         self.launches = [(int(a), int(b - a)) for a, b in zip(first, first[1:])]   # (first tile, tiles)
+        self.partial_numel = max(n for _, n in self.launches) * self.splits * 16384
         t = np.concatenate(parts)
         self.n_tiles = len(t)
         self.tiles = torch.from_numpy(np.ascontiguousarray(t)).to(device)
@@ -2353,11 +2354,12 @@ def seg_linear_presplit(x: torch.Tensor, y: torch.Tensor, planes: Optional[torch
     b_ptr = None if bias is None else bias.data_ptr()
     a_ptr = _addend_ptr(addend, y)
     if plan.tile_frag and plan.splits > 1:
-        pe = max(n for _, n in plan.launches) * plan.splits * 16384
+        pe = plan.partial_numel
         partials = torch.empty(pe, dtype=torch.float32, device=x.device)
-        for t0, n_t in plan.launches:
+        tiles = plan.tiles.data_ptr()
+        for t0, n_t in plan.launches:   # (a tile is 8 x int64)
             N.check(N.lib().tace_seg_linear_presplit_frag_split(
-                x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr, plan.tiles[t0:t0 + n_t].data_ptr(), n_t,
+                x.data_ptr(), y.data_ptr(), a_ptr, frag.data_ptr(), b_ptr, tiles + 64 * t0, n_t,
                 plan.contribs.data_ptr(), int(plan.tile_aligned), plan.splits, partials.data_ptr(), pe, float(alpha), st),
                 "tace_seg_linear_presplit_frag_split")
     elif plan.tile_frag:
