@@ -746,12 +746,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
   }
 
-  // which of this lane's outputs are not finite (bit 8 i + 4 j + q)
+  // which of this lane's outputs are not finite (bit 8 i + 4 j + q); none in
+  // all but rare tiles, so one sum of zeros asks first
   unsigned odd = 0;
   if constexpr (!SPLIT) {
     if (!tiles) {
+      float z = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8 * WM; ++e) odd |= (unsigned)!__builtin_isfinite(acc[e >> 3][(e >> 2) & 1][e & 3]) << e;
+      for (int e = 0; e < 8 * WM; ++e) z = fmaf(acc[e >> 3][(e >> 2) & 1][e & 3], 0.f, z);
+      if (z != z) {
+#pragma unroll
+        for (int e = 0; e < 8 * WM; ++e) odd |= (unsigned)!__builtin_isfinite(acc[e >> 3][(e >> 2) & 1][e & 3]) << e;
+      }
     }
   }
   // the bias of this lane's 8 columns (no loads are outstanding here)
